@@ -400,6 +400,37 @@ def test_linear_backward(dev, orc, dtype, m, n, k, scratch):
         check_bf16_normwise(dw.to_host(), rdw, "dw")
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("m,n,pad", [
+    # 16-byte columns: rows about the 8 x 256 in flight, column edges of a workgroup, row shares
+    (1, 8, 0), (2047, 24, 0), (2049, 40, 0), (9000, 64, 0),
+    # one column per thread: ragged widths, padded rows
+    (300, 33, 0), (4100, 7, 0), (260, 24, 3)])
+def test_linear_backward_bias_gradient(dev, dtype, m, n, pad):
+    import ctypes
+    from teenygrad_amd._lib import check as chk, lib
+    rng = np.random.default_rng(m + n)
+    tdt, k = (tg.bf16 if dtype == "bf16" else tg.f32), 8
+    dy = np.full((m, n + pad), 1e30, np.float32)
+    dy[:, :n] = rb(rng.standard_normal((m, n), dtype=np.float32))
+    x, w = rb(rng.standard_normal((m, k), dtype=np.float32)), rb(rng.standard_normal((n, k), dtype=np.float32))
+    xb, wb, dyb = up(dev, x, dtype), up(dev, w, dtype), up(dev, dy, dtype)
+    dx, dw, db = tg.Buffer(tdt, (m, k)), tg.Buffer(tdt, (n, k)), tg.Buffer(tdt, (n,))
+    ref = dy[:, :n].astype(np.float64).sum(0)
+    # a tree of at most 13 + 5 fp32 additions, each within 2^-24 of its partial sum
+    bound = 18 * 2.0 ** -24 * np.abs(dy[:, :n]).astype(np.float64).sum(0)
+    # without a workspace each of 32 to 256 row groups is summed in order: m / 32 more additions at most
+    for ws in (K.linear_backward_workspace_size(m, n, k, tdt), 0):
+        print(f"[linear db] {dtype} M={m} N={n} pad={pad} workspace={ws}", flush=True)
+        with stream_workspace(dev, ws):
+            chk(lib.teeny_linear_backward(xb.ptr, wb.ptr, dyb.ptr, dx.ptr, dw.ptr, db.ptr, m, n, k, k, 1, 1, k,
+                                          n + pad, 1, k, 1, 1, k, 1, tdt.code, None))
+            got = db.to_host()
+        err = np.abs((from_bf16(got) if dtype == "bf16" else got).astype(np.float64) - ref)
+        limit = bound * (1 + m / 32 / 18) + (2.0 ** -8 * np.abs(ref) if dtype == "bf16" else 0)
+        assert np.all(err <= limit), f"db: {np.max(err - limit)} beyond its bound"
+
+
 def test_linear_backward_strided_and_empty(dev, orc):
     # x given transposed in memory (stride_xm 1, stride_xk M) and dy rows
     # padded to 16 bytes (the RuntimeOp's backward_grad_output_row_stride):
