@@ -9,10 +9,12 @@
 // symmetric int8 (granularity PerChannel{axis: 0}, groups.rs:82-87).
 //
 // bf16 and int8 weights run on the MFMA core (gemm_core.hpp) whenever the
-// operands are K-contiguous and 16-byte aligned; anything else (fp32, odd
-// strides, ragged K for int8) runs gemm_generic: a 64 x 64 LDS-tiled fp32 FMA
-// kernel that accumulates each output in k order.
+// operands are K-contiguous and 16-byte aligned, fp32 operands with one unit
+// stride each on the fp32 matrix cores (gemm_f32.hpp); anything else (two odd
+// strides, bf16 off the vector grid, ragged K for int8) runs gemm_generic: a
+// 64 x 64 LDS-tiled fp32 FMA kernel that accumulates each output in k order.
 #include "gemm_core.hpp"
+#include "gemm_f32.hpp"
 
 namespace teeny {
 
@@ -193,6 +195,18 @@ static void launch_linear_db(const T *dy, int64_t sm, int64_t sn, T *db, int64_t
                        static_cast<int>(shares), db, sdb, static_cast<int>(N));
 }
 
+// fp32 GEMM: the matrix cores where gemm_f32.hpp reads the operands.
+static teeny_status launch_f32(const float *A, int64_t sam, int64_t sak, const float *B, int64_t sbn, int64_t sbk,
+                               float *C, int64_t scm, int64_t scn, const float *bias, int64_t M, int64_t N, int64_t K,
+                               hipStream_t s) {
+  if (gemm_f32_ok(sam, sak, sbn, sbk, M, N, K)) {
+    launch_gemm_f32(A, sam, sak, B, sbn, sbk, C, scm, scn, bias, M, N, K, s, stream_scratch(s));
+    return TEENY_OK;
+  }
+  return launch_generic<float, float, float>(A, sam, sak, B, sbn, sbk, C, scm, scn, nullptr, bias, nullptr, M, N, K,
+                                             TEENY_ACT_NONE, s);
+}
+
 static GemmParams plain_params(const void *A, int64_t lda, const void *B, int64_t ldb, void *C,
                                int64_t ldc, const float *scale, const float *bias,
                                const bf16 *bias_bf16, int64_t M, int64_t N, int64_t K) {
@@ -230,10 +244,9 @@ teeny_status teeny_linear_forward(const void *x, const void *w, const void *b, v
                 "linear_forward: x/w/y");
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == TEENY_F32) {
-    teeny_status st = launch_generic<float, float, float>(
-        static_cast<const float *>(x), stride_xm, stride_xk, static_cast<const float *>(w),
-        stride_wn, stride_wk, static_cast<float *>(y), stride_ym, stride_yn, nullptr,
-        static_cast<const float *>(b), nullptr, M, N, K, TEENY_ACT_NONE, s);
+    teeny_status st = launch_f32(static_cast<const float *>(x), stride_xm, stride_xk, static_cast<const float *>(w),
+                                 stride_wn, stride_wk, static_cast<float *>(y), stride_ym, stride_yn,
+                                 static_cast<const float *>(b), M, N, K, s);
     if (st != TEENY_OK) return st;
     return after_launch("linear_forward", s);
   }
@@ -322,10 +335,8 @@ teeny_status teeny_linear_backward(const void *x, const void *w, const void *dy,
     if (conv) {
       st = teeny_conv2d_backward_dx(dy, w, dx, M, K, N, 1, 1, 1, 1, &kConv1x1, dtype, TEENY_NHWC, stream);
     } else if (dtype == TEENY_F32) {
-      st = launch_generic<float, float, float>(static_cast<const float *>(dy), stride_dym, stride_dyn,
-                                               static_cast<const float *>(w), stride_wk, stride_wn,
-                                               static_cast<float *>(dx), stride_dxm, stride_dxk, nullptr, nullptr,
-                                               nullptr, M, K, N, TEENY_ACT_NONE, s);
+      st = launch_f32(static_cast<const float *>(dy), stride_dym, stride_dyn, static_cast<const float *>(w), stride_wk,
+                      stride_wn, static_cast<float *>(dx), stride_dxm, stride_dxk, nullptr, M, K, N, s);
     } else {
       st = launch_generic<bf16, bf16, bf16>(static_cast<const bf16 *>(dy), stride_dym, stride_dyn,
                                             static_cast<const bf16 *>(w), stride_wk, stride_wn,
@@ -339,10 +350,8 @@ teeny_status teeny_linear_backward(const void *x, const void *w, const void *dy,
     if (conv) {
       st = teeny_conv2d_backward_dw(dy, x, dw, M, K, N, 1, 1, 1, 1, &kConv1x1, dtype, TEENY_NHWC, stream);
     } else if (dtype == TEENY_F32) {
-      st = launch_generic<float, float, float>(static_cast<const float *>(dy), stride_dyn, stride_dym,
-                                               static_cast<const float *>(x), stride_xk, stride_xm,
-                                               static_cast<float *>(dw), stride_dwn, stride_dwk, nullptr, nullptr,
-                                               nullptr, N, K, M, TEENY_ACT_NONE, s);
+      st = launch_f32(static_cast<const float *>(dy), stride_dyn, stride_dym, static_cast<const float *>(x), stride_xk,
+                      stride_xm, static_cast<float *>(dw), stride_dwn, stride_dwk, nullptr, N, K, M, s);
     } else {
       st = launch_generic<bf16, bf16, bf16>(static_cast<const bf16 *>(dy), stride_dyn, stride_dym,
                                             static_cast<const bf16 *>(x), stride_xk, stride_xm,
@@ -377,6 +386,10 @@ teeny_status teeny_linear_backward_workspace_size(int64_t M, int64_t N, int64_t 
     teeny_status st = teeny_conv2d_backward_workspace_size(M, K, N, 1, 1, 1, 1, &kConv1x1, dtype, TEENY_NHWC, bytes);
     if (st != TEENY_OK) return st;
   }
+  if (dtype == TEENY_F32) {  // the products of dx and dw
+    if (gemm_f32_ok(N, 1, 1, K, M, K, N)) *bytes = std::max(*bytes, gemm_f32_scratch_bytes(M, K, N));
+    if (gemm_f32_ok(1, N, 1, K, N, K, M)) *bytes = std::max(*bytes, gemm_f32_scratch_bytes(N, K, M));
+  }
   const int64_t shares = linear_db_shares(M, N);
   if (shares > 1) *bytes = std::max(*bytes, static_cast<size_t>(shares) * N * 4);
   return TEENY_OK;
@@ -391,7 +404,11 @@ teeny_status teeny_linear_workspace_size(int64_t M, int64_t N, int64_t K, teeny_
                 "linear_workspace_size: size exceeds 2^31-1");
   TEENY_REQUIRE(dtype == TEENY_F32 || dtype == TEENY_BF16 || dtype == TEENY_I8, TEENY_ERR_UNSUPPORTED_DTYPE,
                 "linear_workspace_size: dtype must be F32, BF16 or I8");
-  if (M == 0 || N == 0 || K == 0 || dtype == TEENY_F32) return TEENY_OK;
+  if (M == 0 || N == 0 || K == 0) return TEENY_OK;
+  if (dtype == TEENY_F32) {
+    if (gemm_f32_ok(K, 1, K, 1, M, N, K)) *bytes = gemm_f32_scratch_bytes(M, N, K);
+    return TEENY_OK;
+  }
   if (K % (dtype == TEENY_I8 ? 16 : 8) != 0) return TEENY_OK;  // generic kernel, no scratch
   // contiguous operands, as the MFMA path requires
   const GemmParams p = plain_params(nullptr, K, nullptr, K, nullptr, N, nullptr, nullptr, nullptr, M, N, K);

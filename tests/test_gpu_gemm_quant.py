@@ -27,6 +27,43 @@ def test_linear_f32_fixture(dev, orc, with_bias):
     check_f32(got, orc.linear(x, w, b if with_bias else None), "linear f32")
 
 
+F32_GEMM = [  # (M, N, K): tile edges, ragged vectors, k tails, splits, fewer than a 16-byte load spans
+    (1, 5, 4), (3, 3, 3), (31, 65, 29), (33, 64, 31), (64, 64, 32), (65, 63, 33), (129, 127, 97), (4, 4, 161),
+    (5, 1000, 700), (200, 72, 3001), (2300, 2200, 40)]
+
+
+@pytest.mark.parametrize("m,n,k", F32_GEMM)
+@pytest.mark.parametrize("xt,wt", [(False, False), (True, False), (False, True), (True, True)])
+def test_linear_f32_strides(dev, m, n, k, xt, wt):
+    # x and w along k or along their rows, rows padded by 3 (NaN between them), y transposed as well
+    rng = np.random.default_rng(m + 3 * n + 5 * k)
+    x = rng.standard_normal((m, k), dtype=np.float32)
+    w = rng.standard_normal((n, k), dtype=np.float32)
+    b = rng.standard_normal(n, dtype=np.float32)
+
+    def pad(a):
+        out = np.full((a.shape[0], a.shape[1] + 3), np.nan, np.float32)
+        out[:, :a.shape[1]] = a
+        return out
+
+    xb, wb = dev.upload(pad(x.T if xt else x)), dev.upload(pad(w.T if wt else w))
+    bb = dev.upload(b)
+    sx, sw = ((1, m + 3) if xt else (k + 3, 1)), ((1, n + 3) if wt else (k + 3, 1))
+    ref = x.astype(np.float64) @ w.astype(np.float64).T + b
+    # k fp32 products and sums: each within 2^-24 of a partial sum no larger than sum |x| |w| (+ |b|)
+    bound = (k + 2) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T + np.abs(b))
+    for ws in (K.linear_workspace_size(m, n, k, tg.f32), 0):
+        for yt in (False, True):
+            print(f"[linear f32] M={m} N={n} K={k} xt={xt} wt={wt} yt={yt} workspace={ws}", flush=True)
+            y = dev.upload(np.full((n, m) if yt else (m, n), np.nan, np.float32))
+            with stream_workspace(dev, ws):
+                tg.check(_lib.lib.teeny_linear_forward(xb.ptr, wb.ptr, bb.ptr, y.ptr, m, n, k, *sx, *sw,
+                                                       *((1, m) if yt else (n, 1)), tg.f32.code, None))
+                got = y.to_host()
+            err = np.abs((got.T if yt else got).astype(np.float64) - ref)
+            assert np.all(err <= bound), f"{np.max(err - bound)} beyond the bound"
+
+
 def with_scratch(dev, scratch, need, fn):
     """Runs fn() with no stream workspace, or with one of ``need`` bytes."""
     if scratch == "workspace":
