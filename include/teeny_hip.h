@@ -436,8 +436,9 @@ teeny_status teeny_conv2d_backward_workspace_size(int64_t B, int64_t C_IN, int64
  * 256 for both dtypes.  dtype BF16 at head_dim 64 and 128 runs the MFMA flash
  * kernel, which needs 16-byte aligned q/k/v/o and one head's K (and V) below
  * 2 GiB (n_ctx_k * head_dim * 2 bytes; TEENY_ERR_SHAPE_MISMATCH otherwise);
- * the other bf16 head sizes and fp32 run the reference's per-query-row
- * structure (fp32 arithmetic on bf16 operands). */
+ * the other bf16 head sizes and fp32 run fp32 products (on bf16 operands
+ * widened to fp32), on the fp32 matrix cores up to head_dim 128 and in the
+ * reference's per-query-row structure at 256. */
 teeny_status teeny_flash_attention2_forward(const void *q, const void *k, const void *v, void *o,
                                             float *l, int64_t n_ctx_q, int64_t n_ctx_k,
                                             float softmax_scale, int64_t BH, int64_t head_dim,
@@ -473,9 +474,10 @@ teeny_status teeny_attention_forward(const void *q, const void *k, const void *v
  * non-causal).  No atomics: each output row is written once.  bf16 with
  * head_dim 64 / 128 and 16-byte aligned tensors runs on the MFMA kernels
  * (dkv needs a stream workspace of teeny_attention_backward_workspace_size
- * bytes for its D_m pre-pass, else it takes the per-row kernel); fp32 and
- * any other head_dim in {16, 32, 64, 128, 256} run the reference's per-row
- * structure. */
+ * bytes for its D_m pre-pass, else it takes the fp32 kernel); fp32 and any
+ * other head_dim in {16, 32, 64, 128, 256} run fp32 products, on the fp32
+ * matrix cores up to head_dim 128 and in the reference's per-row structure at
+ * 256. */
 teeny_status teeny_flash_attention2_backward_dq(const void *q, const void *k, const void *v, const void *o,
                                                 const void *dout, const float *l, void *dq, int64_t n_ctx_q,
                                                 int64_t n_ctx_k, float softmax_scale, int64_t BH, int64_t head_dim,

@@ -31,12 +31,15 @@
 // (b, h) pairs at a time: they stream the same K/V tiles, which then come
 // from that XCD's L2 rather than once per workgroup from HBM.
 //
-// fa_fwd_rows (fp32 at any power-of-two head_dim <= 256, and bf16 at the
-// head sizes the MFMA kernel does not take: 16, 32, 256).  The reference's
-// per-query-row structure — grid (N_q, BH), one wave per query row — with
-// the key loop vectorised across lanes: each lane scores one key of a
-// 64-key chunk, and the chunk is folded into the running (m, l, acc) state.
-// bf16 operands are widened to fp32 on load; all arithmetic is fp32.
+// fa_fwd_f32 (attn_f32.hpp: fp32 at head_dim 16 .. 128, bf16 at 16 and 32):
+// fp32 products on the fp32 matrix cores.
+//
+// fa_fwd_rows (head_dim 256).  The reference's per-query-row structure — grid
+// (N_q, BH), one wave per query row — with the key loop vectorised across
+// lanes: each lane scores one key of a 64-key chunk, and the chunk is folded
+// into the running (m, l, acc) state.  bf16 operands are widened to fp32 on
+// load; all arithmetic is fp32.
+#include "attn_f32.hpp"
 #include "mfma.hpp"
 
 namespace teeny {
@@ -397,7 +400,7 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void fa_fwd_bf16(const bf16 
   }  // pass
 }
 
-// Per-row path: grid (nq, BH), one wave per query row (flash_attn2.rs:48-51).
+// Per-row path (head_dim 256): grid (nq, BH), one wave per query row (flash_attn2.rs:48-51).
 template <typename T, int D>
 __global__ __launch_bounds__(64) void fa_fwd_rows(const T *__restrict__ Q, const T *__restrict__ K,
                                                   const T *__restrict__ V, T *__restrict__ O,
@@ -466,6 +469,15 @@ static void launch_rows(const void *q, const void *k, const void *v, void *o, fl
                      scale, causal, kv_group);
 }
 
+template <typename T, int D>
+static void launch_f32(const void *q, const void *k, const void *v, void *o, float *l, int nq, int nk, float scale,
+                       int BH, int causal, int kv_group, hipStream_t s) {
+  const bool split = fa_f32_split(cdiv(nq, 32) * BH, cdiv(nk, 32));
+  fa_f32_launch(fa_fwd_f32<T, D, 1>, fa_fwd_f32<T, D, 4>, nq, BH, split, s, static_cast<const T *>(q),
+                static_cast<const T *>(k), static_cast<const T *>(v), static_cast<T *>(o), l,
+                static_cast<uint32_t>(nq), static_cast<uint32_t>(nk), scale, causal, kv_group);
+}
+
 template <int D>
 static void launch_bf16(const void *q, const void *k, const void *v, void *o, float *l, int nq,
                         int nk, float scale, int BH, int causal, int kv_group, hipStream_t s) {
@@ -511,19 +523,19 @@ static teeny_status attention_entry(const void *q, const void *k, const void *v,
   const int bh = static_cast<int>(BH), group = static_cast<int>(q_heads / kv_heads);
   if (dtype == TEENY_F32) {
     switch (head_dim) {
-      case 16: launch_rows<float, 16>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s); break;
-      case 32: launch_rows<float, 32>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s); break;
-      case 64: launch_rows<float, 64>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s); break;
-      case 128: launch_rows<float, 128>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s); break;
+      case 16: launch_f32<float, 16>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s); break;
+      case 32: launch_f32<float, 32>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s); break;
+      case 64: launch_f32<float, 64>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s); break;
+      case 128: launch_f32<float, 128>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s); break;
       case 256: launch_rows<float, 256>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s); break;
       default: return fail(TEENY_ERR_UNSUPPORTED, nm + ": f32 head_dim must be 16, 32, 64, 128 or 256");
     }
     return after_launch(name, s);
   }
   if (dtype == TEENY_BF16) {
-    switch (head_dim) {  // head sizes off the matrix-core kernel: the per-row kernel
-      case 16: launch_rows<bf16, 16>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s); break;
-      case 32: launch_rows<bf16, 32>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s); break;
+    switch (head_dim) {  // head sizes off the bf16 matrix-core kernel
+      case 16: launch_f32<bf16, 16>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s); break;
+      case 32: launch_f32<bf16, 32>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s); break;
       case 256: launch_rows<bf16, 256>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s); break;
       case 64:
       case 128: break;

@@ -34,16 +34,19 @@
 // and the transposing reads (4 rows x 64 bytes per half-wave) touch
 // distinct banks.
 //
-// Any other case (fp32, other head sizes, unaligned bf16): the reference's
-// per-row structure, one wave per query row (dq) or key row (dkv), with the
-// inner loop vectorised across lanes.
+// Any other case (fp32, other head sizes, unaligned bf16, dk/dv alone without
+// a workspace): fp32 products on the fp32 matrix cores (attn_f32.hpp);
+// head_dim 256, whose operands and accumulators do not fit a wave's registers
+// there, runs the reference's per-row structure, one wave per query row (dq)
+// or key row (dkv), with the inner loop vectorised across lanes.
+#include "attn_f32.hpp"
 #include "mfma.hpp"
 
 namespace teeny {
 
 constexpr float kBwdLog2e = 1.4426950408889634f;
 
-// ── generic kernels ───────────────────────────────────────────────────────
+// ── per-row kernels (head_dim 256) ───────────────────────────────────────────────────────
 
 template <typename T, int D>
 __global__ __launch_bounds__(64) void fa_bwd_dq_rows(const T *__restrict__ Q, const T *__restrict__ K,
@@ -603,22 +606,44 @@ static void rows_dkv(const BwdArgs &a, const float *delta) {
                      static_cast<T *>(a.dk), static_cast<T *>(a.dv), a.nq, a.nk, a.scale, a.causal, a.group);
 }
 
+template <typename T, int D>
+static void f32_dq(const BwdArgs &a, float *delta_out) {
+  const bool split = fa_f32_split(cdiv(a.nq, 32) * a.BH, cdiv(a.nk, 32));
+  fa_f32_launch(fa_bwd_dq_f32<T, D, 1>, fa_bwd_dq_f32<T, D, 4>, a.nq, a.BH, split, a.s, static_cast<const T *>(a.q),
+                static_cast<const T *>(a.k), static_cast<const T *>(a.v), static_cast<const T *>(a.o),
+                static_cast<const T *>(a.dout), a.l, static_cast<T *>(a.dq), delta_out, static_cast<uint32_t>(a.nq),
+                static_cast<uint32_t>(a.nk), a.scale, a.causal, a.group);
+}
+
+template <typename T, int D>
+static void f32_dkv(const BwdArgs &a, const float *delta) {
+  const int64_t heads = a.BH / a.group;
+  const bool split = fa_f32_split(cdiv(a.nk, 32) * heads, cdiv(a.nq, 32) * a.group);
+  fa_f32_launch(fa_bwd_dkv_f32<T, D, 1>, fa_bwd_dkv_f32<T, D, 4>, a.nk, heads, split, a.s,
+                static_cast<const T *>(a.q), static_cast<const T *>(a.k), static_cast<const T *>(a.v),
+                static_cast<const T *>(a.o), static_cast<const T *>(a.dout), a.l, delta, static_cast<T *>(a.dk),
+                static_cast<T *>(a.dv), static_cast<uint32_t>(a.nq), static_cast<uint32_t>(a.nk), a.scale, a.causal,
+                a.group);
+}
+
+// dq (writing D_m to `delta` when not NULL) or dk/dv (reading it when not NULL).
+template <typename T, int D>
+static void f32_step(const BwdArgs &a, bool dq, float *delta) {
+  if (dq) f32_dq<T, D>(a, delta);
+  else f32_dkv<T, D>(a, delta);
+}
+
 template <typename T>
-static bool rows_launch(const BwdArgs &a, bool dq, const float *delta) {
-#define TEENY_BWD_ROWS(DD)          \
-  case DD:                          \
-    if (dq) rows_dq<T, DD>(a);      \
-    else rows_dkv<T, DD>(a, delta); \
-    return true;
+static void f32_launch(const BwdArgs &a, bool dq, float *delta) {
   switch (a.D) {
-    TEENY_BWD_ROWS(16)
-    TEENY_BWD_ROWS(32)
-    TEENY_BWD_ROWS(64)
-    TEENY_BWD_ROWS(128)
-    TEENY_BWD_ROWS(256)
-    default: return false;
+    case 16: f32_step<T, 16>(a, dq, delta); break;
+    case 32: f32_step<T, 32>(a, dq, delta); break;
+    case 64: f32_step<T, 64>(a, dq, delta); break;
+    case 128: f32_step<T, 128>(a, dq, delta); break;
+    default:  // 256
+      if (dq) rows_dq<T, 256>(a);
+      else rows_dkv<T, 256>(a, nullptr);
   }
-#undef TEENY_BWD_ROWS
 }
 
 template <int D>
@@ -742,12 +767,16 @@ static teeny_status bwd_entry(BwdArgs a, int64_t batch, int64_t q_heads, int64_t
       mfma_step(a, 0, delta);
       mfma_step(a, 1, delta);
     } else {
-      rows_launch<bf16>(a, false, nullptr);
+      f32_launch<bf16>(a, false, nullptr);
     }
     return after_launch(name, a.s);
   }
-  if (which & 1) (dtype == TEENY_F32 ? rows_launch<float> : rows_launch<bf16>)(a, true, nullptr);
-  if (which & 2) (dtype == TEENY_F32 ? rows_launch<float> : rows_launch<bf16>)(a, false, nullptr);
+  // dq first: given a workspace it leaves D_m there for dk/dv
+  const Scratch scr = stream_scratch(a.s);
+  const bool ws = which == 3 && a.D != 256 && scr.ptr != nullptr && scr.bytes >= delta_bytes(a);
+  float *delta = ws ? static_cast<float *>(scr.ptr) : nullptr;
+  if (which & 1) (dtype == TEENY_F32 ? f32_launch<float> : f32_launch<bf16>)(a, true, delta);
+  if (which & 2) (dtype == TEENY_F32 ? f32_launch<float> : f32_launch<bf16>)(a, false, delta);
   return after_launch(name, a.s);
 }
 
