@@ -460,6 +460,13 @@ teeny_status teeny_attention_forward(const void *q, const void *k, const void *v
                                      int64_t n_ctx_k, int64_t head_dim, float softmax_scale,
                                      int32_t causal, teeny_dtype dtype, teeny_stream stream);
 
+/* Stream workspace that lets attention_forward / flash_attention2_forward
+ * (batch = BH, one head) share a head's keys out over the device when there
+ * are few query rows (bf16 at head_dim 64 or 128); 0 where none is used. */
+teeny_status teeny_attention_workspace_size(int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t n_ctx_q,
+                                            int64_t n_ctx_k, int64_t head_dim, int32_t causal, teeny_dtype dtype,
+                                            size_t *bytes);
+
 /* Attention backward.  Reference: flash_attention2_backward_dq(q, k, v, o,
  * do, l, dq, n_ctx_q, n_ctx_k, softmax_scale) with grid (n_ctx_q, BH, 1) and
  * flash_attention2_backward_dkv(q, k, v, o, do, l, dk, dv, n_ctx_q, n_ctx_k,

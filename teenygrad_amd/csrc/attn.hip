@@ -6,7 +6,7 @@
 // o = acc / l and L = m + log(l) (:133-157).  Non-causal only in the
 // reference; `causal` here masks key j > query i (top-left aligned).
 //
-// Two kernels:
+// The kernels:
 //
 // fa_fwd_bf16 (the MI355X path).  One workgroup = WAVES waves (4 as
 // launched) of 32 queries of one (b, h).  K and V tiles of 64 keys are
@@ -31,6 +31,9 @@
 // (b, h) pairs at a time: they stream the same K/V tiles, which then come
 // from that XCD's L2 rather than once per workgroup from HBM.
 //
+// fa_split_bf16 (attn_split.hpp: few queries per K/V head, bf16 at head_dim 64
+// and 128): the keys shared out over waves and workgroups.
+//
 // fa_fwd_f32 (attn_f32.hpp: fp32 at head_dim 16 .. 128, bf16 at 16 and 32):
 // fp32 products on the fp32 matrix cores.
 //
@@ -39,7 +42,10 @@
 // lanes: each lane scores one key of a 64-key chunk, and the chunk is folded
 // into the running (m, l, acc) state.  bf16 operands are widened to fp32 on
 // load; all arithmetic is fp32.
+#include <algorithm>
+
 #include "attn_f32.hpp"
+#include "attn_split.hpp"
 #include "mfma.hpp"
 
 namespace teeny {
@@ -547,6 +553,24 @@ static teeny_status attention_entry(const void *q, const void *k, const void *v,
     // K and V of one (batch, head) are read through 32-bit buffer offsets
     TEENY_REQUIRE(n_ctx_k * head_dim * 2 <= 0x7fffffff, TEENY_ERR_SHAPE_MISMATCH,
                   nm + ": bf16 K/V of one head must be below 2 GiB");
+    const Scratch scr = stream_scratch(s);
+    const SplitPlan plan = split_plan(BH, group, nq, nk, head_dim, causal != 0, scr.ptr != nullptr ? scr.bytes : 0);
+    if (plan.use) {
+      SplitArgs a{};
+      a.Q = static_cast<const bf16 *>(q);
+      a.K = static_cast<const bf16 *>(k);
+      a.V = static_cast<const bf16 *>(v);
+      a.O = static_cast<bf16 *>(o);
+      a.L = l;
+      a.part = static_cast<float *>(scr.ptr);
+      a.rows = group * nq;
+      a.nq = nq;
+      a.nk = nk;
+      a.scale_log2 = softmax_scale * kLog2e;
+      if (head_dim == 64) (causal ? split_launch<64, true> : split_launch<64, false>)(plan, a, BH, group, s);
+      else (causal ? split_launch<128, true> : split_launch<128, false>)(plan, a, BH, group, s);
+      return after_launch(name, s);
+    }
     if (head_dim == 64) launch_bf16<64>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s);
     else launch_bf16<128>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s);
     return after_launch(name, s);
@@ -575,4 +599,23 @@ extern "C" teeny_status teeny_attention_forward(const void *q, const void *k, co
                                                 teeny_stream stream) {
   return attention_entry(q, k, v, o, l, batch, q_heads, kv_heads, n_ctx_q, n_ctx_k, head_dim, softmax_scale,
                          causal, dtype, stream, "attention_forward");
+}
+
+extern "C" teeny_status teeny_attention_workspace_size(int64_t batch, int64_t q_heads, int64_t kv_heads,
+                                                       int64_t n_ctx_q, int64_t n_ctx_k, int64_t head_dim,
+                                                       int32_t causal, teeny_dtype dtype, size_t *bytes) {
+  const std::string nm("attention_workspace_size");
+  TEENY_REQUIRE(bytes != nullptr, TEENY_ERR_NULL_POINTER, nm + ": bytes");
+  *bytes = 0;
+  TEENY_REQUIRE(n_ctx_q >= 0 && n_ctx_k >= 0 && batch >= 0 && q_heads >= 0 && kv_heads >= 0,
+                TEENY_ERR_SHAPE_MISMATCH, nm + ": negative size");
+  TEENY_REQUIRE(kv_heads > 0 ? q_heads % kv_heads == 0 : q_heads == 0, TEENY_ERR_SHAPE_MISMATCH,
+                nm + ": q_heads must be a multiple of kv_heads");
+  TEENY_REQUIRE(q_heads == 0 || batch <= 65535 / q_heads, TEENY_ERR_SHAPE_MISMATCH,
+                nm + ": batch * q_heads exceeds 65535");
+  if (batch == 0 || q_heads == 0 || n_ctx_q == 0 || n_ctx_k == 0 || dtype != TEENY_BF16 ||
+      (head_dim != 64 && head_dim != 128) || n_ctx_k * head_dim * 2 > 0x7fffffff)
+    return TEENY_OK;
+  *bytes = split_plan(batch * q_heads, q_heads / kv_heads, n_ctx_q, n_ctx_k, head_dim, causal != 0, ~size_t{0}).bytes;
+  return TEENY_OK;
 }

@@ -1,0 +1,283 @@
+// Attention forward for few query rows, bf16 at head_dim 64 and 128 (one token
+// at a time, a few draft tokens, short prompts, few heads): the keys of a head
+// are shared out over waves and workgroups.
+//
+// Bound: reading K and V once.  fa_fwd_bf16 gives each query head a workgroup
+// of 128 query rows, so with one query it multiplies mostly padding, reads a
+// K/V head once per query head that shares it, and runs as many workgroups
+// as there are heads.  Here the query rows that share a K/V head (its query
+// heads times their queries, consecutive in memory) are packed into column
+// blocks of 32; a workgroup of four waves takes one block and a range of the
+// keys, each wave every fourth 32-key tile of it, and the workgroups of a
+// block meet through the stream's workspace (fp32 partial outputs with their
+// max and sum, combined by a second small kernel in range order).
+// A wave works alone, with no barrier in its loop: S^T = K Q^T takes K's
+// fragments straight from memory to registers (each is used once, so LDS
+// would only add a copy), V's tile goes through the wave's own LDS for the
+// transposing read.  Both are refilled as soon as they are used, so a wave
+// has up to 16 KiB in flight, 128 KiB per CU, which covers the latency at
+// the full HBM rate.  Rounding points are fa_fwd_bf16's: probabilities to
+// bf16, everything else fp32.
+#pragma once
+
+#include "mfma.hpp"
+
+namespace teeny {
+
+struct SplitArgs {
+  const bf16 *Q, *K, *V;
+  bf16 *O;
+  float *L;
+  float *part;        // [unit][range][row][D] fp32, then [unit][range][row][2]; null: one range
+  int64_t ml_off;     // offset of the second array in floats
+  int rows;           // query rows per K/V head
+  int nq;             // queries per query head
+  int blocks;         // column blocks per K/V head
+  int nk, range;      // keys, keys per range (a multiple of 32)
+  float scale_log2;
+};
+
+template <int D, bool CAUSAL>
+__global__ __launch_bounds__(256, 2) void fa_split_bf16(SplitArgs p) {
+  constexpr int CPR = D / 8, RPB = 128 / D, NS = D / 16, ND = D / 32, NV = 32 * CPR / 64;
+  constexpr int RED = D * 33;  // a wave's partial output [D][33]
+  __shared__ __attribute__((aligned(16))) float red[4][RED];
+  __shared__ float ml[2][4][32];
+  static_assert(RED * 4 >= 32 * D * 2, "the V tile shares the reduction's space");
+  auto fv = [](int row) { return (4 * (row / RPB)) & (CPR - 1) & ~3; };
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 31, g = lane >> 5;
+  const int64_t unit = blockIdx.y;  // (K/V head, column block)
+  const int64_t hk = unit / p.blocks;
+  const int c0 = static_cast<int>(unit - hk * p.blocks) * 32, ncol = min(32, p.rows - c0);
+  const int64_t row0 = hk * p.rows + c0;
+  const bf16 *Kb = p.K + hk * p.nk * D, *Vb = p.V + hk * p.nk * D;
+  // causal: the row's query sees the keys up to its own index, the block's rows those up to their last one's
+  const int qi = CAUSAL ? (c0 + min(c, ncol - 1)) % p.nq : 0;
+  int k_end = p.nk;
+  if constexpr (CAUSAL) k_end = min(p.nk, c0 % p.nq + ncol > p.nq ? p.nq : c0 % p.nq + ncol);
+  const int kb = blockIdx.x * p.range, ke = min(k_end, kb + p.range);
+  bf16 *vt = reinterpret_cast<bf16 *>(red[w]);
+
+  const float sc = fmaxf(fabsf(p.scale_log2), 1.17549435e-38f);  // as fa_fwd_bf16: the sign goes to Q
+  const uint32_t qsign = p.scale_log2 < 0.0f ? 0x80008000u : 0u;
+  bf16x8 qf[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    u32x4 raw = *reinterpret_cast<const u32x4 *>(p.Q + (row0 + min(c, ncol - 1)) * D + 16 * s + 8 * g);
+    raw ^= qsign;
+    __builtin_memcpy(&qf[s], &raw, 16);
+  }
+  f32x16 acc[ND];
+#pragma unroll
+  for (int d = 0; d < ND; ++d) acc[d] = zero16();
+  float m_run = -INFINITY, l_run = 0.0f;
+
+  // the transposing read of V (see fa_fwd_bf16)
+  const int hh = lane >> 4, m16 = lane & 15, v_row = 4 * g + (m16 >> 2);
+  const int vofs = v_row * D + ((fv(v_row) | (2 * (hh & 1) + ((m16 & 3) >> 1))) << 3) + (m16 & 1) * 4;
+
+  u32x4 kr[NS], vr[NV];
+  auto load_k = [&](int k0) {
+    const bf16 *row = Kb + static_cast<int64_t>(min(k0 + c, p.nk - 1)) * D + 8 * g;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) kr[s] = *reinterpret_cast<const u32x4 *>(row + 16 * s);
+  };
+  auto load_v = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int t = 64 * i + lane;
+      vr[i] = *reinterpret_cast<const u32x4 *>(Vb + static_cast<int64_t>(min(k0 + t / CPR, p.nk - 1)) * D + 8 * (t % CPR));
+    }
+  };
+  int k0 = kb + 32 * w;
+  if (k0 < ke) {
+    load_k(k0);
+    load_v(k0);
+  }
+  for (; k0 < ke; k0 += 128) {
+    f32x16 s = zero16();
+#pragma unroll
+    for (int i = 0; i < NS; ++i) s = mfma32x32x16(__builtin_bit_cast(bf16x8, kr[i]), qf[i], s);
+    const bool more = k0 + 128 < ke, edge = k0 + 32 > p.nk;
+    const bool masks = edge || (CAUSAL && __any(k0 + 31 > qi));
+    if (more) load_k(k0 + 128);
+    float mx = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      if (masks && (k0 + mfma32_row(v, g) >= p.nk || (CAUSAL && k0 + mfma32_row(v, g) > qi))) s[v] = -INFINITY;
+      mx = __builtin_elementwise_maximum(mx, s[v]);
+    }
+    mx = __builtin_elementwise_maximum(mx, __shfl_xor(mx, 32, 64)) * sc;
+    if (__any(mx > m_run + 8.0f)) {  // rescaled rarely, as in fa_fwd_bf16: p <= 2^8
+      const float m_new = fmaxf(m_run, mx);
+      const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.0f : m_new));
+      l_run *= alpha;
+#pragma unroll
+      for (int d = 0; d < ND; ++d) acc[d] *= alpha;
+      m_run = m_new;
+    }
+    const float neg_m = m_run == -INFINITY ? 0.0f : -m_run;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      s[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], sc, neg_m));
+      l_run += s[v];
+    }
+    // rows past nk are zeros, so that a zero probability meets no stray infinity
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int t = 64 * i + lane, r = t / CPR;
+      u32x4 v = vr[i];
+      if (edge && k0 + r >= p.nk) v = u32x4{0u, 0u, 0u, 0u};
+      *reinterpret_cast<u32x4 *>(vt + r * D + (((t % CPR) ^ fv(r)) << 3)) = v;
+    }
+    if (more) load_v(k0 + 128);
+    // the wave's lanes read what its other lanes wrote
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      bf16x8 pb;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bf16x2 pr = cvt_pk_bf16(s[8 * tt + 2 * j], s[8 * tt + 2 * j + 1]);
+        pb[2 * j] = pr[0];
+        pb[2 * j + 1] = pr[1];
+      }
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        const bf16 *vp = vt + 16 * tt * D + (vofs ^ (d << 5));
+        const bf16x4 lo = ds_read_tr16(vp), hi = ds_read_tr16(vp + 8 * D);
+        acc[d] = mfma32x32x16(cat8(lo, hi), pb, acc[d]);
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  l_run += __shfl_xor(l_run, 32, 64);
+
+  // the four waves' parts: a common max, then the sum of their outputs
+  if (g == 0) {
+    ml[0][w][c] = m_run;
+    ml[1][w][c] = l_run;
+  }
+  __syncthreads();
+  float m = ml[0][0][c], l = 0.0f;
+#pragma unroll
+  for (int i = 1; i < 4; ++i) m = fmaxf(m, ml[0][i][c]);
+  const float ref = m == -INFINITY ? 0.0f : m;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) l += ml[1][i][c] * __builtin_amdgcn_exp2f(ml[0][i][c] - ref);
+  const bool whole = p.part == nullptr;
+  const float mul = __builtin_amdgcn_exp2f(m_run - ref) * (whole ? 1.0f / l : 1.0f);
+  if (c < ncol) {
+#pragma unroll
+    for (int d = 0; d < ND; ++d)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) red[w][(32 * d + mfma32_row(v, g)) * 33 + c] = acc[d][v] * mul;
+  }
+  __syncthreads();
+  const int64_t slot = (unit * gridDim.x + blockIdx.x) * 32;  // part rows of this (unit, range)
+  for (int i = threadIdx.x; i < ncol * (D / 4); i += 256) {
+    const int r = i / (D / 4), d = 4 * (i % (D / 4));
+    f32x4 o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      o[j] = (red[0][(d + j) * 33 + r] + red[1][(d + j) * 33 + r]) + (red[2][(d + j) * 33 + r] + red[3][(d + j) * 33 + r]);
+    if (whole) {
+      bf16x4 o4;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o4[j] = static_cast<bf16>(o[j]);
+      *reinterpret_cast<bf16x4 *>(p.O + (row0 + r) * D + d) = o4;
+    } else {
+      *reinterpret_cast<f32x4 *>(p.part + (slot + r) * D + d) = o;
+    }
+  }
+  if (w == 0 && g == 0 && c < ncol) {
+    if (!whole) {
+      p.part[p.ml_off + (slot + c) * 2] = m;
+      p.part[p.ml_off + (slot + c) * 2 + 1] = l;
+    } else if (p.L != nullptr) {
+      p.L[row0 + c] = (m + log2f(l)) * 0.6931471805599453f;
+    }
+  }
+}
+
+// One wave per query row: the ranges' parts, in range order.
+template <int D>
+__global__ __launch_bounds__(256) void fa_split_combine(SplitArgs p, int ranges, int64_t total) {
+  constexpr int V = D / 64;
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (row >= total) return;
+  const int64_t hk = row / p.rows;
+  const int r = static_cast<int>(row - hk * p.rows);
+  const int64_t slot = (hk * p.blocks + r / 32) * ranges * 32 + r % 32;
+  const float *ml = p.part + p.ml_off;
+  float m = -INFINITY;
+  for (int i = 0; i < ranges; ++i) m = fmaxf(m, ml[(slot + 32 * i) * 2]);
+  const float ref = m == -INFINITY ? 0.0f : m;
+  float l = 0.0f, o[V] = {};
+  for (int i = 0; i < ranges; ++i) {
+    const float f = __builtin_amdgcn_exp2f(ml[(slot + 32 * i) * 2] - ref);
+    l += ml[(slot + 32 * i) * 2 + 1] * f;
+#pragma unroll
+    for (int j = 0; j < V; ++j) o[j] = __builtin_fmaf(p.part[(slot + 32 * i) * D + lane * V + j], f, o[j]);
+  }
+  const float inv = 1.0f / l;
+#pragma unroll
+  for (int j = 0; j < V; ++j) p.O[row * D + lane * V + j] = static_cast<bf16>(o[j] * inv);
+  if (p.L != nullptr && lane == 0) p.L[row] = (m + log2f(l)) * 0.6931471805599453f;
+}
+
+// Whether this path is the better one, and into how many ranges it cuts the
+// keys.  fa_fwd_bf16 is the faster kernel on a full chip; its workgroups are
+// four column blocks each (eight, causal: two query blocks to a workgroup), so
+// it wants four (eight) times the blocks to fill it.  Measured in us
+// (heads x queries x keys x head_dim; fa_fwd_bf16 / here): 256 blocks, 16 x
+// 512 x 512 x 64 causal 16.4 / 9.0, 4 x 2048 x 2048 x 128 causal 47.6 / 26.2,
+// 8 x 1024 x 1024 x 128 22.3 / 16.6; 512 blocks, 16 x 1024 x 1024 x 128 causal
+// 31.4 / 26.9 but not causal 23.4 / 27.8, 4 x 4096 x 4096 x 128 71.6 / 81.1;
+// 1024 blocks, 64 x 512 x 512 x 128 16.6 / 32.0.  At up to 32 queries most of
+// fa_fwd_bf16's rows are padding and this path is taken at any size: 32 heads
+// sharing 8 K/V heads, one query, batch x keys 1 x 16384 262 / 31, 32 x 1000
+// 57 / 23, 16 x 4000 106 / 52 (5 TB/s).  Ranges cost a second launch and pay
+// from about 512 keys each: 8 x 64 x 2048 25.3 -> 15.1, 8 x 128 x 4096 44.3 ->
+// 19.0, but 8 x 128 x 512 11.0 -> 12.3 with two.
+struct SplitPlan {
+  bool use = false;
+  int blocks = 0, ranges = 1, range = 0;
+  size_t bytes = 0;  // workspace of the ranges
+};
+
+// BH query heads of nq rows, group of them to a K/V head.
+inline SplitPlan split_plan(int64_t BH, int64_t group, int64_t nq, int64_t nk, int64_t D, bool causal, size_t scratch) {
+  SplitPlan pl;
+  const int64_t cus = device_cu_count(), blocks = cdiv(group * nq, 32), units = BH / group * blocks;
+  if (units > (causal && nq > 128 ? 2 : 1) * cus && nq > 32) return pl;
+  pl.use = true;
+  pl.blocks = static_cast<int>(blocks);
+  int64_t ranges = units > cus / 2 ? 1 : std::max<int64_t>(1, std::min(2 * cus / units, nk / 512));
+  auto size = [&](int64_t n) { return n > 1 ? static_cast<size_t>(units) * n * 32 * (D + 2) * 4 : 0; };
+  if (size(ranges) > scratch) ranges = 1;
+  pl.range = static_cast<int>(cdiv(cdiv(nk, ranges), 32) * 32);
+  pl.ranges = static_cast<int>(cdiv(nk, pl.range));
+  pl.bytes = size(pl.ranges);
+  return pl;
+}
+
+template <int D, bool CAUSAL>
+inline void split_launch(const SplitPlan &pl, SplitArgs p, int64_t BH, int64_t group, hipStream_t s) {
+  const int64_t units = BH / group * pl.blocks;
+  p.blocks = pl.blocks;
+  p.range = pl.range;
+  p.ml_off = units * pl.ranges * 32 * D;
+  if (pl.ranges == 1) p.part = nullptr;
+  hipLaunchKernelGGL((fa_split_bf16<D, CAUSAL>), dim3(pl.ranges, static_cast<unsigned>(units)), dim3(256), 0, s, p);
+  if (pl.ranges > 1) {
+    const int64_t total = BH / group * p.rows;
+    hipLaunchKernelGGL(fa_split_combine<D>, dim3(static_cast<unsigned>(cdiv(total, 4))), dim3(256), 0, s, p, pl.ranges,
+                       total);
+  }
+}
+
+}  // namespace teeny

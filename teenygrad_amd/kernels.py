@@ -1249,6 +1249,16 @@ def attention(q: Buffer, k: Buffer, v: Buffer, q_heads: int, kv_heads: int,
     return o
 
 
+def attention_workspace_size(batch: int, q_heads: int, kv_heads: int, n_ctx_q: int, n_ctx_k: int, head_dim: int,
+                             causal: bool = False, dtype=bf16) -> int:
+    """Stream workspace bytes that let ``attention`` (or ``flash_attention`` with batch = BH and one head) share a
+    head's keys out over the device."""
+    out = ctypes.c_size_t(0)
+    check(lib.teeny_attention_workspace_size(batch, q_heads, kv_heads, n_ctx_q, n_ctx_k, head_dim, int(bool(causal)),
+                                             from_any(dtype).code, ctypes.byref(out)))
+    return int(out.value)
+
+
 def attention_backward(q: Buffer, k: Buffer, v: Buffer, o: Buffer, do: Buffer, lse: Buffer,
                        q_heads: int = 1, kv_heads: int = 1, softmax_scale: Optional[float] = None,
                        causal: bool = False, dq: Optional[Buffer] = None, dk: Optional[Buffer] = None,

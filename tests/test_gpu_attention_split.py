@@ -1,0 +1,65 @@
+"""bf16 attention with few queries per K/V head (the keys shared out over waves
+and, given a workspace, over workgroups) against the CPU oracle."""
+import numpy as np
+import pytest
+
+import teenygrad_amd as tg
+from gpu_util import check_bf16, stream_workspace
+from teenygrad_amd import kernels as K
+from teenygrad_amd.dtypes import from_bf16, to_bf16
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # batch, q_heads, kv_heads, nq, nk, d: rows of a column block, tile and range edges
+    (1, 1, 1, 1, 1, 128), (2, 2, 1, 1, 31, 64), (1, 8, 2, 1, 129, 128), (3, 4, 4, 2, 512, 64),
+    (1, 32, 4, 5, 1000, 128), (2, 8, 1, 4, 257, 64), (1, 3, 1, 32, 700, 128), (1, 2, 2, 31, 2049, 64),
+    (2, 16, 2, 1, 3001, 128), (1, 1, 1, 32, 33, 128)]
+
+
+@pytest.mark.parametrize("b,hq,hkv,nq,nk,d", CASES)
+@pytest.mark.parametrize("scale", [None, -0.1, 0.0])
+def test_few_queries(dev, orc, b, hq, hkv, nq, nk, d, scale):
+    rng = np.random.default_rng(nq + 3 * nk + d)
+    q, k, v = (from_bf16(to_bf16(rng.standard_normal((n, m, d), dtype=np.float32)))
+               for n, m in ((b * hq, nq), (b * hkv, nk), (b * hkv, nk)))
+    scale = 1 / np.sqrt(d) if scale is None else scale
+    oo, ol = orc.flash_attention(q, *(np.repeat(a, hq // hkv, axis=0) for a in (k, v)), scale)
+    bufs = [dev.upload(to_bf16(a), tg.bf16) for a in (q, k, v)]
+    for ws in (K.attention_workspace_size(b, hq, hkv, nq, nk, d), 0):
+        print(f"[attn split] b={b} hq={hq} hkv={hkv} nq={nq} nk={nk} d={d} scale={scale} workspace={ws}", flush=True)
+        lse = tg.Buffer(tg.f32, (b * hq, nq))
+        with stream_workspace(dev, ws):
+            o = K.attention(*bufs, hq, hkv, scale, lse=lse).to_host()
+        check_bf16(o, oo, "o")
+        assert np.max(np.abs(lse.to_host() - ol)) < 1e-3
+
+
+@pytest.mark.parametrize("b,hq,hkv,nq,nk,d", [
+    # rows of one and of several heads in a block, ranges past the last query, keys that no query sees
+    (1, 4, 2, 20, 300, 128), (2, 2, 2, 33, 33, 64), (1, 6, 1, 50, 70, 64), (1, 1, 1, 1500, 1400, 128),
+    (1, 2, 2, 700, 1100, 64), (3, 4, 1, 129, 129, 128)])
+def test_causal(dev, orc, b, hq, hkv, nq, nk, d):
+    rng = np.random.default_rng(nq + 3 * nk + d)
+    q, k, v = (from_bf16(to_bf16(rng.standard_normal((n, m, d), dtype=np.float32)))
+               for n, m in ((b * hq, nq), (b * hkv, nk), (b * hkv, nk)))
+    oo, ol = orc.flash_attention(q, *(np.repeat(a, hq // hkv, axis=0) for a in (k, v)), 1 / np.sqrt(d), True)
+    bufs = [dev.upload(to_bf16(a), tg.bf16) for a in (q, k, v)]
+    for ws in (K.attention_workspace_size(b, hq, hkv, nq, nk, d, True), 0):
+        print(f"[attn split] causal b={b} hq={hq} hkv={hkv} nq={nq} nk={nk} d={d} workspace={ws}", flush=True)
+        lse = tg.Buffer(tg.f32, (b * hq, nq))
+        with stream_workspace(dev, ws):
+            o = K.attention(*bufs, hq, hkv, causal=True, lse=lse).to_host()
+        check_bf16(o, oo, "o")
+        assert np.max(np.abs(lse.to_host() - ol)) < 1e-3
+
+
+def test_rows_past_the_keys(dev, orc):
+    # the head after this one holds no numbers: its rows are read only as padding
+    q, k, v = (from_bf16(to_bf16(np.random.default_rng(1).standard_normal((2, n, 128), dtype=np.float32)))
+               for n in (1, 300, 300))
+    k[1], v[1] = np.nan, np.inf
+    oo, _ = orc.flash_attention(q[:1], k[:1], v[:1])
+    with stream_workspace(dev, K.attention_workspace_size(2, 1, 1, 1, 300, 128)):
+        o = K.flash_attention(*(dev.upload(to_bf16(a), tg.bf16) for a in (q, k, v))).to_host()
+    check_bf16(o[:1], oo, "o")
+    assert np.isnan(from_bf16(o[1])).all()
