@@ -554,9 +554,10 @@ static teeny_status attention_entry(const void *q, const void *k, const void *v,
     TEENY_REQUIRE(n_ctx_k * head_dim * 2 <= 0x7fffffff, TEENY_ERR_SHAPE_MISMATCH,
                   nm + ": bf16 K/V of one head must be below 2 GiB");
     const Scratch scr = stream_scratch(s);
-    const SplitPlan plan = split_plan(BH, group, nq, nk, head_dim, causal != 0, scr.ptr != nullptr ? scr.bytes : 0);
+    const AttnSplitPlan plan =
+        attn_split_plan(BH, group, nq, nk, head_dim, causal != 0, scr.ptr != nullptr ? scr.bytes : 0);
     if (plan.use) {
-      SplitArgs a{};
+      AttnSplitArgs a{};
       a.Q = static_cast<const bf16 *>(q);
       a.K = static_cast<const bf16 *>(k);
       a.V = static_cast<const bf16 *>(v);
@@ -567,8 +568,8 @@ static teeny_status attention_entry(const void *q, const void *k, const void *v,
       a.nq = nq;
       a.nk = nk;
       a.scale_log2 = softmax_scale * kLog2e;
-      if (head_dim == 64) (causal ? split_launch<64, true> : split_launch<64, false>)(plan, a, BH, group, s);
-      else (causal ? split_launch<128, true> : split_launch<128, false>)(plan, a, BH, group, s);
+      if (head_dim == 64) (causal ? attn_split_launch<64, true> : attn_split_launch<64, false>)(plan, a, BH, group, s);
+      else (causal ? attn_split_launch<128, true> : attn_split_launch<128, false>)(plan, a, BH, group, s);
       return after_launch(name, s);
     }
     if (head_dim == 64) launch_bf16<64>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s);
@@ -616,6 +617,7 @@ extern "C" teeny_status teeny_attention_workspace_size(int64_t batch, int64_t q_
   if (batch == 0 || q_heads == 0 || n_ctx_q == 0 || n_ctx_k == 0 || dtype != TEENY_BF16 ||
       (head_dim != 64 && head_dim != 128) || n_ctx_k * head_dim * 2 > 0x7fffffff)
     return TEENY_OK;
-  *bytes = split_plan(batch * q_heads, q_heads / kv_heads, n_ctx_q, n_ctx_k, head_dim, causal != 0, ~size_t{0}).bytes;
+  *bytes = attn_split_plan(batch * q_heads, q_heads / kv_heads, n_ctx_q, n_ctx_k, head_dim, causal != 0, ~size_t{0})
+               .bytes;
   return TEENY_OK;
 }

@@ -46,7 +46,7 @@ template <> struct FaVec4<float> {
 template <> struct FaVec4<bf16> {
   typedef fa_bf16x4u type;
   static __device__ __forceinline__ f32x4 wide(fa_bf16x4u v) {
-    return f32x4{static_cast<float>(v[0]), static_cast<float>(v[1]), static_cast<float>(v[2]), static_cast<float>(v[3])};
+    return f32x4{to_f32(v[0]), to_f32(v[1]), to_f32(v[2]), to_f32(v[3])};
   }
 };
 template <typename T> __device__ __forceinline__ f32x4 fa_load4(const T *p) {
@@ -91,7 +91,8 @@ template <typename T, int D> struct FaTile {
     }
   }
   // Rows past n are zeros.  Whether any value is an infinity or NaN, if asked.
-  template <bool CHECK = false> __device__ __forceinline__ bool store(float *lds, uint32_t r0, uint32_t n, int lane) const {
+  template <bool CHECK = false>
+  __device__ __forceinline__ bool store(float *lds, uint32_t r0, uint32_t n, int lane) const {
     bool odd = false;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -149,7 +150,8 @@ template <int D> struct FaAcc {
     }
   }
   // The same with the rows where seen(row) is false left out, not multiplied by zero.
-  template <typename F> __device__ __forceinline__ void masked_outer(const float *tile, const f32x16 &x, int h, F seen) {
+  template <typename F>
+  __device__ __forceinline__ void masked_outer(const float *tile, const f32x16 &x, int h, F seen) {
     for (int r = 0; r < 16; ++r) {
       float mine = 0.0f;
 #pragma unroll
@@ -184,7 +186,8 @@ template <int D> struct FaAcc {
 // Writes rows c0 .. c0 + 31 (below n) of out [n, D] from the sum of `parts`
 // [D][33] blocks `stride` floats apart; `step` threads, this one `t`.
 template <typename T, int D, int PARTS>
-__device__ __forceinline__ void fa_write(T *out, uint32_t c0, uint32_t n, const float *red, int stride, int t, int step) {
+__device__ __forceinline__ void fa_write(T *out, uint32_t c0, uint32_t n, const float *red, int stride, int t,
+                                         int step) {
   for (int i = t; i < 32 * (D / 4); i += step) {
     const int row = i / (D / 4), d = 4 * (i % (D / 4));
     if (c0 + row >= n) continue;
@@ -320,8 +323,8 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_fwd_f32(const T *__re
 template <typename T, int D, int SPLIT>
 __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_bwd_dq_f32(
     const T *__restrict__ Q, const T *__restrict__ K, const T *__restrict__ V, const T *__restrict__ O,
-    const T *__restrict__ dO, const float *__restrict__ L, T *__restrict__ dQ, float *__restrict__ delta_out, uint32_t nq,
-    uint32_t nk, float scale, int causal, int kv_group, int nqb) {
+    const T *__restrict__ dO, const float *__restrict__ L, T *__restrict__ dQ, float *__restrict__ delta_out,
+    uint32_t nq, uint32_t nk, float scale, int causal, int kv_group, int nqb) {
   using Tile = FaTile<T, D>;
   __shared__ __attribute__((aligned(16))) float lds[4][2 * Tile::FLOATS];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;

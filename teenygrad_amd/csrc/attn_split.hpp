@@ -24,7 +24,7 @@
 
 namespace teeny {
 
-struct SplitArgs {
+struct AttnSplitArgs {
   const bf16 *Q, *K, *V;
   bf16 *O;
   float *L;
@@ -38,7 +38,7 @@ struct SplitArgs {
 };
 
 template <int D, bool CAUSAL>
-__global__ __launch_bounds__(256, 2) void fa_split_bf16(SplitArgs p) {
+__global__ __launch_bounds__(256, 2) void fa_split_bf16(AttnSplitArgs p) {
   constexpr int CPR = D / 8, RPB = 128 / D, NS = D / 16, ND = D / 32, NV = 32 * CPR / 64;
   constexpr int RED = D * 33;  // a wave's partial output [D][33]
   __shared__ __attribute__((aligned(16))) float red[4][RED];
@@ -86,7 +86,8 @@ __global__ __launch_bounds__(256, 2) void fa_split_bf16(SplitArgs p) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int t = 64 * i + lane;
-      vr[i] = *reinterpret_cast<const u32x4 *>(Vb + static_cast<int64_t>(min(k0 + t / CPR, p.nk - 1)) * D + 8 * (t % CPR));
+      const int64_t row = min(k0 + t / CPR, p.nk - 1);
+      vr[i] = *reinterpret_cast<const u32x4 *>(Vb + row * D + 8 * (t % CPR));
     }
   };
   int k0 = kb + 32 * w;
@@ -181,8 +182,10 @@ __global__ __launch_bounds__(256, 2) void fa_split_bf16(SplitArgs p) {
     const int r = i / (D / 4), d = 4 * (i % (D / 4));
     f32x4 o;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      o[j] = (red[0][(d + j) * 33 + r] + red[1][(d + j) * 33 + r]) + (red[2][(d + j) * 33 + r] + red[3][(d + j) * 33 + r]);
+    for (int j = 0; j < 4; ++j) {
+      const int at = (d + j) * 33 + r;
+      o[j] = (red[0][at] + red[1][at]) + (red[2][at] + red[3][at]);
+    }
     if (whole) {
       bf16x4 o4;
 #pragma unroll
@@ -204,7 +207,7 @@ __global__ __launch_bounds__(256, 2) void fa_split_bf16(SplitArgs p) {
 
 // One wave per query row: the ranges' parts, in range order.
 template <int D>
-__global__ __launch_bounds__(256) void fa_split_combine(SplitArgs p, int ranges, int64_t total) {
+__global__ __launch_bounds__(256) void fa_split_combine(AttnSplitArgs p, int ranges, int64_t total) {
   constexpr int V = D / 64;
   const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -243,15 +246,16 @@ __global__ __launch_bounds__(256) void fa_split_combine(SplitArgs p, int ranges,
 // 57 / 23, 16 x 4000 106 / 52 (5 TB/s).  Ranges cost a second launch and pay
 // from about 512 keys each: 8 x 64 x 2048 25.3 -> 15.1, 8 x 128 x 4096 44.3 ->
 // 19.0, but 8 x 128 x 512 11.0 -> 12.3 with two.
-struct SplitPlan {
+struct AttnSplitPlan {
   bool use = false;
   int blocks = 0, ranges = 1, range = 0;
   size_t bytes = 0;  // workspace of the ranges
 };
 
 // BH query heads of nq rows, group of them to a K/V head.
-inline SplitPlan split_plan(int64_t BH, int64_t group, int64_t nq, int64_t nk, int64_t D, bool causal, size_t scratch) {
-  SplitPlan pl;
+inline AttnSplitPlan attn_split_plan(int64_t BH, int64_t group, int64_t nq, int64_t nk, int64_t D, bool causal,
+                                     size_t scratch) {
+  AttnSplitPlan pl;
   const int64_t cus = device_cu_count(), blocks = cdiv(group * nq, 32), units = BH / group * blocks;
   if (units > (causal && nq > 128 ? 2 : 1) * cus && nq > 32) return pl;
   pl.use = true;
@@ -266,7 +270,7 @@ inline SplitPlan split_plan(int64_t BH, int64_t group, int64_t nq, int64_t nk, i
 }
 
 template <int D, bool CAUSAL>
-inline void split_launch(const SplitPlan &pl, SplitArgs p, int64_t BH, int64_t group, hipStream_t s) {
+inline void attn_split_launch(const AttnSplitPlan &pl, AttnSplitArgs p, int64_t BH, int64_t group, hipStream_t s) {
   const int64_t units = BH / group * pl.blocks;
   p.blocks = pl.blocks;
   p.range = pl.range;

@@ -10,11 +10,13 @@
 //
 // bf16 and int8 weights run on the MFMA core (gemm_core.hpp) whenever the
 // operands are K-contiguous and 16-byte aligned, fp32 operands with one unit
-// stride each on the fp32 matrix cores (gemm_f32.hpp); anything else (two odd
+// stride each on the fp32 matrix cores (gemm_f32.hpp), and up to 64 rows of
+// bf16 on weight-streaming waves (gemm_skinny.hpp); anything else (two odd
 // strides, bf16 off the vector grid, ragged K for int8) runs gemm_generic: a
 // 64 x 64 LDS-tiled fp32 FMA kernel that accumulates each output in k order.
 #include "gemm_core.hpp"
 #include "gemm_f32.hpp"
+#include "gemm_skinny.hpp"
 
 namespace teeny {
 
@@ -256,7 +258,8 @@ teeny_status teeny_linear_forward(const void *x, const void *w, const void *b, v
     if (mfma_ok) {
       GemmParams p = plain_params(x, stride_xm, w, stride_wn, y, stride_ym, nullptr, nullptr,
                                   static_cast<const bf16 *>(b), M, N, K);
-      launch_gemm_mfma<false, kAPlain>(p, TEENY_ACT_NONE, s, stream_scratch(s));
+      if (gemm_skinny_ok(false, M, N, K)) launch_gemm_skinny<false>(p, TEENY_ACT_NONE, s);
+      else launch_gemm_mfma<false, kAPlain>(p, TEENY_ACT_NONE, s, stream_scratch(s));
     } else {
       teeny_status st = launch_generic<bf16, bf16, bf16>(
           static_cast<const bf16 *>(x), stride_xm, stride_xk, static_cast<const bf16 *>(w),
@@ -287,7 +290,8 @@ teeny_status teeny_w8a16_linear_forward(const void *x, const int8_t *qweight, co
     GemmParams p = plain_params(x, K, qweight, K, y, N, scale, bias, nullptr, M, N, K);
     // int8 weights stay int8 up to the registers feeding the MFMA (no
     // dequantized copy in HBM)
-    launch_gemm_mfma<true, kAPlain>(p, act, s, stream_scratch(s));
+    if (gemm_skinny_ok(true, M, N, K)) launch_gemm_skinny<true>(p, act, s);
+    else launch_gemm_mfma<true, kAPlain>(p, act, s, stream_scratch(s));
   } else {
     teeny_status st = launch_generic<bf16, int8_t, bf16>(
         static_cast<const bf16 *>(x), K, 1, qweight, K, 1, static_cast<bf16 *>(y), N, 1, scale,
@@ -410,6 +414,7 @@ teeny_status teeny_linear_workspace_size(int64_t M, int64_t N, int64_t K, teeny_
     return TEENY_OK;
   }
   if (K % (dtype == TEENY_I8 ? 16 : 8) != 0) return TEENY_OK;  // generic kernel, no scratch
+  if (gemm_skinny_ok(dtype == TEENY_I8, M, N, K)) return TEENY_OK;
   // contiguous operands, as the MFMA path requires
   const GemmParams p = plain_params(nullptr, K, nullptr, K, nullptr, N, nullptr, nullptr, nullptr, M, N, K);
   *bytes = dtype == TEENY_I8 ? gemm_scratch_bytes<true, kAPlain>(p) : gemm_scratch_bytes<false, kAPlain>(p);

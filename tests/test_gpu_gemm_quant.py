@@ -27,6 +27,34 @@ def test_linear_f32_fixture(dev, orc, with_bias):
     check_f32(got, orc.linear(x, w, b if with_bias else None), "linear f32")
 
 
+SKINNY = [  # (M, N, K): row blocks of 16, column tails, K tails of 16 .. 64, fewer chunks than waves
+    (1, 16, 16), (1, 1, 64), (7, 100, 528), (15, 33, 4096), (16, 48, 80), (17, 65, 1008), (32, 31, 2080), (33, 47, 1040),
+    (64, 130, 4656), (2, 11008, 64)]
+
+
+@pytest.mark.parametrize("m,n,k", SKINNY)
+@pytest.mark.parametrize("weights", ["int8", "bf16"])
+def test_few_rows(dev, m, n, k, weights):
+    rng = np.random.default_rng(m + 3 * n + 5 * k)
+    x = rb(rng.standard_normal((m, k), dtype=np.float32)).reshape(m, k)
+    bias = rb(rng.standard_normal(n, dtype=np.float32))
+    xb = dev.upload(to_bf16(x), tg.bf16)
+    print(f"[few rows] M={m} N={n} K={k} {weights}", flush=True)
+    if weights == "int8":
+        q = rng.integers(-128, 128, (n, k)).astype(np.int8)
+        scale = rng.uniform(0.005, 0.02, n).astype(np.float32)
+        w = q.astype(np.float64) * scale[:, None]
+        got = K.w8a16_linear(xb, dev.upload(q), dev.upload(scale), dev.upload(bias)).to_host()
+    else:
+        w = rb(rng.standard_normal((n, k), dtype=np.float32)).reshape(n, k).astype(np.float64)
+        got = K.linear(xb, dev.upload(to_bf16(w.astype(np.float32)), tg.bf16), dev.upload(to_bf16(bias), tg.bf16)).to_host()
+    ref = x.astype(np.float64) @ w.T + bias
+    # k fp32 sums, each within 2^-24 of at most sum |x| |w|, and the bf16 result
+    bound = (k + 3) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T + np.abs(bias)) + 2.0 ** -8 * np.abs(ref)
+    err = np.abs(from_bf16(got).astype(np.float64).reshape(m, n) - ref)
+    assert np.all(err <= bound), f"{np.max(err - bound)} beyond the bound"
+
+
 F32_GEMM = [  # (M, N, K): tile edges, ragged vectors, k tails, splits, fewer than a 16-byte load spans
     (1, 5, 4), (3, 3, 3), (31, 65, 29), (33, 64, 31), (64, 64, 32), (65, 63, 33), (129, 127, 97), (4, 4, 161),
     (5, 1000, 700), (200, 72, 3001), (2300, 2200, 40)]
