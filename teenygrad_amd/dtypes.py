@@ -21,6 +21,14 @@ class DType:
     host: type
     itemsize: int
 
+    def __eq__(self, other):
+        # nearly always one of the objects below: no field tuples to build
+        if self is other:
+            return True
+        if not isinstance(other, DType):
+            return NotImplemented
+        return (self.name, self.code, self.host, self.itemsize) == (other.name, other.code, other.host, other.itemsize)
+
 
 f32 = DType("f32", _lib.F32, np.float32, 4)
 bf16 = DType("bf16", _lib.BF16, np.uint16, 2)

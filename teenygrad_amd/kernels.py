@@ -95,7 +95,7 @@ class DispatchPacker(ArgVisitor):
 
 
 def _prod(s: Sequence[int]) -> int:
-    return int(np.prod(s)) if len(s) else 1
+    return int(math.prod(s))
 
 
 def _need(cond: bool, msg: str) -> None:
@@ -858,11 +858,13 @@ class LinearForward(RuntimeOp):
 
 def _out(like: Buffer, out: Optional[Buffer], shape=None, dtype=None) -> Buffer:
     """The output buffer: `out` if given (its size and dtype must match), else a new one."""
-    shape = tuple(shape if shape is not None else like.shape)
-    dtype = from_any(dtype or like.dtype)
+    shape = like.shape if shape is None else tuple(shape)
+    dtype = from_any(dtype) if dtype else like.dtype
     if out is not None:
-        _need(out.numel == _prod(shape), f"output holds {out.numel} elements, op writes {_prod(shape)}")
-        _need(out.dtype == dtype, f"output dtype {out.dtype.name}, op writes {dtype.name}")
+        if out.numel != _prod(shape):
+            raise ValueError(f"output holds {out.numel} elements, op writes {_prod(shape)}")
+        if out.dtype != dtype:
+            raise ValueError(f"output dtype {out.dtype.name}, op writes {dtype.name}")
         return out
     return Buffer(dtype, shape)
 
@@ -870,20 +872,24 @@ def _out(like: Buffer, out: Optional[Buffer], shape=None, dtype=None) -> Buffer:
 # Shape rules of each entry point, as pure functions of buffer shapes (so the
 # rules are testable without a device).  Every wrapper below checks its
 # buffers with these before calling the C ABI, which cannot see allocation
-# sizes through raw pointers.
+# sizes through raw pointers.  The checks run on every call, next to launches
+# of 3 us: their messages are formatted only when one fails.
 
 def linear_dims(x_shape, w_shape, b_shape=None) -> Tuple[int, int, int]:
     _need(len(x_shape) == 2 and len(w_shape) == 2, "linear: x and w must be 2-D")
     m, k = x_shape
     n, kw = w_shape
-    _need(k == kw, f"linear: x has K={k}, w has K={kw}")
-    _need(b_shape is None or _prod(b_shape) == n, f"linear: bias must have {n} elements")
+    if k != kw:
+        raise ValueError(f"linear: x has K={k}, w has K={kw}")
+    if not (b_shape is None or _prod(b_shape) == n):
+        raise ValueError(f"linear: bias must have {n} elements")
     return int(m), int(n), int(k)
 
 
 def w8a16_dims(x_shape, q_shape, scale_shape, bias_shape=None) -> Tuple[int, int, int]:
     m, n, k = linear_dims(x_shape, q_shape, bias_shape)
-    _need(_prod(scale_shape) == n, f"w8a16: scale must have N={n} elements, has {_prod(scale_shape)}")
+    if _prod(scale_shape) != n:
+        raise ValueError(f"w8a16: scale must have N={n} elements, has {_prod(scale_shape)}")
     return m, n, k
 
 
@@ -898,10 +904,12 @@ def conv2d_dims(x_shape, w_shape, stride, padding, groups, layout, b_shape=None)
     else:
         b, cin, h, wd = x_shape
         cout, cg, kh, kw = w_shape
-    _need(groups > 0 and cin % groups == 0 and cout % groups == 0,
-          f"conv2d: groups={groups} must divide C_IN={cin} and C_OUT={cout}")
-    _need(cg == cin // groups, f"conv2d: weight has {cg} input channels per group, expected {cin // groups}")
-    _need(b_shape is None or _prod(b_shape) == cout, f"conv2d: bias must have {cout} elements")
+    if not (groups > 0 and cin % groups == 0 and cout % groups == 0):
+        raise ValueError(f"conv2d: groups={groups} must divide C_IN={cin} and C_OUT={cout}")
+    if cg != cin // groups:
+        raise ValueError(f"conv2d: weight has {cg} input channels per group, expected {cin // groups}")
+    if not (b_shape is None or _prod(b_shape) == cout):
+        raise ValueError(f"conv2d: bias must have {cout} elements")
     _need(h + 2 * ph >= kh and wd + 2 * pw >= kw, "conv2d: kernel larger than padded input")
     oh, ow = (h + 2 * ph - kh) // sh + 1, (wd + 2 * pw - kw) // sw + 1
     return b, cin, cout, h, wd, oh, ow, kh, kw, sh, sw, ph, pw
@@ -913,16 +921,20 @@ def attention_dims(q_shape, k_shape, v_shape, lse_shape=None):
     bh, nq, d = q_shape
     _need(tuple(k_shape) == tuple(v_shape), "attention: k and v shapes differ")
     _need(k_shape[0] == bh and k_shape[2] == d, "attention: k/v must share BH and D with q")
-    _need(lse_shape is None or _prod(lse_shape) == bh * nq, f"attention: lse must have {bh * nq} elements")
+    if not (lse_shape is None or _prod(lse_shape) == bh * nq):
+        raise ValueError(f"attention: lse must have {bh * nq} elements")
     return int(bh), int(nq), int(k_shape[1]), int(d)
 
 
 def norm_dims(x_shape, weight_shape, bias_shape=None, rrms_shape=None):
     n = int(x_shape[-1])
     m = _prod(x_shape) // n
-    _need(_prod(weight_shape) == n, f"norm: weight must have N={n} elements")
-    _need(bias_shape is None or _prod(bias_shape) == n, f"norm: bias must have N={n} elements")
-    _need(rrms_shape is None or _prod(rrms_shape) == m, f"norm: rrms must have M={m} elements")
+    if _prod(weight_shape) != n:
+        raise ValueError(f"norm: weight must have N={n} elements")
+    if not (bias_shape is None or _prod(bias_shape) == n):
+        raise ValueError(f"norm: bias must have N={n} elements")
+    if not (rrms_shape is None or _prod(rrms_shape) == m):
+        raise ValueError(f"norm: rrms must have M={m} elements")
     return m, n
 
 
@@ -946,8 +958,8 @@ def silu(x: Buffer, y: Optional[Buffer] = None, stream: Optional[Stream] = None)
 
 def _act_grad(fn, what: str, dy: Buffer, saved: Buffer, dx: Optional[Buffer],
               stream: Optional[Stream]) -> Buffer:
-    _need(dy.dtype == saved.dtype and dy.numel == saved.numel,
-          f"{what}: dy and the saved tensor must match in dtype and size")
+    if not (dy.dtype == saved.dtype and dy.numel == saved.numel):
+        raise ValueError(f"{what}: dy and the saved tensor must match in dtype and size")
     dx = _out(dy, dx)
     check(fn(dy.ptr, saved.ptr, dx.ptr, dy.numel, dy.dtype.code, _h(stream)))
     return dx
@@ -1011,10 +1023,11 @@ def layer_norm_backward(dy: Buffer, x: Buffer, weight: Buffer, mean: Buffer, rst
     """layernorm.rs:300-482: returns dx; dweight / dbias (fp32 [N]) accumulate in place."""
     m, n = norm_dims(x.shape, weight.shape)
     _need(dy.shape == x.shape and dy.dtype == x.dtype and weight.dtype == x.dtype, "layer_norm_backward: dy/x/weight")
-    _need(mean.numel == m and rstd.numel == m and mean.dtype == f32 and rstd.dtype == f32,
-          f"layer_norm_backward: mean/rstd fp32 [{m}]")
+    if not (mean.numel == m and rstd.numel == m and mean.dtype == f32 and rstd.dtype == f32):
+        raise ValueError(f"layer_norm_backward: mean/rstd fp32 [{m}]")
     for g in (dweight, dbias):
-        _need(g is None or (g.numel == n and g.dtype == f32), f"layer_norm_backward: dweight/dbias fp32 [{n}]")
+        if not (g is None or (g.numel == n and g.dtype == f32)):
+            raise ValueError(f"layer_norm_backward: dweight/dbias fp32 [{n}]")
     dx = _out(x, dx)
     check(lib.teeny_layer_norm_backward(dy.ptr, x.ptr, dx.ptr, weight.ptr, dweight.ptr if dweight else None,
                                         dbias.ptr if dbias else None, mean.ptr, rstd.ptr, m, n, x.dtype.code,
@@ -1124,8 +1137,8 @@ def conv2d_bn_act(x: Buffer, w: Buffer, bn_scale: Buffer, bn_shift: Buffer, stri
     b, cin, cout, h, wd, oh, ow, kh, kw, sh, sw, ph, pw = conv2d_dims(
         x.shape, w.shape, stride, padding, groups, "nhwc" if nhwc else "nchw")
     _need(w.dtype == x.dtype, "conv2d_bn_act: w dtype must match x")
-    _need(bn_scale.numel == cout and bn_shift.numel == cout and bn_scale.dtype == f32 and bn_shift.dtype == f32,
-          f"conv2d_bn_act: bn_scale / bn_shift fp32 [{cout}]")
+    if not (bn_scale.numel == cout and bn_shift.numel == cout and bn_scale.dtype == f32 and bn_shift.dtype == f32):
+        raise ValueError(f"conv2d_bn_act: bn_scale / bn_shift fp32 [{cout}]")
     yshape = (b, oh, ow, cout) if nhwc else (b, cout, oh, ow)
     strides = None
     if y_strides is not None:
@@ -1163,7 +1176,8 @@ def conv2d_backward_dx(dy: Buffer, w: Buffer, x_shape, stride=(1, 1), padding=(0
                        layout: str = "nchw", dx: Optional[Buffer] = None, stream: Optional[Stream] = None) -> Buffer:
     """conv2d.rs:171-284: dx of x's shape from dy (y's shape) and w."""
     dims, prm, lay, yshape = _conv_bwd_args(x_shape, w.shape, stride, padding, groups, layout, dy.dtype)
-    _need(tuple(dy.shape) == tuple(yshape) and w.dtype == dy.dtype, f"conv2d_backward_dx: dy must be {yshape}")
+    if not (tuple(dy.shape) == tuple(yshape) and w.dtype == dy.dtype):
+        raise ValueError(f"conv2d_backward_dx: dy must be {yshape}")
     dx = _out(dy, dx, tuple(x_shape))
     check(lib.teeny_conv2d_backward_dx(dy.ptr, w.ptr, dx.ptr, *dims, ctypes.byref(prm), dy.dtype.code, lay,
                                        _h(stream)))
@@ -1174,7 +1188,8 @@ def conv2d_backward_dw(dy: Buffer, x: Buffer, w_shape, stride=(1, 1), padding=(0
                        layout: str = "nchw", dw: Optional[Buffer] = None, stream: Optional[Stream] = None) -> Buffer:
     """conv2d.rs:286-397: dw of w's shape from dy and x."""
     dims, prm, lay, yshape = _conv_bwd_args(x.shape, w_shape, stride, padding, groups, layout, dy.dtype)
-    _need(tuple(dy.shape) == tuple(yshape) and x.dtype == dy.dtype, f"conv2d_backward_dw: dy must be {yshape}")
+    if not (tuple(dy.shape) == tuple(yshape) and x.dtype == dy.dtype):
+        raise ValueError(f"conv2d_backward_dw: dy must be {yshape}")
     dw = _out(dy, dw, tuple(w_shape))
     check(lib.teeny_conv2d_backward_dw(dy.ptr, x.ptr, dw.ptr, *dims, ctypes.byref(prm), dy.dtype.code, lay,
                                        _h(stream)))
@@ -1327,7 +1342,8 @@ def quantize_affine(data: Buffer, shape, granularity="channel", axis=0, group_si
     (qvalues int8, scales f32, zero_points i32, groups u32 or None)."""
     ng = quant_num_groups(shape, granularity, axis, group_size)
     n = _prod(shape)
-    _need(data.dtype == f32 and data.numel == n, f"quantize_affine: data must be fp32 with {n} elements")
+    if not (data.dtype == f32 and data.numel == n):
+        raise ValueError(f"quantize_affine: data must be fp32 with {n} elements")
     q = Buffer(i8, tuple(shape))
     scales = Buffer(f32, (max(ng, 1),))
     zps = Buffer("i32", (max(ng, 1),))
@@ -1344,8 +1360,8 @@ def dequantize_affine(q: Buffer, scales: Buffer, zero_points: Optional[Buffer], 
                       stream: Optional[Stream] = None) -> Buffer:
     ng = quant_num_groups(shape, granularity, axis, group_size)
     _need(q.numel == _prod(shape) and q.dtype == i8, "dequantize_affine: q must be int8 of the shape")
-    _need(scales.numel >= ng and (zero_points is None or zero_points.numel >= ng),
-          f"dequantize_affine: scales/zero_points need {ng} entries")
+    if not (scales.numel >= ng and (zero_points is None or zero_points.numel >= ng)):
+        raise ValueError(f"dequantize_affine: scales/zero_points need {ng} entries")
     out = _out(q, out, tuple(shape), f32)
     sh = (ctypes.c_int64 * max(1, len(shape)))(*shape)
     check(lib.teeny_dequantize_affine(q.ptr, scales.ptr,
@@ -1372,7 +1388,8 @@ def linear_backward(x: Buffer, w: Buffer, dy: Buffer, use_bias: bool = True, dx:
     -> (dx [M,K] = dy w, dw [N,K] = dy^T x, db [N] = column sums of dy, or
     None without bias).  Written, not accumulated."""
     m, n, k = linear_dims(x.shape, w.shape)
-    _need(tuple(dy.shape) == (m, n), f"linear_backward: dy must be [{m}, {n}], is {list(dy.shape)}")
+    if tuple(dy.shape) != (m, n):
+        raise ValueError(f"linear_backward: dy must be [{m}, {n}], is {list(dy.shape)}")
     _need(w.dtype == x.dtype and dy.dtype == x.dtype, "linear_backward: x/w/dy dtypes differ")
     dx = _out(x, dx, (m, k))
     dw = _out(x, dw, (n, k))
@@ -1408,7 +1425,8 @@ def w8a16_conv2d(x: Buffer, qweight: Buffer, scale: Buffer, bias: Optional[Buffe
     """x NHWC bf16 [B,H,W,Cin], qweight int8 [Cout,KH,KW,Cin/G], scale f32 [Cout]."""
     b, cin, cout, h, wd, oh, ow, kh, kw, sh, sw, ph, pw = conv2d_dims(
         x.shape, qweight.shape, stride, padding, groups, "nhwc", bias.shape if bias is not None else None)
-    _need(_prod(scale.shape) == cout, f"w8a16_conv2d: scale must have {cout} elements")
+    if _prod(scale.shape) != cout:
+        raise ValueError(f"w8a16_conv2d: scale must have {cout} elements")
     _need(x.dtype == bf16 and qweight.dtype == i8 and scale.dtype == f32 and
           (bias is None or bias.dtype == f32), "w8a16_conv2d: x bf16, qweight int8, scale/bias fp32")
     y = _out(x, y, (b, oh, ow, cout), bf16)
