@@ -267,6 +267,25 @@ __global__ __launch_bounds__(256) void fa_bwd_delta_bf16(const bf16 *__restrict_
   if (row < rows && t % CPR == 0) delta[row] = s;
 }
 
+// Block order of a causal grid: workgroup `id` of nb blocks per head (block
+// 0 the longest, nb - 1 the shortest) -> (head, block).  An XCD takes
+// consecutive ids and has 64 workgroups resident, two per CU, the id 32 later
+// being the second one of a CU.  Heads go in groups that fill those 64 slots:
+// the first half of a group's ids are its longer blocks, longest first, and
+// the second half the others, shortest first, so that a CU's two workgroups
+// add up to the same length everywhere.  (In head order both are the same
+// block of two heads, and the longest pair sets the time.)  With the masks
+// compared on edge tiles only (dq, and dk/dv at head_dim 64), dq + dk/dv in
+// us: 64 heads x 1024 x 64 87 -> 68, 256 x 2048 x 128 1306 -> 1177, 64 x 1024
+// x 128 139 -> 122.  More than 64 blocks per head: plain, longest first.
+__device__ __forceinline__ void causal_order(int id, int nb, int heads, int &head, int &blk) {
+  const int per = nb > 64 ? 1 : max(1, min(64 / nb, heads / 8));
+  const int g0 = id / (per * nb) * per, n = min(per, heads - g0), j = id - g0 * nb;
+  const int half = nb > 64 ? nb : (nb + 1) / 2, i = j / n;
+  head = g0 + j - i * n;
+  blk = i < half ? i : nb - 1 - (i - half);
+}
+
 // dK, dV for the 32 * WAVES keys of one workgroup (wave w: keys k0 + 0..31),
 // head_dim 64.  (At head_dim 128 the K^T / V^T operands and both
 // accumulators take 192 of a lane's registers: one workgroup per CU; that
@@ -282,7 +301,8 @@ __global__ __launch_bounds__(64 * WAVES, (D == 128 ? 4 : 8) / WAVES) void fa_bwd
   __shared__ __attribute__((aligned(16))) float lbuf[2][BM], dbuf[2][BM];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 5, c = lane & 31;
   const int tile_id = xcd_remap(blockIdx.x, gridDim.x);
-  const int bhk = tile_id / nkb, kblk = tile_id % nkb;
+  int bhk = tile_id / nkb, kblk = tile_id % nkb;
+  if (CAUSAL) causal_order(tile_id, nkb, gridDim.x / nkb, bhk, kblk);  // key block 0 meets every query
   const int kb0 = kblk * BN, k0 = kb0 + 32 * w, key = k0 + c;
   const bf16 *Kr = K + (static_cast<int64_t>(bhk) * nk + key) * D;
   const bf16 *Vr = V + (static_cast<int64_t>(bhk) * nk + key) * D;
@@ -342,15 +362,19 @@ __global__ __launch_bounds__(64 * WAVES, (D == 128 ? 4 : 8) / WAVES) void fa_bwd
 #pragma unroll
       for (int a = 0; a < 4; ++a) {
         const f32x4 l4 = *reinterpret_cast<const f32x4 *>(&lbuf[b][32 * sb + 8 * a + 4 * g]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) p[4 * a + e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * a + e], sc, -l4[e]));
+      }
+      if (CAUSAL && q0 < k0 + 31) {  // a branch, so that only the diagonal's tiles compare
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int v = 0; v < 16; ++v) p[v] = key > q0 + mfma32_row(v, g) ? 0.0f : p[v];
+      }
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
         const f32x4 d4 = *reinterpret_cast<const f32x4 *>(&dbuf[b][32 * sb + 8 * a + 4 * g]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int v = 4 * a + e;
-          float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], sc, -l4[e]));
-          if (CAUSAL && key > q0 + 8 * a + 4 * g + e) pv = 0.0f;
-          p[v] = pv;
-          ds[v] = pv * (dp[v] - d4[e]);
-        }
+        for (int e = 0; e < 4; ++e) ds[4 * a + e] = p[4 * a + e] * (dp[4 * a + e] - d4[e]);
       }
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
@@ -392,7 +416,8 @@ __global__ __launch_bounds__(256, 2) void fa_bwd_dkv_vl_bf16(
   __shared__ __attribute__((aligned(16))) float lbuf[2][BM], dbuf[2][BM];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 5, c = lane & 31;
   const int tile_id = xcd_remap(blockIdx.x, gridDim.x);
-  const int bhk = tile_id / nkb, kblk = tile_id % nkb;
+  int bhk = tile_id / nkb, kblk = tile_id % nkb;
+  if (CAUSAL) causal_order(tile_id, nkb, gridDim.x / nkb, bhk, kblk);  // key block 0 meets every query
   const int kb0 = kblk * BN, k0 = kb0 + 32 * w, key = k0 + c;
   const bf16 *Kr = K + (static_cast<int64_t>(bhk) * nk + key) * D;
   // the workgroup's V rows (rows past nk read as zeros), one DMA pass
@@ -454,6 +479,8 @@ __global__ __launch_bounds__(256, 2) void fa_bwd_dkv_vl_bf16(
         for (int e = 0; e < 4; ++e) {
           const int v = 4 * a + e;
           float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], sc, -l4[e]));
+          // compared on every tile: behind a branch for the diagonal's tiles
+          // all of p and dP stay live and the wave spills (1.29 -> 1.61 ms)
           if (CAUSAL && key > q0 + 8 * a + 4 * g + e) pv = 0.0f;
           p[v] = pv;
           ds[v] = pv * (dp[v] - d4[e]);
@@ -494,8 +521,11 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void fa_bwd_dq_bf16(
   __shared__ __attribute__((aligned(16))) bf16 kbuf[2][TILE], vbuf[2][TILE];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 5, c = lane & 31;
   const int tile_id = xcd_remap(blockIdx.x, gridDim.x);
-  const int bh = tile_id / nqb, slot = tile_id % nqb;
-  const int qb = CAUSAL ? nqb - 1 - slot : slot;  // causal: heaviest blocks first
+  int bh = tile_id / nqb, qb = tile_id % nqb;
+  if (CAUSAL) {  // the last query block meets every key
+    causal_order(tile_id, nqb, gridDim.x / nqb, bh, qb);
+    qb = nqb - 1 - qb;
+  }
   const int q0 = qb * BM + 32 * w, qi = q0 + c;
   const int64_t qrow = static_cast<int64_t>(bh) * nq + qi;
   bf16x8 qT[NS], doT[NS];
@@ -552,12 +582,17 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void fa_bwd_dq_bf16(
       }
       float ds[16];
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int kv = kbase + mfma32_row(v, g);
-        float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], sc, -l2));
-        if (kv >= nk || (CAUSAL && kv > qi)) pv = 0.0f;
-        ds[v] = pv * (dp[v] - delta);
+      for (int v = 0; v < 16; ++v) ds[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[v], sc, -l2));
+      if (kbase + 32 > nk || (CAUSAL && kbase + 31 > q0)) {  // a branch, so that only edge tiles compare
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int kv = kbase + mfma32_row(v, g);
+          ds[v] = kv >= nk || (CAUSAL && kv > qi) ? 0.0f : ds[v];
+        }
       }
+#pragma unroll
+      for (int v = 0; v < 16; ++v) ds[v] *= dp[v] - delta;
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const bf16x8 db8 = pack_b(ds, t);
