@@ -718,28 +718,20 @@ inline int64_t tiles_of(const GemmParams &p, int bm, int bn) {
   return static_cast<int64_t>((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
 }
 
-// Host launcher: 128 x 128 x 64 tiles (two workgroups per CU); narrow
-// outputs (N <= 64, e.g. the 64-channel convs) and grids that 128 x 128
-// tiles leave short of the CU count take 128 x 64 x 32 tiles with a
-// two-tile prefetch.  Measured on MI355X, larger tiles (256 x 128,
-// 256 x 256 with AGPR accumulators and one workgroup per CU) were no faster
-// for these shapes.
-// Split-K factor for a BM x BN x BK tiling: only deep-K problems (K >= 2048)
-// whose tiles cover fewer than half the CUs (ResNet stage 4: 100 tiles, K =
-// 2048 and 4608) are split, towards two workgroups per CU, with at most
-// four splits (the fp32 partials cost 8 * S * M * N bytes of extra
-// traffic).  Measured on MI355X: at 196 tiles (stage 3) splitting does not
-// pay; the 7x7 3x3 512 -> 512 layers (K = 4608) take 36 us with four
-// splits against 44, 41, 43 and 44 us with 2, 3, 6 and 8.
-inline int splitk_factor(const GemmParams &p, int bm, int bn, int bk) {
-  const int64_t tiles = tiles_of(p, bm, bn);
-  const int n_k = (p.K + bk - 1) / bk;
-  const int64_t cus = device_cu_count();
-  const int64_t target = 2 * cus;
-  if (2 * tiles >= cus || n_k * bk < 2048) return 1;
-  int sp = static_cast<int>((target + tiles - 1) / tiles);
-  sp = min(sp, min(4, n_k / 4));
-  return max(sp, 1);
+// Split-K factor of the 64 x 64 x 64 tiles: four slices of a deep K (2048 or
+// more) when the tiles fill the CUs at most once and the k-tiles per slice
+// outweigh the slices' fp32 traffic and their reduction, which grow with the
+// tile count.  Measured in us, one slice / four: 100 x 512 x 2048 12.2 / 10.1,
+// 250 x 1024 x 4096 21.4 / 14.0, 256 x 2048 x 8192 39.1 / 23.5, int8 514 x
+// 1792 x 7168 41.1 / 35.9, but 784 x 512 x 2048 12.7 / 14.0, 1000 x 1024 x
+// 4096 22.8 / 24.8 (M x N x K).  Up to half as many tiles more than CUs leave
+// most CUs idle in the second round, which slices of a K from 4608 on fill:
+// 2304 x 512 x 4608 35.2 / 29.0, 1100 x 1024 x 8192 54.5 / 41.5; 1500 x 1024 x
+// 4096 29.5 / 30.7.  (So the slices take 25 MB at most.)
+inline int splitk_factor(const GemmParams &p) {
+  const int64_t tiles = tiles_of(p, 64, 64), n_k = (p.K + 63) / 64, cus = device_cu_count();
+  if (tiles <= cus) return n_k >= 32 && 3 * n_k >= tiles ? 4 : 1;
+  return 2 * tiles <= 3 * cus && n_k >= 72 ? 4 : 1;
 }
 
 // Split plan: how many K slices hold k-tiles and the bytes of their fp32
@@ -750,12 +742,11 @@ struct SplitPlan {
   size_t bytes = 0;
 };
 
-template <int BM, int BN, int BK>
 inline SplitPlan split_plan(const GemmParams &p) {
   SplitPlan sp;
-  const int f = splitk_factor(p, BM, BN, BK);
+  const int f = splitk_factor(p);
   if (f > 1) {
-    const int n_k = (p.K + BK - 1) / BK;
+    const int n_k = (p.K + 63) / 64;
     sp.kt_split = (n_k + f - 1) / f;
     sp.used = (n_k + sp.kt_split - 1) / sp.kt_split;
     sp.bytes = static_cast<size_t>(sp.used) * p.M * p.N * sizeof(float);
@@ -765,20 +756,20 @@ inline SplitPlan split_plan(const GemmParams &p) {
 
 // Runs split along K when the plan splits and the caller's scratch holds the
 // partial sums; otherwise unsplit (same products, one accumulation chain).
-template <int BM, int BN, int BK, int WAVES_M, int PF, bool INT8B, int AMODE>
+template <bool INT8B, int AMODE>
 inline void launch_split(GemmParams p, hipStream_t s, Scratch scr) {
-  const SplitPlan sp = split_plan<BM, BN, BK>(p);
+  const SplitPlan sp = split_plan(p);
   if (sp.used > 1 && scr.ptr != nullptr && scr.bytes >= sp.bytes) {
     p.ws = static_cast<float *>(scr.ptr);
     p.kt_split = sp.kt_split;
-    launch_tile<BM, BN, BK, WAVES_M, PF, INT8B, AMODE>(p, s, sp.used);
+    launch_tile<64, 64, 64, 2, 2, INT8B, AMODE>(p, s, sp.used);
     const int64_t groups = static_cast<int64_t>(p.M) * ((p.N + 7) / 8);
     hipLaunchKernelGGL(gemm_splitk_finalize, dim3(static_cast<unsigned>((groups + 255) / 256)), dim3(256), 0,
                        s, p, sp.used);
     return;
   }
   p.ws = nullptr;
-  launch_tile<BM, BN, BK, WAVES_M, PF, INT8B, AMODE>(p, s);
+  launch_tile<64, 64, 64, 2, 2, INT8B, AMODE>(p, s);
 }
 
 template <bool INT8B, int AMODE>
@@ -803,14 +794,19 @@ inline void launch_persist_default(const GemmParams &p, hipStream_t s);
 //  * the 256 x 256 LDS-DMA kernel (gemm_dma.hpp) when its tiles fill the chip;
 //  * narrow outputs (N <= 64): 64 x 64 x 64 tiles for deep K (more
 //    workgroups to hide latency), else 128 x 64 x 32;
+//  * grids of 128 x 128 tiles that leave CUs idle: 128 x 64 x 64 if those
+//    fill the CUs, else 64 x 64 x 64, split along K where that pays.  A tile's
+//    time per k-tile is the CU's LDS traffic for it (its operands written,
+//    and read 1 to 2 KiB per MFMA), so on a CU with one workgroup the smaller
+//    tile is done sooner: in us, 128 x 64 / 64 x 64 tiles, M x N x K: 196 x
+//    1024 x 256 5.6 / 5.2, 3136 x 256 x 1024 10.5 / 8.5, 500 x 1024 x 1024
+//    10.6 / 8.3, 4000 x 256 x 768 9.1 / 7.4; but 2000 x 1024 x 4096 (256 tiles
+//    of 128 x 64) 30.6 / 33.6;
 //  * short K (<= 256, the 1x1 convs): 128 x 128 x 32 with a two-tile
 //    prefetch, so the few k-tiles still overlap loads with MFMAs;
-//  * grids of 128 x 128 tiles that leave CUs idle and do not split along K:
-//    128 x 64 x 64 (twice the workgroups);
-//  * otherwise 128 x 128 x 64, split along K when badly under-filled (the
-//    int8 3x3 conv 32 x 256 x 28 x 28 -> 256, 392 tiles: 48.7 us, against
-//    54.4 us for 128 x 128 x 32 with the two-tile prefetch and 70 us for
-//    128 x 64 x 64).
+//  * otherwise 128 x 128 x 64 (two workgroups per CU; the int8 3x3 conv 32 x
+//    256 x 28 x 28 -> 256, 392 tiles: 48.7 us, against 54.4 us for 128 x 128 x
+//    32 with the two-tile prefetch and 70 us for 128 x 64 x 64).
 enum GemmTiles { kTilesPersist, kTilesStream, kTilesBig, kTiles128x64, kTiles64x64, kTiles128x128Short, kTiles128x64Deep, kTiles128x128 };
 
 template <bool INT8B, int AMODE>
@@ -822,27 +818,16 @@ inline GemmTiles gemm_tiles(const GemmParams &p) {
     if (plain_rows && big_gemm_fits<INT8B, AMODE>(p)) return kTilesBig;
   }
   if (p.N <= 64) return p.K >= 512 ? kTiles64x64 : kTiles128x64;
-  if (p.K <= 256) return kTiles128x128Short;
-  // 128 x 64 tiles with a two-tile prefetch when 128 x 128 tiles leave CUs
-  // idle: unsplit up to K = 2048 (7x7 2048 -> 512: 17.5 us against 25 us
-  // for four K slices plus their reduction), split beyond (a 4608-deep K
-  // chain of 72 k-tiles is long enough that slicing it wins)
-  if (tiles_of(p, 128, 128) < device_cu_count() && (split_plan<128, 128, 64>(p).used == 1 || p.K <= 2048))
-    return kTiles128x64Deep;
-  return kTiles128x128;
+  const int64_t cus = device_cu_count();
+  if (tiles_of(p, 128, 128) < cus)
+    return tiles_of(p, 128, 64) < cus || splitk_factor(p) > 1 ? kTiles64x64 : kTiles128x64Deep;
+  return p.K <= 256 ? kTiles128x128Short : kTiles128x128;
 }
 
 // Scratch bytes that let launch_gemm_mfma take its split plan (0: none used).
 template <bool INT8B, int AMODE>
 inline size_t gemm_scratch_bytes(const GemmParams &p) {
-  switch (gemm_tiles<INT8B, AMODE>(p)) {
-    case kTiles128x64: return split_plan<128, 64, 32>(p).bytes;
-    case kTiles64x64: return split_plan<64, 64, 64>(p).bytes;
-    case kTiles128x128Short: return split_plan<128, 128, 32>(p).bytes;
-    case kTiles128x64Deep: return split_plan<128, 64, 64>(p).bytes;
-    case kTiles128x128: return split_plan<128, 128, 64>(p).bytes;
-    default: return 0;
-  }
+  return gemm_tiles<INT8B, AMODE>(p) == kTiles64x64 ? split_plan(p).bytes : 0;
 }
 
 // Byte extents of the A and B operands as the kernels address them.
@@ -931,11 +916,11 @@ inline bool launch_gemm_mfma(GemmParams p, int act, hipStream_t s, Scratch scr) 
     case kTilesBig:
       if constexpr (AMODE != kAConvScalar) launch_big_gemm<INT8B, AMODE>(p, s);
       break;
-    case kTiles128x64: launch_split<128, 64, 32, 2, 2, INT8B, AMODE>(p, s, scr); break;
-    case kTiles64x64: launch_split<64, 64, 64, 2, 2, INT8B, AMODE>(p, s, scr); break;
-    case kTiles128x128Short: launch_split<128, 128, 32, 2, 2, INT8B, AMODE>(p, s, scr); break;
-    case kTiles128x64Deep: launch_split<128, 64, 64, 2, 2, INT8B, AMODE>(p, s, scr); break;
-    default: launch_split<128, 128, 64, 2, 1, INT8B, AMODE>(p, s, scr); break;
+    case kTiles128x64: launch_tile<128, 64, 32, 2, 2, INT8B, AMODE>(p, s); break;
+    case kTiles64x64: launch_split<INT8B, AMODE>(p, s, scr); break;
+    case kTiles128x128Short: launch_tile<128, 128, 32, 2, 2, INT8B, AMODE>(p, s); break;
+    case kTiles128x64Deep: launch_tile<128, 64, 64, 2, 2, INT8B, AMODE>(p, s); break;
+    default: launch_tile<128, 128, 64, 2, 1, INT8B, AMODE>(p, s); break;
   }
   return true;
 }

@@ -27,6 +27,40 @@ def test_linear_f32_fixture(dev, orc, with_bias):
     check_f32(got, orc.linear(x, w, b if with_bias else None), "linear f32")
 
 
+SMALL_GRID = [  # (M, N, K, K slices): 64 x 64 tiles with ragged edges, unsplit and in four slices of ragged K
+    (65, 65, 64, 1), (130, 72, 272, 1), (1000, 520, 1040, 1), (100, 200, 2048, 4), (257, 130, 2064, 4),
+    (70, 1000, 4112, 4), (1023, 1024, 4096, 1), (1100, 1000, 4624, 4)]
+
+
+@pytest.mark.parametrize("m,n,k,slices", SMALL_GRID)
+@pytest.mark.parametrize("weights", ["int8", "bf16"])
+def test_small_grids(dev, m, n, k, slices, weights):
+    rng = np.random.default_rng(m + 3 * n + 5 * k)
+    x = rb(rng.standard_normal((m, k), dtype=np.float32)).reshape(m, k)
+    bias = rb(rng.standard_normal(n, dtype=np.float32))
+    xb = dev.upload(to_bf16(x), tg.bf16)
+    need = K.linear_workspace_size(m, n, k, tg.i8 if weights == "int8" else tg.bf16)
+    if dev.info()["compute_units"] == 256:
+        assert need == (slices * m * n * 4 if slices > 1 else 0), need
+    if weights == "int8":
+        q = rng.integers(-128, 128, (n, k)).astype(np.int8)
+        scale = rng.uniform(0.005, 0.02, n).astype(np.float32)
+        w, args = q.astype(np.float64) * scale[:, None], (dev.upload(q), dev.upload(scale), dev.upload(bias))
+        fn = K.w8a16_linear
+    else:
+        w = rb(rng.standard_normal((n, k), dtype=np.float32)).reshape(n, k).astype(np.float64)
+        args, fn = (dev.upload(to_bf16(w.astype(np.float32)), tg.bf16), dev.upload(to_bf16(bias), tg.bf16)), K.linear
+    ref = x.astype(np.float64) @ w.T + bias
+    # k fp32 sums, each within 2^-24 of at most sum |x| |w|, and the bf16 result
+    bound = (k + 8) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T + np.abs(bias)) + 2.0 ** -8 * np.abs(ref)
+    for ws in {need, 0}:
+        print(f"[small grid] M={m} N={n} K={k} {weights} workspace={ws}", flush=True)
+        with stream_workspace(dev, ws):
+            got = fn(xb, *args).to_host()
+        err = np.abs(from_bf16(got).astype(np.float64).reshape(m, n) - ref)
+        assert np.all(err <= bound), f"{np.max(err - bound)} beyond the bound"
+
+
 SKINNY = [  # (M, N, K): row blocks of 16, column tails, K tails of 16 .. 64, fewer chunks than waves
     (1, 16, 16), (1, 1, 64), (7, 100, 528), (15, 33, 4096), (16, 48, 80), (17, 65, 1008), (32, 31, 2080), (33, 47, 1040),
     (64, 130, 4656), (2, 11008, 64)]
