@@ -1231,8 +1231,12 @@ static DwPlan dw_plan(const ConvGeo &q, size_t workspace) {
   d.tiles_m = static_cast<int>(cdiv(M, kDwTile));
   d.tiles_n = static_cast<int>(cdiv(N, kDwTile));
   const int64_t tiles = static_cast<int64_t>(d.tiles_m) * d.tiles_n, stages = cdiv(P, kDwStage);
-  int64_t splits = cdiv(2 * static_cast<int64_t>(device_cu_count()), tiles);  // about two workgroups per CU
-  splits = std::min<int64_t>(splits, std::max<int64_t>(1, stages / 4));       // at least 4 stages per split
+  // as many as two workgroups per CU hold at once (one split more of the 144
+  // tiles of 7x7 512 -> 512 at batch 64 starts a second round: 57 us of dw
+  // against 34), and at least 7 stages each, next to which the fp32 partials
+  // are cheap (14x14 256 -> 256 at batch 16 with 4 / 7 stages 23.5 / 20.1 us)
+  int64_t splits = std::max<int64_t>(1, 2 * static_cast<int64_t>(device_cu_count()) / tiles);
+  splits = std::min<int64_t>(splits, std::max<int64_t>(1, stages / 7));
   while (splits > 1 && static_cast<size_t>(splits) * M * N * 4 > workspace) --splits;
   d.stages_per_split = static_cast<int>(cdiv(stages, splits));
   d.splits = static_cast<int>(cdiv(stages, d.stages_per_split));  // no empty split
@@ -1244,7 +1248,9 @@ static DwPlan dw_plan(const ConvGeo &q, size_t workspace) {
 // The split count the kernel would like (what the workspace-size query reports).
 static size_t dw_scratch_bytes(const ConvGeo &q) { return dw_plan(q, static_cast<size_t>(1) << 26).part_bytes; }
 
-template <bool PART>
+// ROWS: a 1x1 stride-1 conv without padding (and linear_backward's dw): the
+// rows of x are the pixels themselves.
+template <bool PART, bool ROWS>
 __global__ __launch_bounds__(256, 2) void conv_dw_mfma(const bf16 *__restrict__ dy, const bf16 *__restrict__ x,
                                                        bf16 *__restrict__ dw, float *__restrict__ part, ConvGeo q,
                                                        int tiles_m, int tiles_n, int stages_per_split, int P) {
@@ -1268,28 +1274,62 @@ __global__ __launch_bounds__(256, 2) void conv_dw_mfma(const bf16 *__restrict__ 
   const int lrow = tid >> 4;
   const int chunk = (tid & 15) ^ bswz<128>(lrow);
   const int a_col = co0 + 8 * chunk;
-  const bool a_ok = a_col < M;
   const int nb = n0 + 8 * chunk;
-  const bool b_ok = nb < N;
   const int tap = nb / q.Cin, ci = nb % q.Cin;  // C_IN % 8 == 0: a chunk never straddles two taps
   const int kh = tap / q.KW, kw = tap % q.KW;
-  auto issue = [&](int s, int b) __attribute__((always_inline)) {
-    const int p0 = (st0 + s) * kDwStage;
+  // Byte offsets of the thread's four rows of the next stage, advanced by 64
+  // pixels per stage with adds: dividing the pixel index of every row of every
+  // stage took longer than the stage's products (dw of 2000 x 1024 -> 4096
+  // 46 -> 34 us, of 28x28 3x3 128 -> 128 at batch 64 38.5 -> 30.7 us).  Rows
+  // past the last pixel lie past the extents, a column past the edge starts at
+  // kOffNone and stays above them, and both read as zeros.
+  const int rpx = ROWS ? 0 : q.OW * q.OH;
+  const int d_bb = ROWS ? 0 : kDwStage / rpx, d_oh = ROWS ? 0 : kDwStage % rpx / q.OW, d_ow = ROWS ? 0 : kDwStage % q.OW;
+  const int px = q.Cin * 2;  // bytes per pixel of x
+  const int step = ROWS ? kDwStage * px : ((d_bb * q.H + d_oh * q.SH) * q.W + d_ow * q.SW) * px;
+  const int wrap_w = (q.SH * q.W - q.OW * q.SW) * px, wrap_h = (q.H - q.OH * q.SH) * q.W * px;
+  const int lim_w = q.OW * q.SW - q.PW + kw, lim_h = q.OH * q.SH - q.PH + kh;
+  uint32_t aoff[4], boff[4];
+  int ih[4], iw[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int p = st0 * kDwStage + 16 * i + lrow;
+    aoff[i] = a_col < M ? (p * M + a_col) * 2 : kOffNone;
+    if constexpr (ROWS) {
+      ih[i] = iw[i] = 0;
+      boff[i] = nb < N ? p * px + ci * 2 : kOffNone;
+    } else {
+      const int r = p / q.OW, bb = r / q.OH;
+      iw[i] = (p - r * q.OW) * q.SW - q.PW + kw;
+      ih[i] = (r - bb * q.OH) * q.SH - q.PH + kh;
+      boff[i] = ((bb * q.H + ih[i]) * q.W + iw[i]) * px + ci * 2;
+    }
+  }
+  // the next stage's DMA into buffer b
+  auto issue = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int p = p0 + 16 * i + lrow;
-      int aoff = kOffNone, boff = kOffNone;
-      if (p < P) {
-        if (a_ok) aoff = (p * M + a_col) * 2;
-        if (b_ok) {
-          const int ow = p % q.OW, r = p / q.OW;
-          const int oh = r % q.OH, bb = r / q.OH;
-          const int ih = oh * q.SH - q.PH + kh, iw = ow * q.SW - q.PW + kw;
-          if (ih >= 0 && ih < q.H && iw >= 0 && iw < q.W) boff = (((bb * q.H + ih) * q.W + iw) * q.Cin + ci) * 2;
-        }
+      uint32_t xo = boff[i];
+      if constexpr (!ROWS) {
+        const bool in = static_cast<unsigned>(ih[i]) < static_cast<unsigned>(q.H) &
+                        static_cast<unsigned>(iw[i]) < static_cast<unsigned>(q.W) & nb < N;
+        xo = in ? xo : kOffNone;
       }
-      buffer_lds_dma16(dys, aoff, __builtin_amdgcn_readfirstlane(lds_address(abuf[b] + (NT * i + 64 * w) * 8)));
-      buffer_lds_dma16(xs, boff, __builtin_amdgcn_readfirstlane(lds_address(bbuf[b] + (NT * i + 64 * w) * 8)));
+      buffer_lds_dma16(dys, aoff[i], __builtin_amdgcn_readfirstlane(lds_address(abuf[b] + (NT * i + 64 * w) * 8)));
+      buffer_lds_dma16(xs, xo, __builtin_amdgcn_readfirstlane(lds_address(bbuf[b] + (NT * i + 64 * w) * 8)));
+      aoff[i] += kDwStage * M * 2;
+      boff[i] += step;
+      if constexpr (!ROWS) {
+        iw[i] += d_ow * q.SW;
+        ih[i] += d_oh * q.SH;
+        const bool ow_wraps = iw[i] >= lim_w;
+        iw[i] -= ow_wraps ? q.OW * q.SW : 0;
+        ih[i] += ow_wraps ? q.SH : 0;
+        boff[i] += ow_wraps ? wrap_w : 0;
+        const bool oh_wraps = ih[i] >= lim_h;
+        ih[i] -= oh_wraps ? q.OH * q.SH : 0;
+        boff[i] += oh_wraps ? wrap_h : 0;
+      }
     }
   };
   f32x16 acc[2][2];
@@ -1298,13 +1338,13 @@ __global__ __launch_bounds__(256, 2) void conv_dw_mfma(const bf16 *__restrict__ 
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = zero16();
   if (nst > 0) {
-    issue(0, 0);
+    issue(0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   }
   for (int s = 0; s < nst; ++s) {
     const int b = s & 1;
-    if (s + 1 < nst) issue(s + 1, b ^ 1);
+    if (s + 1 < nst) issue(b ^ 1);
 #pragma unroll
     for (int kk = 0; kk < kDwStage / 16; ++kk) {
       bf16x8 af[2], bfr[2];
@@ -1412,11 +1452,13 @@ static bool conv_dw_mfma_launch(const void *dy, const void *x, void *dw, const C
   if (!d.ok) return false;
   const int P = q.B * q.OH * q.OW;
   const dim3 grid(static_cast<unsigned>(d.tiles_m * d.tiles_n * d.splits));
+  const bool rows = q.KH == 1 && q.KW == 1 && q.SH == 1 && q.SW == 1 && q.PH == 0 && q.PW == 0;
+  float *part = d.splits > 1 ? static_cast<float *>(scr.ptr) : nullptr;
+  auto kern = d.splits > 1 ? (rows ? conv_dw_mfma<true, true> : conv_dw_mfma<true, false>)
+                           : (rows ? conv_dw_mfma<false, true> : conv_dw_mfma<false, false>);
+  hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, static_cast<const bf16 *>(dy), static_cast<const bf16 *>(x),
+                     static_cast<bf16 *>(dw), part, q, d.tiles_m, d.tiles_n, d.stages_per_split, P);
   if (d.splits > 1) {
-    float *part = static_cast<float *>(scr.ptr);
-    hipLaunchKernelGGL(conv_dw_mfma<true>, grid, dim3(256), 0, s, static_cast<const bf16 *>(dy),
-                       static_cast<const bf16 *>(x), static_cast<bf16 *>(dw), part, q, d.tiles_m, d.tiles_n,
-                       d.stages_per_split, P);
     const int64_t mn = static_cast<int64_t>(q.Cout) * q.KH * q.KW * q.Cin;
     int sub = 1;
     while (sub < 8 && cdiv(d.splits, sub) > 8) sub *= 2;
@@ -1426,10 +1468,6 @@ static bool conv_dw_mfma_launch(const void *dy, const void *x, void *dw, const C
     else
       hipLaunchKernelGGL(conv_dw_reduce, dim3(static_cast<unsigned>(cdiv(mn / 4, 256 / sub))), dim3(256), 0, s, part,
                          static_cast<bf16 *>(dw), d.splits, mn, sub);
-  } else {
-    hipLaunchKernelGGL(conv_dw_mfma<false>, grid, dim3(256), 0, s, static_cast<const bf16 *>(dy),
-                       static_cast<const bf16 *>(x), static_cast<bf16 *>(dw), nullptr, q, d.tiles_m, d.tiles_n,
-                       d.stages_per_split, P);
   }
   return true;
 }
