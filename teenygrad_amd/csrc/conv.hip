@@ -512,10 +512,14 @@ static ConvPath conv_path(const ConvGeo &q) {
 }
 
 // Scratch the int8 conv needs to run on the band-tiled kernel: a bf16 copy of
-// its weights (0: no band-tiled shape).
-static size_t tile_w8_scratch_bytes(const GemmParams &p) {
+// its weights (0: no band-tiled shape); the slices of a small batch follow it.
+static size_t tile_w8_copy_bytes(const GemmParams &p) {
   const int64_t n = static_cast<int64_t>(p.N) * p.K;
   return tile_conv_shape(p) != 0 && n % 16 == 0 ? static_cast<size_t>(n) * 2 : 0;
+}
+static size_t tile_w8_scratch_bytes(const GemmParams &p) {
+  const size_t copy = tile_w8_copy_bytes(p), slices = copy > 0 ? tile_conv_scratch_bytes(p) : 0;
+  return slices > 0 ? round256(copy) + slices : copy;
 }
 
 // Scratch bytes that let a conv take its fastest plan.
@@ -527,8 +531,9 @@ static size_t conv_scratch_bytes(const ConvGeo &q) {
     case kConvPlain: return gemm_scratch_bytes<INT8B, kAPlain>(p);
     case kConvVec:
       if (INT8B && tile_w8_scratch_bytes(p) > 0) return tile_w8_scratch_bytes(p);
-      // the row-band and band-tiled kernels need none
-      if (!INT8B && (band_fits<64, 3, 3, 56, 4>(p) || tile_conv_shape(p) != 0)) return 0;
+      // the row-band kernel needs none, the band-tiled kernel only for its slices
+      if (!INT8B && band_fits<64, 3, 3, 56, 4>(p)) return 0;
+      if (!INT8B && tile_conv_shape(p) != 0) return tile_conv_scratch_bytes(p);
       return gemm_scratch_bytes<INT8B, kAConvVec>(p);
     case kConvScalarGemm: return gemm_scratch_bytes<INT8B, kAConvScalar>(p);
     case kConvS2D: {
@@ -633,14 +638,16 @@ __global__ __launch_bounds__(256) void w8_to_bf16(const int8_t *__restrict__ q, 
 // 48.0 -> 41.2 us against the int8 implicit GEMM.  False (nothing launched)
 // without enough scratch.
 static bool try_conv_tile_w8(GemmParams p, int act, hipStream_t s, const Scratch scr) {
-  const size_t need = tile_w8_scratch_bytes(p);
+  const size_t need = tile_w8_copy_bytes(p);
   if (need == 0 || scr.ptr == nullptr || scr.bytes < need || !aligned(scr.ptr, 16)) return false;
   bf16 *wb = static_cast<bf16 *>(scr.ptr);
   const int64_t n16 = static_cast<int64_t>(need) / 32;
   hipLaunchKernelGGL(w8_to_bf16, dim3(static_cast<unsigned>(cdiv(n16, 256))), dim3(256), 0, s,
                      static_cast<const int8_t *>(p.B), wb, n16);
   p.B = wb;
-  return try_conv_tile<false>(p, act, s);
+  const size_t off = round256(need);
+  const Scratch rest = scr.bytes > off ? Scratch{static_cast<char *>(scr.ptr) + off, scr.bytes - off} : Scratch{};
+  return try_conv_tile<false>(p, act, s, rest);
 }
 
 // bf16 NHWC, groups == 1 -> MFMA implicit GEMM.  Returns false if not taken.
@@ -665,7 +672,7 @@ static bool try_conv_mfma(const void *x, const void *w, const float *scale, cons
   if constexpr (INT8B) {
     if (path == kConvVec && try_conv_tile_w8(p, act, s, scr)) return true;
   } else {
-    if (path == kConvVec && try_conv_tile<false>(p, act, s)) return true;
+    if (path == kConvVec && try_conv_tile<false>(p, act, s, scr)) return true;
   }
   switch (path) {
     case kConvPlain: return launch_gemm_mfma<INT8B, kAPlain>(p, act, s, scr);

@@ -59,6 +59,10 @@ struct TileConvParams {
   int x_bytes, w_bytes;  // byte extents (below 2^31)
   // stride-2 3x3 dx mode: element offset of each sub-pixel phase's weights
   int phase_off[4];
+  // PART: fp32 partial sums [slice][B OH OW][C_OUT] of `ch_slice` 32-channel
+  // chunks of C_IN each
+  float *part;
+  int ch_slice;
 };
 
 // IPB > 1: a band is IPB whole images of RB = OH rows (the 7x7 layers),
@@ -109,7 +113,7 @@ struct TileShape {
 };
 
 template <int KH, int KW, int OWT, int RB, int BN, bool INT8B, bool DX2 = false, int IPB = 1, bool S2 = false,
-          int KS = 1>
+          int KS = 1, bool PART = false>
 __global__ __launch_bounds__((TileShape<KH, KW, OWT, RB, BN, INT8B, DX2, IPB, S2, KS>::NT), 1) void conv_tile_kernel(
     TileConvParams p) {
   using S = TileShape<KH, KW, OWT, RB, BN, INT8B, DX2, IPB, S2, KS>;
@@ -129,11 +133,15 @@ __global__ __launch_bounds__((TileShape<KH, KW, OWT, RB, BN, INT8B, DX2, IPB, S2
   const int n_bands = IPB > 1 ? (p.B + IPB - 1) / IPB : p.B * bands_per_img;
   const int per_phase = n_bands * n_tiles;
   const int n_units = (DX2 ? 2 : 1) * per_phase;
-  const int nch = p.Cin / 32;
   const int G = static_cast<int>(gridDim.x);
   // consecutive units on one XCD: the channel tiles of a band (and
   // neighbouring bands) read the same input rows from that XCD's L2
-  const int wg = xcd_remap(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+  const int id = xcd_remap(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+  // PART: one unit's slice of C_IN per workgroup
+  const int wg = PART ? id % n_units : id;
+  const int slice = PART ? id / n_units : 0;
+  const int ch0 = slice * p.ch_slice;
+  const int nch = PART ? min(p.Cin / 32 - ch0, p.ch_slice) : p.Cin / 32;
   const int my_units = wg < n_units ? (n_units - 1 - wg) / G + 1 : 0;
   const int n_stages = my_units * nch;
   // unit u: co tile fastest (the tiles of one band share its input in L2);
@@ -213,7 +221,7 @@ __global__ __launch_bounds__((TileShape<KH, KW, OWT, RB, BN, INT8B, DX2, IPB, S2
   };
   auto dma_stage = [&](int st) __attribute__((always_inline)) {
     if (st % nch == 0) dma_unit(st);
-    const int c0 = (st % nch) * 32;
+    const int c0 = (ch0 + st % nch) * 32;
     const uint32_t buf = smem0 + (st % S::NSTG) * S::STAGE;
 #pragma unroll
     for (int r = 0; r < DI; ++r) {
@@ -464,7 +472,22 @@ __global__ __launch_bounds__((TileShape<KH, KW, OWT, RB, BN, INT8B, DX2, IPB, S2
             }
         }
       }
-      if (hk == 0) {
+      if constexpr (PART) {
+        // lane (c, g): channels 32 i + 8 q + 4 g .. + 3 of pixel 32 pbk + c
+        int b, oh0, n0, ph;
+        unit_of(st, b, oh0, n0, ph);
+        const int64_t pix = (static_cast<int64_t>(b) * p.OH + oh0) * OWT + 32 * pbk + c;
+        const int64_t pixels = static_cast<int64_t>(p.B) * p.OH * OWT;
+        if (hk == 0 && 32 * pbk + c < S::NPX && pix < pixels) {
+          float *dst = p.part + (slice * pixels + pix) * p.Cout + n0 + 4 * g;
+#pragma unroll
+          for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              *reinterpret_cast<f32x4 *>(dst + 32 * i + 8 * q) =
+                  f32x4{acc[i][4 * q], acc[i][4 * q + 1], acc[i][4 * q + 2], acc[i][4 * q + 3]};
+        }
+      } else if (hk == 0) {
 #pragma unroll
         for (int set = 0; set < NSET; ++set) {
           if (!DX2 && ea.sig) epilogue(st, std::true_type{}, set);
@@ -503,10 +526,48 @@ inline bool tile_conv_fits(const GemmParams &p) {
          static_cast<int64_t>(p.N) * p.K * (INT8B ? 1 : 2) < 0x7fffffff;
 }
 
-template <int KH, int KW, int OWT, int RB, int BN, bool INT8B, int IPB = 1, bool S2 = false, int KS = 1>
-inline void launch_tile_conv(const GemmParams &p, int act, hipStream_t s) {
+// Slices of C_IN for a small batch of 7x7 images, whose units leave most CUs
+// idle: two or four, as fit the CUs, of at least four 32-channel chunks, each
+// a workgroup that writes fp32 partial sums to the scratch.  512 -> 512 in us,
+// whole / sliced: batch 1 22.3 / 14.3, 4 22.4 / 15.0, 16 23.1 / 17.6, stride 2
+// batch 2 22.8 / 15.6.  The wider images' units have half the chunks or fewer,
+// and the second launch costs what slices of two save (14x14 256 -> 256, batch
+// 1 18.1 / 14.1 but 16 18.7 / 20.9).
+struct TileSlices {
+  int slices = 1, ch_slice = 0;
+  size_t bytes = 0;
+};
+
+inline TileSlices tile_conv_slices(const GemmParams &p) {
+  const int B = p.M / (p.OH * p.OW), nch = p.Cin / 32, units = (B + 1) / 2 * (p.N / 64);
+  TileSlices t;
+  int n = 1;
+  while (p.OW == 7 && n < 4 && 2 * n * units <= device_cu_count() && 2 * n <= nch / 4) n *= 2;
+  if (n == 1) return t;
+  t.ch_slice = (nch + n - 1) / n;
+  t.slices = (nch + t.ch_slice - 1) / t.ch_slice;
+  t.bytes = static_cast<size_t>(t.slices) * p.M * p.N * sizeof(float);
+  return t;
+}
+
+template <int KH, int KW, int OWT, int RB, int BN, bool INT8B, int IPB = 1, bool S2 = false, int KS = 1,
+          bool PART = false>
+inline void launch_tile_conv(const GemmParams &p, int act, hipStream_t s, Scratch scr = {}) {
+  if constexpr (!PART && IPB == 2) {  // the 7x7 shapes
+    const TileSlices sl = tile_conv_slices(p);
+    if (sl.slices > 1 && scr.ptr != nullptr && scr.bytes >= sl.bytes) {
+      GemmParams q = p;
+      q.act = act;
+      q.ws = static_cast<float *>(scr.ptr);
+      launch_tile_conv<KH, KW, OWT, RB, BN, INT8B, IPB, S2, KS, true>(q, act, s, scr);
+      const int64_t groups = static_cast<int64_t>(p.M) * ((p.N + 7) / 8);
+      hipLaunchKernelGGL(gemm_splitk_finalize, dim3(static_cast<unsigned>((groups + 255) / 256)), dim3(256), 0, s, q,
+                         sl.slices);
+      return;
+    }
+  }
   using S = TileShape<KH, KW, OWT, RB, BN, INT8B, false, IPB, S2, KS>;
-  auto kern = &conv_tile_kernel<KH, KW, OWT, RB, BN, INT8B, false, IPB, S2, KS>;
+  auto kern = &conv_tile_kernel<KH, KW, OWT, RB, BN, INT8B, false, IPB, S2, KS, PART>;
   static const bool attr_set = [kern] {
     return hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                S::LDS) == hipSuccess;
@@ -532,7 +593,13 @@ inline void launch_tile_conv(const GemmParams &p, int act, hipStream_t s) {
   t.w_bytes = static_cast<int>(static_cast<int64_t>(p.N) * p.K * (INT8B ? 1 : 2));
   const int bands = IPB > 1 ? (t.B + IPB - 1) / IPB : t.B * (p.OH / RB);
   const int units = bands * (p.N / BN);
-  const int grid = std::min(units, device_cu_count());
+  int grid = std::min(units, device_cu_count());
+  if constexpr (PART) {
+    const TileSlices sl = tile_conv_slices(p);
+    t.part = p.ws;
+    t.ch_slice = sl.ch_slice;
+    grid = units * sl.slices;
+  }
   hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(grid)), dim3(S::NT), S::LDS, s, t);
 }
 
@@ -560,8 +627,14 @@ inline int tile_conv_shape(const GemmParams &p) {
   return 0;
 }
 
+// Scratch bytes of its slices of C_IN (0: unsliced, or none of the shapes).
+inline size_t tile_conv_scratch_bytes(const GemmParams &p) {
+  const int shape = tile_conv_shape(p);
+  return shape == 3 || shape == 4 ? tile_conv_slices(p).bytes : 0;
+}
+
 template <bool INT8B>
-inline bool try_conv_tile(const GemmParams &p, int act, hipStream_t s) {
+inline bool try_conv_tile(const GemmParams &p, int act, hipStream_t s, Scratch scr) {
   if constexpr (!INT8B) {
     switch (tile_conv_shape(p)) {
       case 1: launch_tile_conv<3, 3, 14, 14, 64, false>(p, act, s); return true;
@@ -570,8 +643,8 @@ inline bool try_conv_tile(const GemmParams &p, int act, hipStream_t s) {
       // (with two waves per pixel block, each on half of every chunk's
       // channels: 512 -> 512 at batch 64 30.2 -> 26.1 us, stride 2 34.5 ->
       // 30.0 us, against one wave per block and SIMD)
-      case 3: launch_tile_conv<3, 3, 7, 7, 64, false, 2, false, 2>(p, act, s); return true;
-      case 4: launch_tile_conv<3, 3, 7, 7, 64, false, 2, true, 2>(p, act, s); return true;
+      case 3: launch_tile_conv<3, 3, 7, 7, 64, false, 2, false, 2>(p, act, s, scr); return true;
+      case 4: launch_tile_conv<3, 3, 7, 7, 64, false, 2, true, 2>(p, act, s, scr); return true;
       case 5: launch_tile_conv<3, 3, 14, 7, 64, false, 1, true, 2>(p, act, s); return true;
       default: break;
     }

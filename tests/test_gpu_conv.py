@@ -543,3 +543,44 @@ def test_bf16_nhwc_grouped(dev, orc, case):
     if act is not None:
         ref = {"relu": orc.relu, "silu": orc.silu, "gelu": orc.gelu}[act](ref)
     check_bf16(got, ref, str(case))
+
+
+SLICED = [  # B, H, C_IN, C_OUT, stride: 7x7 outputs whose units leave CUs idle; two or four slices, even and ragged
+    (1, 7, 512, 64, 1), (3, 7, 544, 128, 1), (4, 7, 288, 64, 1), (5, 14, 512, 64, 2), (2, 14, 672, 128, 2)]
+
+
+@pytest.mark.parametrize("B,H,Cin,Cout,s", SLICED)
+@pytest.mark.parametrize("weights", ["bf16", "int8"])
+def test_small_batch_slices(dev, B, H, Cin, Cout, s, weights):
+    rng = np.random.default_rng(B + H + Cin + Cout)
+    x = rb(rng.standard_normal((B, H, H, Cin), dtype=np.float32)).reshape(B, H, H, Cin)
+    shape = (Cout, 3, 3, Cin)
+    bias = rb(rng.normal(0, 0.1, Cout).astype(np.float32))
+    xb = dev.upload(to_bf16(x), tg.bf16)
+    if weights == "int8":
+        q = rng.integers(-128, 128, shape).astype(np.int8)
+        scale = rng.uniform(1e-4, 5e-4, Cout).astype(np.float32)
+        w = q * scale[:, None, None, None].astype(np.float64)
+        args, fn = (dev.upload(q), dev.upload(scale), dev.upload(bias)), K.w8a16_conv2d
+    else:
+        w = rb(rng.standard_normal(shape, dtype=np.float32) * np.float32(0.02)).reshape(shape).astype(np.float64)
+        args = (dev.upload(to_bf16(w.astype(np.float32)), tg.bf16), dev.upload(to_bf16(bias), tg.bf16))
+        fn = lambda *a, **k: K.conv2d(*a, layout="nhwc", **k)  # noqa: E731
+    oh = (H - 1) // s + 1
+    xp = np.zeros((B, H + 2, H + 2, Cin))
+    xp[:, 1:-1, 1:-1] = x
+    taps = [(xp[:, a:a + s * (oh - 1) + 1:s, c:c + s * (oh - 1) + 1:s], w[:, a, c]) for a in range(3) for c in range(3)]
+    ref = sum(t @ k.T for t, k in taps) + bias
+    # 9 C_IN fp32 sums, each within 2^-24 of at most sum |x| |w|, and the bf16 result
+    bound = (9 * Cin + 8) * 2.0 ** -24 * (sum(np.abs(t) @ np.abs(k).T for t, k in taps) + np.abs(bias)) \
+        + 2.0 ** -8 * np.abs(ref)
+    need = K.conv2d_workspace_size((B, H, H, Cin), shape, s, 1, 1, tg.i8 if weights == "int8" else tg.bf16)
+    copy = Cout * 9 * Cin * 2 if weights == "int8" else 0
+    if dev.info()["compute_units"] == 256:
+        assert need > copy, need
+    for ws in (need, copy):  # with and without room for the slices
+        print(f"[conv slices] B={B} H={H} {Cin}->{Cout} s={s} {weights} workspace={ws}", flush=True)
+        with stream_workspace(dev, ws):
+            got = fn(xb, *args, stride=s, padding=1, act="relu").to_host()
+        err = np.abs(from_bf16(got).astype(np.float64).reshape(ref.shape) - np.maximum(ref, 0))
+        assert np.all(err <= bound), f"{np.max(err - bound)} beyond the bound"
