@@ -478,8 +478,8 @@ static void launch_rows(const void *q, const void *k, const void *v, void *o, fl
 template <typename T, int D>
 static void launch_f32(const void *q, const void *k, const void *v, void *o, float *l, int nq, int nk, float scale,
                        int BH, int causal, int kv_group, hipStream_t s) {
-  const bool split = fa_f32_split(cdiv(nq, 32) * BH, cdiv(nk, 32));
-  fa_f32_launch(fa_fwd_f32<T, D, 1>, fa_fwd_f32<T, D, 4>, nq, BH, split, s, static_cast<const T *>(q),
+  const int split = fa_f32_split(cdiv(nq, 32) * BH, cdiv(nk, 32), D);
+  fa_f32_launch(TEENY_FA_F32(fa_fwd_f32, T, D, split), nq, BH, split, s, static_cast<const T *>(q),
                 static_cast<const T *>(k), static_cast<const T *>(v), static_cast<T *>(o), l,
                 static_cast<uint32_t>(nq), static_cast<uint32_t>(nk), scale, causal, kv_group);
 }

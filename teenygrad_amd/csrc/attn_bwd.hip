@@ -528,6 +528,16 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void fa_bwd_dq_bf16(
   }
   const int q0 = qb * BM + 32 * w, qi = q0 + c;
   const int64_t qrow = static_cast<int64_t>(bh) * nq + qi;
+  const int kv_end = CAUSAL ? min(nk, qb * BM + BM) : nk;
+  const int n_kt = (kv_end + BN - 1) / BN;
+  const int wave_end = CAUSAL ? min(kv_end, q0 + 32) : kv_end;
+  const bf16 *Kb = K + static_cast<int64_t>(bh / kv_group) * nk * D;
+  const bf16 *Vb = V + static_cast<int64_t>(bh / kv_group) * nk * D;
+  const __amdgpu_buffer_rsrc_t krs = buffer_rsrc(Kb, nk * D * 2), vrs = buffer_rsrc(Vb, nk * D * 2);
+  if (n_kt > 0) {  // in flight next to the rows of Q, dO and O
+    dma_tile<D, BN, NT>(krs, kbuf[0], 0, tid);
+    dma_tile<D, BN, NT>(vrs, vbuf[0], 0, tid);
+  }
   bf16x8 qT[NS], doT[NS];
   float dpart = 0.0f;
 #pragma unroll
@@ -551,15 +561,7 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void fa_bwd_dq_bf16(
   f32x16 dq[ND];
 #pragma unroll
   for (int d = 0; d < ND; ++d) dq[d] = zero16();
-  const int kv_end = CAUSAL ? min(nk, qb * BM + BM) : nk;
-  const int n_kt = (kv_end + BN - 1) / BN;
-  const int wave_end = CAUSAL ? min(kv_end, q0 + 32) : kv_end;
-  const bf16 *Kb = K + static_cast<int64_t>(bh / kv_group) * nk * D;
-  const bf16 *Vb = V + static_cast<int64_t>(bh / kv_group) * nk * D;
-  const __amdgpu_buffer_rsrc_t krs = buffer_rsrc(Kb, nk * D * 2), vrs = buffer_rsrc(Vb, nk * D * 2);
   if (n_kt > 0) {
-    dma_tile<D, BN, NT>(krs, kbuf[0], 0, tid);
-    dma_tile<D, BN, NT>(vrs, vbuf[0], 0, tid);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   }
@@ -643,8 +645,8 @@ static void rows_dkv(const BwdArgs &a, const float *delta) {
 
 template <typename T, int D>
 static void f32_dq(const BwdArgs &a, float *delta_out) {
-  const bool split = fa_f32_split(cdiv(a.nq, 32) * a.BH, cdiv(a.nk, 32));
-  fa_f32_launch(fa_bwd_dq_f32<T, D, 1>, fa_bwd_dq_f32<T, D, 4>, a.nq, a.BH, split, a.s, static_cast<const T *>(a.q),
+  const int split = fa_f32_split(cdiv(a.nq, 32) * a.BH, cdiv(a.nk, 32), D);
+  fa_f32_launch(TEENY_FA_F32(fa_bwd_dq_f32, T, D, split), a.nq, a.BH, split, a.s, static_cast<const T *>(a.q),
                 static_cast<const T *>(a.k), static_cast<const T *>(a.v), static_cast<const T *>(a.o),
                 static_cast<const T *>(a.dout), a.l, static_cast<T *>(a.dq), delta_out, static_cast<uint32_t>(a.nq),
                 static_cast<uint32_t>(a.nk), a.scale, a.causal, a.group);
@@ -653,9 +655,8 @@ static void f32_dq(const BwdArgs &a, float *delta_out) {
 template <typename T, int D>
 static void f32_dkv(const BwdArgs &a, const float *delta) {
   const int64_t heads = a.BH / a.group;
-  const bool split = fa_f32_split(cdiv(a.nk, 32) * heads, cdiv(a.nq, 32) * a.group);
-  fa_f32_launch(fa_bwd_dkv_f32<T, D, 1>, fa_bwd_dkv_f32<T, D, 4>, a.nk, heads, split, a.s,
-                static_cast<const T *>(a.q), static_cast<const T *>(a.k), static_cast<const T *>(a.v),
+  const int split = fa_f32_split(cdiv(a.nk, 32) * heads, cdiv(a.nq, 32) * a.group, D);
+  fa_f32_launch(TEENY_FA_F32(fa_bwd_dkv_f32, T, D, split), a.nk, heads, split, a.s, static_cast<const T *>(a.q), static_cast<const T *>(a.k), static_cast<const T *>(a.v),
                 static_cast<const T *>(a.o), static_cast<const T *>(a.dout), a.l, delta, static_cast<T *>(a.dk),
                 static_cast<T *>(a.dv), static_cast<uint32_t>(a.nq), static_cast<uint32_t>(a.nk), a.scale, a.causal,
                 a.group);

@@ -18,8 +18,9 @@
 // r % 4 of column c, which is also the k that the next product's step r
 // gives that lane.
 //
-// Small grids (fewer than 2048 blocks of 32 columns) give each block to a
-// workgroup of four waves that share out the tiles and merge in LDS;
+// Small grids give each block of 32 columns to a workgroup whose waves share
+// out the tiles and merge in LDS: eight waves (two per SIMD, head_dim up to
+// 64) while the blocks do not outnumber the CUs, four below 2048 blocks;
 // otherwise the four waves of a workgroup take a block each.  Results do not
 // depend on timing (no atomics).
 //
@@ -203,8 +204,11 @@ __device__ __forceinline__ void fa_write(T *out, uint32_t c0, uint32_t n, const 
   }
 }
 
+// Waves of a workgroup: those that share a column block, or four blocks' own.
+template <int SPLIT> constexpr int kFaWaves = SPLIT == 1 ? 4 : SPLIT;
+
 // blocks of 32 columns: this wave's (column block, head), its share of the
-// tiles, or false past the last block.  Grid (x, heads), four waves.
+// tiles, or false past the last block.  Grid (x, heads).
 template <int SPLIT>
 __device__ __forceinline__ bool fa_unit(int w, int blocks, int &blk, int64_t &head) {
   const int64_t total = static_cast<int64_t>(gridDim.x) * gridDim.y;
@@ -217,14 +221,16 @@ __device__ __forceinline__ bool fa_unit(int w, int blocks, int &blk, int64_t &he
 }
 
 template <typename T, int D, int SPLIT>
-__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_fwd_f32(const T *__restrict__ Q, const T *__restrict__ K,
+__global__ __launch_bounds__(64 * kFaWaves<SPLIT>, D <= 64 ? 2 : 1) void fa_fwd_f32(const T *__restrict__ Q, const T *__restrict__ K,
                                                                    const T *__restrict__ V, T *__restrict__ O,
                                                                    float *__restrict__ L, uint32_t nq, uint32_t nk,
                                                                    float scale, int causal, int kv_group, int nqb) {
   using Tile = FaTile<T, D>;
-  __shared__ __attribute__((aligned(16))) float lds[4][2 * Tile::FLOATS];
-  __shared__ float ml[2][4][32];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+  __shared__ __attribute__((aligned(16))) float lds[kFaWaves<SPLIT>][2 * Tile::FLOATS];
+  __shared__ float ml[2][kFaWaves<SPLIT>][32];
+  // wave-uniform, so that the tile loop and its masks are scalar branches
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
   int qb;
   int64_t bh;
   if (!fa_unit<SPLIT>(w, nqb, qb, bh)) return;
@@ -255,11 +261,14 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_fwd_f32(const T *__re
     const uint32_t last = causal ? min(kend - 1, qi) : kend - 1;  // last key that this lane's query sees
     float mx = m;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s[r] *= scale;
-      if ((diag || k0 + 32 > kend) && k0 + 8 * (r / 4) + 4 * h + r % 4 > last) s[r] = -INFINITY;
-      mx = fmaxf(mx, s[r]);
+    for (int r = 0; r < 16; ++r) s[r] *= scale;
+    if (diag || k0 + 32 > kend) {
+      asm volatile("" ::: "memory");  // a branch: whole tiles compare nothing
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = k0 + 8 * (r / 4) + 4 * h + r % 4 > last ? -INFINITY : s[r];
     }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
     mx = fmaxf(mx, other_half(mx));
     const float ref = mx == -INFINITY ? 0.0f : mx;
     if (__any(mx > m)) {
@@ -298,16 +307,16 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_fwd_f32(const T *__re
     __syncthreads();
     float mx = ml[0][0][c], sum = 0.0f;
 #pragma unroll
-    for (int i = 1; i < 4; ++i) mx = fmaxf(mx, ml[0][i][c]);
+    for (int i = 1; i < SPLIT; ++i) mx = fmaxf(mx, ml[0][i][c]);
     const float ref = mx == -INFINITY ? 0.0f : mx;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) sum += ml[1][i][c] * exp_near(ml[0][i][c] - ref);
+    for (int i = 0; i < SPLIT; ++i) sum += ml[1][i][c] * exp_near(ml[0][i][c] - ref);
     mul = exp_near(m - ref);
     acc.put(lds[w], mul / sum, c, h);
     m = mx;
     l = sum;
     __syncthreads();
-    fa_write<T, D, 4>(Ob, q0, nq, &lds[0][0], 2 * Tile::FLOATS, threadIdx.x, 256);
+    fa_write<T, D, SPLIT>(Ob, q0, nq, &lds[0][0], 2 * Tile::FLOATS, threadIdx.x, 64 * SPLIT);
   } else {
     wave_fence();
     acc.put(lds[w], 1.0f / l, c, h);
@@ -321,13 +330,15 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_fwd_f32(const T *__re
 
 // dq (and D_m = rowsum(o do) to delta_out, if given).
 template <typename T, int D, int SPLIT>
-__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_bwd_dq_f32(
+__global__ __launch_bounds__(64 * kFaWaves<SPLIT>, D <= 64 ? 2 : 1) void fa_bwd_dq_f32(
     const T *__restrict__ Q, const T *__restrict__ K, const T *__restrict__ V, const T *__restrict__ O,
     const T *__restrict__ dO, const float *__restrict__ L, T *__restrict__ dQ, float *__restrict__ delta_out,
     uint32_t nq, uint32_t nk, float scale, int causal, int kv_group, int nqb) {
   using Tile = FaTile<T, D>;
-  __shared__ __attribute__((aligned(16))) float lds[4][2 * Tile::FLOATS];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+  __shared__ __attribute__((aligned(16))) float lds[kFaWaves<SPLIT>][2 * Tile::FLOATS];
+  // wave-uniform, so that the tile loop and its masks are scalar branches
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
   int qb;
   int64_t bh;
   if (!fa_unit<SPLIT>(w, nqb, qb, bh)) return;
@@ -336,41 +347,48 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_bwd_dq_f32(
   const T *Kb = K + (bh / kv_group) * nk * D, *Vb = V + (bh / kv_group) * nk * D;
   float *kt = lds[w], *vt = lds[w] + Tile::FLOATS;
 
-  f32x4 q[D / 8], g[D / 8];
-  fa_cols<T, D>(q, O + bh * nq * D, q0, nq, c, h);
-  fa_cols<T, D>(g, dO + bh * nq * D, q0, nq, c, h);
-  float delta = 0.0f;
-#pragma unroll
-  for (int j = 0; j < D / 8; ++j)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) delta = __builtin_fmaf(q[j][i], g[j][i], delta);
-  delta += other_half(delta);
-  if (delta_out != nullptr && h == 0 && (SPLIT == 1 || w == 0) && qi < nq) delta_out[bh * nq + qi] = delta;
-  fa_cols<T, D>(q, Q + bh * nq * D, q0, nq, c, h);
-  const float lse = L[bh * nq + min(qi, nq - 1)];
-
-  FaAcc<D> dq;
-  dq.zero();
   const uint32_t kend = causal ? min(nk, min(q0 + 32, nq)) : nk;
   const int tiles = static_cast<int>((kend + 31) / 32);
   const uint32_t last = causal ? min(kend - 1, qi) : kend - 1;
   int t = SPLIT == 1 ? 0 : w;
-  // one set of staging registers: V's next tile is in flight during the first
-  // two products, K's during the last
+  // every first load before anything waits for one
+  f32x4 q[D / 8], g[D / 8];
   Tile ts;
+  float delta = 0.0f;
   bool odd = false;  // whether the K tile, one with masked pairs, holds an infinity or NaN
   auto diag = [&](int i) { return causal && 32u * i + 31 > q0; };
   auto store_k = [&](int i) {
     if (diag(i)) odd = ts.template store<true>(kt, 32u * i, nk, lane);
     else ts.store(kt, 32u * i, nk, lane);
   };
-  if (t < tiles) {
-    ts.fetch(Vb, 32u * t, nk, lane);
-    ts.store(vt, 32u * t, nk, lane);
-    ts.fetch(Kb, 32u * t, nk, lane);
-    store_k(t);
-    wave_fence();
+  const float lse = L[bh * nq + min(qi, nq - 1)];
+  {
+    f32x4 o[D / 8];
+    Tile tv;
+    if (t < tiles) {
+      tv.fetch(Vb, 32u * t, nk, lane);
+      ts.fetch(Kb, 32u * t, nk, lane);
+    }
+    fa_cols<T, D>(o, O + bh * nq * D, q0, nq, c, h);
+    fa_cols<T, D>(g, dO + bh * nq * D, q0, nq, c, h);
+    fa_cols<T, D>(q, Q + bh * nq * D, q0, nq, c, h);
+    if (t < tiles) {
+      tv.store(vt, 32u * t, nk, lane);
+      store_k(t);
+      wave_fence();
+    }
+#pragma unroll
+    for (int j = 0; j < D / 8; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) delta = __builtin_fmaf(o[j][i], g[j][i], delta);
   }
+  delta += other_half(delta);
+  if (delta_out != nullptr && h == 0 && (SPLIT == 1 || w == 0) && qi < nq) delta_out[bh * nq + qi] = delta;
+
+  FaAcc<D> dq;
+  dq.zero();
+  // one set of staging registers: V's next tile is in flight during the first
+  // two products, K's during the last
   for (; t < tiles; t += SPLIT) {
     const uint32_t k0 = 32u * t;
     const bool more = t + SPLIT < tiles;
@@ -382,11 +400,12 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_bwd_dq_f32(
       ts.store(vt, k0 + 32 * SPLIT, nk, lane);
       ts.fetch(Kb, k0 + 32 * SPLIT, nk, lane);
     }
-    const bool edge = diag(t) || k0 + 32 > kend;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float ds = exp_near(__builtin_fmaf(s[r], scale, -lse)) * (dp[r] - delta);
-      s[r] = edge && k0 + 8 * (r / 4) + 4 * h + r % 4 > last ? 0.0f : ds;
+    for (int r = 0; r < 16; ++r) s[r] = exp_near(__builtin_fmaf(s[r], scale, -lse)) * (dp[r] - delta);
+    if (diag(t) || k0 + 32 > kend) {
+      asm volatile("" ::: "memory");  // a branch: whole tiles compare nothing
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = k0 + 8 * (r / 4) + 4 * h + r % 4 > last ? 0.0f : s[r];
     }
     if (diag(t) && __any(odd))
       dq.masked_outer(kt, s, h, [&](int row) { return k0 + row <= last; });
@@ -403,7 +422,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_bwd_dq_f32(
   dq.put(lds[w], scale, c, h);
   if constexpr (SPLIT > 1) {
     __syncthreads();
-    fa_write<T, D, 4>(out, q0, nq, &lds[0][0], 2 * Tile::FLOATS, threadIdx.x, 256);
+    fa_write<T, D, SPLIT>(out, q0, nq, &lds[0][0], 2 * Tile::FLOATS, threadIdx.x, 64 * SPLIT);
   } else {
     wave_fence();
     fa_write<T, D, 1>(out, q0, nq, lds[w], 0, lane, 64);
@@ -413,14 +432,16 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_bwd_dq_f32(
 // dk and dv: columns are keys, tiles the queries of every head that shares
 // them.  delta: D_m of every query row, or null (computed here per tile).
 template <typename T, int D, int SPLIT>
-__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_bwd_dkv_f32(
+__global__ __launch_bounds__(64 * kFaWaves<SPLIT>, D <= 64 ? 2 : 1) void fa_bwd_dkv_f32(
     const T *__restrict__ Q, const T *__restrict__ K, const T *__restrict__ V, const T *__restrict__ O,
     const T *__restrict__ dO, const float *__restrict__ L, const float *__restrict__ delta, T *__restrict__ dK,
     T *__restrict__ dV, uint32_t nq, uint32_t nk, float scale, int causal, int kv_group, int nkb) {
   using Tile = FaTile<T, D>;
-  __shared__ __attribute__((aligned(16))) float lds[4][2 * Tile::FLOATS];
-  __shared__ __attribute__((aligned(16))) float rows[4][2][32];  // lse, D_m of the tile's queries
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+  __shared__ __attribute__((aligned(16))) float lds[kFaWaves<SPLIT>][2 * Tile::FLOATS];
+  __shared__ __attribute__((aligned(16))) float rows[kFaWaves<SPLIT>][2][32];  // lse, D_m of the tile's queries
+  // wave-uniform, so that the tile loop and its masks are scalar branches
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
   int kb;
   int64_t hkv;
   if (!fa_unit<SPLIT>(w, nkb, kb, hkv)) return;
@@ -471,10 +492,12 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_bwd_dkv_f32(
     if (diag(q0)) odd_q = ts.template store<true>(qt, q0, nq, lane);
     else ts.store(qt, q0, nq, lane);
   };
-  if (t < tiles) {
+  if (t < tiles) {  // both first tiles in flight together
     fetch_g(t);
+    Tile tq;
+    tq.fetch(Q + head(t) * nq * D, query(t), nq, lane);
     store_g(query(t));
-    fetch_q(t);
+    ts = tq;
     store_q(query(t));
     wave_fence();
   }
@@ -492,11 +515,18 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_bwd_dkv_f32(
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int r = 4 * r4 + i;
-        const uint32_t qi = q0 + 8 * r4 + 4 * h + i;
+        p[r] = exp_near(__builtin_fmaf(p[r], scale, -lse[i]));
+        ds[r] = p[r] * (ds[r] - dm[i]);
+      }
+    }
+    if (masks || q0 + 32 > nq) {
+      asm volatile("" ::: "memory");  // a branch: whole tiles compare nothing
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const uint32_t qi = q0 + 8 * (r / 4) + 4 * h + r % 4;
         const bool out = (masks && qi < key) || qi >= nq;
-        const float pv = exp_near(__builtin_fmaf(p[r], scale, -lse[i]));
-        p[r] = out ? 0.0f : pv;
-        ds[r] = out ? 0.0f : pv * (ds[r] - dm[i]);
+        p[r] = out ? 0.0f : p[r];
+        ds[r] = out ? 0.0f : ds[r];
       }
     }
     auto seen = [&](int row) { return q0 + row >= key && q0 + row < nq; };
@@ -521,8 +551,8 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_bwd_dkv_f32(
   T *dk_out = dK + hkv * nk * D, *dv_out = dV + hkv * nk * D;
   if constexpr (SPLIT > 1) {
     __syncthreads();
-    fa_write<T, D, 4>(dk_out, c0, nk, &lds[0][0], 2 * Tile::FLOATS, threadIdx.x, 256);
-    fa_write<T, D, 4>(dv_out, c0, nk, &lds[0][Tile::FLOATS], 2 * Tile::FLOATS, threadIdx.x, 256);
+    fa_write<T, D, SPLIT>(dk_out, c0, nk, &lds[0][0], 2 * Tile::FLOATS, threadIdx.x, 64 * SPLIT);
+    fa_write<T, D, SPLIT>(dv_out, c0, nk, &lds[0][Tile::FLOATS], 2 * Tile::FLOATS, threadIdx.x, 64 * SPLIT);
   } else {
     wave_fence();
     fa_write<T, D, 1>(dk_out, c0, nk, lds[w], 0, lane, 64);
@@ -530,19 +560,28 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fa_bwd_dkv_f32(
   }
 }
 
-// Launch shapes: blocks of 32 columns over `heads`, one workgroup per block
-// (SPLIT 4) or per four blocks.
-template <typename K1, typename K4, typename... A>
-inline void fa_f32_launch(K1 one, K4 four, int64_t cols, int64_t heads, bool split, hipStream_t s, A... args) {
-  const unsigned blocks = static_cast<unsigned>(cdiv(cols, 32));
-  const dim3 grid(split ? blocks : (blocks + 3) / 4, static_cast<unsigned>(heads));
-  if (split) hipLaunchKernelGGL(four, grid, dim3(256), 0, s, args..., static_cast<int>(blocks));
-  else hipLaunchKernelGGL(one, grid, dim3(256), 0, s, args..., static_cast<int>(blocks));
+// Waves that share a column block.  Eight for a grid of at most one block per
+// CU, which four would leave at one wave per SIMD, if there are tiles for
+// them (four / eight waves in us: 16 heads of 500 queries x 2000 keys x 64,
+// forward 58.3 / 50.1, dq 70.0 / 64.5; all three kernels of 4 heads of 1000 x
+// 1000 x 64 123 / 113, 2 of 1024 x 1024 x 16 60 / 47, but 16 of 200 x 200 x 64
+// 41.3 / 42.5).
+inline int fa_f32_split(int64_t blocks, int64_t tiles, int D) {
+  const int64_t cus = device_cu_count();
+  if (blocks <= cus && tiles >= 12 && D <= 64) return 8;
+  return blocks < 8 * cus && tiles > 1 ? 4 : 1;
 }
 
-// Whether a grid of `blocks` column blocks shares each block's tiles out to
-// the four waves of a workgroup: below eight waves per CU, and if there are
-// tiles to share.
-inline bool fa_f32_split(int64_t blocks, int64_t tiles) { return blocks < 8 * device_cu_count() && tiles > 1; }
+// Blocks of 32 columns over `heads`: a workgroup per block, or per four (split 1).
+template <typename K, typename... A>
+inline void fa_f32_launch(K kernel, int64_t cols, int64_t heads, int split, hipStream_t s, A... args) {
+  const unsigned blocks = static_cast<unsigned>(cdiv(cols, 32));
+  const dim3 grid(split > 1 ? blocks : (blocks + 3) / 4, static_cast<unsigned>(heads));
+  hipLaunchKernelGGL(kernel, grid, dim3(64 * (split == 1 ? 4 : split)), 0, s, args..., static_cast<int>(blocks));
+}
+
+// The kernel template NAME<T, D, SPLIT> for a split (8: D <= 64 only).
+#define TEENY_FA_F32(NAME, T, D, split) \
+  ((split) == 8 ? NAME<T, D, (D <= 64 ? 8 : 4)> : (split) == 4 ? NAME<T, D, 4> : NAME<T, D, 1>)
 
 }  // namespace teeny

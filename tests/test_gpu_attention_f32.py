@@ -40,6 +40,8 @@ CASES = [  # bh, nq, nk, d, causal, group
     # causal with keys that no query sees, and queries past the last key
     (2, 40, 140, 64, True, 1), (2, 140, 40, 128, True, 1),
     (6, 70, 50, 64, True, 3), (8, 40, 100, 32, False, 4),
+    # eight waves sharing 12, 13 and 20 tiles
+    (1, 390, 384, 16, True, 1), (2, 400, 410, 64, False, 1), (2, 630, 640, 32, True, 2),
     # enough blocks for a wave each, and blocks that do not fill a workgroup
     (2100, 20, 30, 16, True, 1), (1100, 40, 40, 16, False, 1), (700, 90, 70, 32, True, 1), (1024, 50, 33, 64, True, 2)]
 
