@@ -267,25 +267,6 @@ __global__ __launch_bounds__(256) void fa_bwd_delta_bf16(const bf16 *__restrict_
   if (row < rows && t % CPR == 0) delta[row] = s;
 }
 
-// Block order of a causal grid: workgroup `id` of nb blocks per head (block
-// 0 the longest, nb - 1 the shortest) -> (head, block).  An XCD takes
-// consecutive ids and has 64 workgroups resident, two per CU, the id 32 later
-// being the second one of a CU.  Heads go in groups that fill those 64 slots:
-// the first half of a group's ids are its longer blocks, longest first, and
-// the second half the others, shortest first, so that a CU's two workgroups
-// add up to the same length everywhere.  (In head order both are the same
-// block of two heads, and the longest pair sets the time.)  With the masks
-// compared on edge tiles only (dq, and dk/dv at head_dim 64), dq + dk/dv in
-// us: 64 heads x 1024 x 64 87 -> 68, 256 x 2048 x 128 1306 -> 1177, 64 x 1024
-// x 128 139 -> 122.  More than 64 blocks per head: plain, longest first.
-__device__ __forceinline__ void causal_order(int id, int nb, int heads, int &head, int &blk) {
-  const int per = nb > 64 ? 1 : max(1, min(64 / nb, heads / 8));
-  const int g0 = id / (per * nb) * per, n = min(per, heads - g0), j = id - g0 * nb;
-  const int half = nb > 64 ? nb : (nb + 1) / 2, i = j / n;
-  head = g0 + j - i * n;
-  blk = i < half ? i : nb - 1 - (i - half);
-}
-
 // dK, dV for the 32 * WAVES keys of one workgroup (wave w: keys k0 + 0..31),
 // head_dim 64.  (At head_dim 128 the K^T / V^T operands and both
 // accumulators take 192 of a lane's registers: one workgroup per CU; that

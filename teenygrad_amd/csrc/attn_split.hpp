@@ -234,12 +234,15 @@ __global__ __launch_bounds__(256) void fa_split_combine(AttnSplitArgs p, int ran
 
 // Whether this path is the better one, and into how many ranges it cuts the
 // keys.  fa_fwd_bf16 is the faster kernel on a full chip; its workgroups are
-// four column blocks each (eight, causal: two query blocks to a workgroup), so
-// it wants four (eight) times the blocks to fill it.  Measured in us
-// (heads x queries x keys x head_dim; fa_fwd_bf16 / here): 256 blocks, 16 x
-// 512 x 512 x 64 causal 16.4 / 9.0, 4 x 2048 x 2048 x 128 causal 47.6 / 26.2,
-// 8 x 1024 x 1024 x 128 22.3 / 16.6; 512 blocks, 16 x 1024 x 1024 x 128 causal
-// 31.4 / 26.9 but not causal 23.4 / 27.8, 4 x 4096 x 4096 x 128 71.6 / 81.1;
+// four column blocks each, so it wants four times the blocks to fill it.
+// Measured in us (heads x queries x keys x head_dim; fa_fwd_bf16 / here): 256
+// blocks, 16 x 512 x 512 x 64 causal 11.9 / 7.7, 4 x 2048 x 2048 x 128 causal
+// 41.0 / 26.4, 8 x 1024 x 1024 x 128 22.3 / 16.6; 512 blocks, not causal 16 x
+// 1024 x 1024 x 128 23.4 / 27.8, 4 x 4096 x 4096 x 128 71.6 / 81.1.  Causal its
+// longest block sets the time until every CU has several to run: at 512 blocks
+// head_dim 64 still gains here, 16 x 1024 x 1024 18.4 / 15.5, 32 x 512 x 512
+// 12.0 / 10.2, 8 x 2048 x 2048 30.8 / 24.6, while 128 does not, 16 x 1024 x 1024
+// 25.2 / 27.4, 32 x 512 x 512 16.5 / 17.7, 8 x 2048 x 2048 41.1 / 44.5;
 // 1024 blocks, 64 x 512 x 512 x 128 16.6 / 32.0.  At up to 32 queries most of
 // fa_fwd_bf16's rows are padding and this path is taken at any size: 32 heads
 // sharing 8 K/V heads, one query, batch x keys 1 x 16384 262 / 31, 32 x 1000
@@ -257,7 +260,7 @@ inline AttnSplitPlan attn_split_plan(int64_t BH, int64_t group, int64_t nq, int6
                                      size_t scratch) {
   AttnSplitPlan pl;
   const int64_t cus = device_cu_count(), blocks = cdiv(group * nq, 32), units = BH / group * blocks;
-  if (units > (causal && nq > 128 ? 2 : 1) * cus && nq > 32) return pl;
+  if (units > (causal && nq > 128 && D == 64 ? 2 : 1) * cus && nq > 32) return pl;
   pl.use = true;
   pl.blocks = static_cast<int>(blocks);
   int64_t ranges = units > cus / 2 ? 1 : std::max<int64_t>(1, std::min(2 * cus / units, nk / 512));

@@ -62,6 +62,32 @@ __device__ __forceinline__ constexpr int mfma32_row(int v, int g) {
   return 8 * (v >> 2) + 4 * g + (v & 3);
 }
 
+// Block order of a causal grid: workgroup `id` of nb blocks per head (block
+// 0 the longest, nb - 1 the shortest) -> (head, block).  An XCD takes
+// consecutive ids and has 64 workgroups resident, two per CU, the id 32 later
+// being the second one of a CU.  Heads go in groups that fill those 64 slots.
+// The XCD's first group meets empty CUs: the first half of its ids are its
+// longer blocks, longest first, and the second half the others, shortest
+// first, so that a CU's two workgroups add up to the same length everywhere.
+// A later group fills the slots as they come free: longest first, as with
+// more than 64 blocks per head.  (In head order a CU's two workgroups are the
+// same block of two heads, and the longest pair sets the time.)  In us, heads
+// x rows x head_dim: the forward, whose workgroups ran the blocks i and
+// nb - 1 - i in turn before, 64 x 1024 x 64 25.6 -> 22.7, 256 x 256 x 64 15.5
+// -> 13.1, 128 x 400 x 128 26.2 -> 21.2, 10 x 2500 x 128 56.2 -> 48.6, 256 x
+// 2048 x 128 334 -> 329; dq + dk/dv, in head order before and with their masks
+// now compared on edge tiles only (dq, and dk/dv at head_dim 64), 64 x 1024 x
+// 64 87 -> 68, 64 x 1024 x 128 139 -> 122, 256 x 2048 x 128 1306 -> 1177.
+__device__ __forceinline__ void causal_order(int id, int nb, int heads, int &head, int &blk) {
+  const int per = nb > 64 ? 1 : max(1, min(64 / nb, heads / 8));
+  const int g0 = id / (per * nb) * per, n = min(per, heads - g0), j = id - g0 * nb, i = j / n;
+  const int chunk = (nb * heads + 7) / 8;  // ids per XCD
+  const bool first = nb <= 64 && g0 * nb % chunk < per * nb;
+  const int half = (nb + 1) / 2;
+  head = g0 + j - i * n;
+  blk = !first || i < half ? i : nb - 1 - (i - half);
+}
+
 __device__ __forceinline__ f32x16 zero16() {
   f32x16 z;
 #pragma unroll
