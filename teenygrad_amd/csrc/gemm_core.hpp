@@ -180,8 +180,11 @@ constexpr int gemm_min_waves() {
 }
 
 // BK: k-tile depth (32 or 64).  PF: global->register prefetch depth in k-tiles (1 or 2).
-template <int BM, int BN, int BK, int WAVES_M, int PF, bool INT8B, int AMODE, bool KVEC = true>
-__global__ __launch_bounds__(256, (gemm_min_waves<BM, BN>())) void gemm_mfma_kernel(GemmParams p0) {
+// KG: groups of four waves, each with its own LDS stages and an equal run of
+// the k-tiles; their sums meet in LDS before the epilogue (no split-K slices:
+// ws is not looked at).
+template <int BM, int BN, int BK, int WAVES_M, int PF, bool INT8B, int AMODE, bool KVEC = true, int KG = 1>
+__global__ __launch_bounds__(256 * KG, (gemm_min_waves<BM, BN>())) void gemm_mfma_kernel(GemmParams p0) {
   GemmParams p = p0;
   if (p0.groups > 1) {
     const int grp = static_cast<int>(blockIdx.y);
@@ -219,11 +222,15 @@ __global__ __launch_bounds__(256, (gemm_min_waves<BM, BN>())) void gemm_mfma_ker
   static_assert(PF == 1 || PF == 2, "prefetch depth");
   constexpr int CP = BN + 8;  // C tile pitch in LDS (elements), epilogue
   constexpr int SMEM = 2 * STAGE > BM * CP ? 2 * STAGE : BM * CP;
-  __shared__ __attribute__((aligned(16))) bf16 smem[SMEM];
+  constexpr int RED = 2 * BM * BN;  // a group's fp32 sums, as bf16 elements
+  static_assert(KG == 1 || BM * CP + (KG - 1) * RED <= KG * SMEM, "the sums fit behind the C tile");
+  __shared__ __attribute__((aligned(16))) bf16 smem0[KG * SMEM];
   // element offset of 16-byte chunk `chunk` within LDS row `row`
   auto chunk_at = [](int row, int chunk) { return (SWZ ? chunk ^ ((row >> 2) & 3) : chunk) * 8; };
 
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x & 255;
+  const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  bf16 *smem = smem0 + kg * SMEM;
   const int lane = tid & 63, w = tid >> 6, g = lane >> 5, c = lane & 31;
   const int wm = w / WAVES_N, wn = w % WAVES_N;
 
@@ -240,9 +247,13 @@ __global__ __launch_bounds__(256, (gemm_min_waves<BM, BN>())) void gemm_mfma_ker
   const int tn = n_fast ? tile % tiles_n : tile / tiles_m;
   const int m0 = tm * BM, n0 = tn * BN;
   const int n_k_all = (p.K + BK - 1) / BK;
-  const int kt_begin = p.ws != nullptr ? split * p.kt_split : 0;
-  const int kt_end = p.ws != nullptr ? min(n_k_all, kt_begin + p.kt_split) : n_k_all;
-  const int k_first = kt_begin * BK;
+  const bool slices = KG == 1 && p.ws != nullptr;
+  const int kt_begin = slices ? split * p.kt_split : 0;
+  const int kt_end = slices ? min(n_k_all, kt_begin + p.kt_split) : n_k_all;
+  // the groups run as many k-tiles each (their barriers are the same ones);
+  // those past K load zeros
+  const int n_k = (kt_end - kt_begin + KG - 1) / KG;
+  const int k_first = (kt_begin + kg * n_k) * BK;
 
   // ── per-thread A row state ────────────────────────────────────────────
   // The vector paths load through buffer resources, unconditionally: a
@@ -490,7 +501,6 @@ __global__ __launch_bounds__(256, (gemm_min_waves<BM, BN>())) void gemm_mfma_ker
 
   // k-tiles of this workgroup (all of K unless split-K): kt counts from 0
   // and k offsets are k_first + kt * BK
-  const int n_k = kt_end - kt_begin;
   if constexpr (PF == 1) {
     // one register set: tile kt+1 is fetched while tile kt is multiplied
     u32x4 ra[A_CH], rb[B_CH];
@@ -552,7 +562,28 @@ __global__ __launch_bounds__(256, (gemm_min_waves<BM, BN>())) void gemm_mfma_ker
   // row chunks: fully coalesced, unlike the accumulator layout (4 consecutive
   // n per lane, rows spread over lanes).  Loops are fully unrolled so every
   // accumulator index is static and the accumulators stay in registers.
-  if (p.ws != nullptr) {
+  if constexpr (KG > 1) {
+    f32x4 *red = reinterpret_cast<f32x4 *>(smem0 + BM * CP);
+    if (kg > 0) {
+#pragma clang loop unroll(full)
+      for (int t = 0; t < NB * MB * 4; ++t) {
+        const int i = t / (MB * 4), j = t / 4 % MB, v4 = t % 4;
+        red[((kg - 1) * NB * MB * 4 + t) * 256 + tid] = f32x4{acc[i][j][4 * v4], acc[i][j][4 * v4 + 1],
+                                                             acc[i][j][4 * v4 + 2], acc[i][j][4 * v4 + 3]};
+      }
+    }
+    __syncthreads();
+    if (kg == 0) {
+      for (int o = 0; o < KG - 1; ++o)
+#pragma clang loop unroll(full)
+        for (int t = 0; t < NB * MB * 4; ++t) {
+          const f32x4 r = red[(o * NB * MB * 4 + t) * 256 + tid];
+#pragma clang loop unroll(full)
+          for (int e = 0; e < 4; ++e) acc[t / (MB * 4)][t / 4 % MB][4 * (t % 4) + e] += r[e];
+        }
+    }
+  }
+  if (slices) {
     // split-K partial: raw fp32 accumulators, four consecutive n per lane
     // (16-byte stores; the four v4 stores of a lane cover 128 contiguous
     // bytes of the row between the two lane halves)
@@ -580,7 +611,8 @@ __global__ __launch_bounds__(256, (gemm_min_waves<BM, BN>())) void gemm_mfma_ker
     return;
   }
   static_assert(WN % 16 == 0 && WM % 16 == 0, "fragment rows keep the swizzle of lane c");
-  bf16 *cs = smem;
+  bf16 *cs = smem0;
+  if (kg == 0) {
   // scale / bias per group of four columns (shared by the MB row blocks)
 #pragma clang loop unroll(full)
   for (int i = 0; i < NB; ++i)
@@ -623,15 +655,16 @@ __global__ __launch_bounds__(256, (gemm_min_waves<BM, BN>())) void gemm_mfma_ker
       }
     }
   }
+  }
   __syncthreads();
-  constexpr int CPR_C = BN / 8;        // 16-byte chunks per C row
-  constexpr int RPP_C = 256 / CPR_C;   // rows per pass
+  constexpr int CPR_C = BN / 8;             // 16-byte chunks per C row
+  constexpr int RPP_C = 256 * KG / CPR_C;   // rows per pass
   const bool vec16 = c_rows_vec16(p);
 #pragma clang loop unroll(full)
   for (int r0 = 0; r0 < BM; r0 += RPP_C) {
-    const int ml = r0 + tid / CPR_C, nl = (tid % CPR_C) * 8;
+    const int ml = r0 + static_cast<int>(threadIdx.x) / CPR_C, nl = (tid % CPR_C) * 8;
     const int m = m0 + ml, n = n0 + nl;
-    if (m < p.M && n < p.N) {
+    if ((BM % RPP_C == 0 || ml < BM) && m < p.M && n < p.N) {
       const u32x4 v = *reinterpret_cast<const u32x4 *>(cs + ml * CP + (((nl >> 3) ^ ((ml >> 4) & 1)) << 3));
       bf16 *dst = p.C + c_row(p, m) + n;
       if (vec16 && n + 8 <= p.N) {
@@ -701,16 +734,16 @@ static __global__ __launch_bounds__(256) void gemm_splitk_finalize(GemmParams p,
 
 // KVEC: K % 8 == 0 and (for the plain A path) 16-byte aligned rows, so no
 // 16-byte chunk straddles K and the element-wise tail paths are compiled out.
-template <int BM, int BN, int BK, int WAVES_M, int PF, bool INT8B, int AMODE>
+template <int BM, int BN, int BK, int WAVES_M, int PF, bool INT8B, int AMODE, int KG = 1>
 inline void launch_tile(const GemmParams &p, hipStream_t s, int splits = 1) {
   const int grid = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN) * splits;
   const unsigned groups = p.groups > 1 ? static_cast<unsigned>(p.groups) : 1u;
   if (p.K % 8 == 0 && AMODE != kAConvScalar) {
-    hipLaunchKernelGGL((gemm_mfma_kernel<BM, BN, BK, WAVES_M, PF, INT8B, AMODE, true>), dim3(grid, groups),
-                       dim3(256), 0, s, p);
+    hipLaunchKernelGGL((gemm_mfma_kernel<BM, BN, BK, WAVES_M, PF, INT8B, AMODE, true, KG>), dim3(grid, groups),
+                       dim3(256 * KG), 0, s, p);
   } else {
-    hipLaunchKernelGGL((gemm_mfma_kernel<BM, BN, BK, WAVES_M, PF, INT8B, AMODE, false>), dim3(grid, groups),
-                       dim3(256), 0, s, p);
+    hipLaunchKernelGGL((gemm_mfma_kernel<BM, BN, BK, WAVES_M, PF, INT8B, AMODE, false, KG>), dim3(grid, groups),
+                       dim3(256 * KG), 0, s, p);
   }
 }
 
@@ -719,18 +752,19 @@ inline int64_t tiles_of(const GemmParams &p, int bm, int bn) {
 }
 
 // Split-K factor of the 64 x 64 x 64 tiles: four slices of a deep K (2048 or
-// more) when the tiles fill the CUs at most once and the k-tiles per slice
-// outweigh the slices' fp32 traffic and their reduction, which grow with the
-// tile count.  Measured in us, one slice / four: 100 x 512 x 2048 12.2 / 10.1,
-// 250 x 1024 x 4096 21.4 / 14.0, 256 x 2048 x 8192 39.1 / 23.5, int8 514 x
-// 1792 x 7168 41.1 / 35.9, but 784 x 512 x 2048 12.7 / 14.0, 1000 x 1024 x
-// 4096 22.8 / 24.8 (M x N x K).  Up to half as many tiles more than CUs leave
-// most CUs idle in the second round, which slices of a K from 4608 on fill:
-// 2304 x 512 x 4608 35.2 / 29.0, 1100 x 1024 x 8192 54.5 / 41.5; 1500 x 1024 x
-// 4096 29.5 / 30.7.  (So the slices take 25 MB at most.)
+// more) when the k-tiles outnumber the tiles, so that they outweigh the
+// slices' fp32 traffic and their reduction.  With more tiles (up to one per
+// CU) groups of waves share K inside the workgroup (launch_split).  Measured
+// in us, slices / groups: 100 x 512 x 2048 10.0 / 10.4, 250 x 1024 x 4096 13.8 /
+// 16.7, 256 x 2048 x 8192 22.8 / 28.2, but 512 x 1024 x 4096 18.4 / 17.0, 800 x
+// 1024 x 8192 33.6 / 29.4, 640 x 1024 x 4096 21.5 / 17.1, int8 514 x 1792 x 7168
+// 36.2 / 30.6 (M x N x K).  Up to half as many tiles more than CUs leave most
+// CUs idle in the second round, which slices of a K from 4608 on fill, against
+// one slice 2304 x 512 x 4608 35.2 / 29.0, 1100 x 1024 x 8192 54.5 / 41.5; 1500
+// x 1024 x 4096 29.5 / 30.7.  (So the slices take 25 MB at most.)
 inline int splitk_factor(const GemmParams &p) {
   const int64_t tiles = tiles_of(p, 64, 64), n_k = (p.K + 63) / 64, cus = device_cu_count();
-  if (tiles <= cus) return n_k >= 32 && 3 * n_k >= tiles ? 4 : 1;
+  if (tiles <= cus) return n_k >= 32 && n_k >= tiles ? 4 : 1;
   return 2 * tiles <= 3 * cus && n_k >= 72 ? 4 : 1;
 }
 
@@ -754,8 +788,14 @@ inline SplitPlan split_plan(const GemmParams &p) {
   return sp;
 }
 
-// Runs split along K when the plan splits and the caller's scratch holds the
-// partial sums; otherwise unsplit (same products, one accumulation chain).
+// 64 x 64 tiles.  Runs split along K when the plan splits and the caller's
+// scratch holds the partial sums; otherwise unsplit (same products).  With at
+// most one workgroup per CU its four waves wait for each k-tile's loads and
+// barrier most of the time (780 clocks per k-tile, 128 of them MFMAs), so K is
+// shared by two groups of waves from 16 k-tiles on, by four from 32.  In us, 1 /
+// 2 / 4 groups: 500 x 1024 x 1024 8.5 / 7.8 / 8.4, 3136 x 256 x 1024 8.6 / 8.3 /
+// 8.3, 640 x 1024 x 4096 21.5 / 18.2 / 17.5, 256 x 4096 x 4096 int8 25.2 / 19.6 /
+// 18.8; 6272 x 128 x 512 6.5 / 6.5 / 6.9.
 template <bool INT8B, int AMODE>
 inline void launch_split(GemmParams p, hipStream_t s, Scratch scr) {
   const SplitPlan sp = split_plan(p);
@@ -769,6 +809,13 @@ inline void launch_split(GemmParams p, hipStream_t s, Scratch scr) {
     return;
   }
   p.ws = nullptr;
+  if constexpr (AMODE != kAConvScalar) {
+    if (tiles_of(p, 64, 64) <= device_cu_count() && p.K > 15 * 64) {
+      if (p.K > 31 * 64) launch_tile<64, 64, 64, 2, 2, INT8B, AMODE, 4>(p, s);
+      else launch_tile<64, 64, 64, 2, 2, INT8B, AMODE, 2>(p, s);
+      return;
+    }
+  }
   launch_tile<64, 64, 64, 2, 2, INT8B, AMODE>(p, s);
 }
 
@@ -794,20 +841,32 @@ inline void launch_persist_default(const GemmParams &p, hipStream_t s);
 //  * the 256 x 256 LDS-DMA kernel (gemm_dma.hpp) when its tiles fill the chip;
 //  * narrow outputs (N <= 64): 64 x 64 x 64 tiles for deep K (more
 //    workgroups to hide latency), else 128 x 64 x 32;
-//  * grids of 128 x 128 tiles that leave CUs idle: 128 x 64 x 64 if those
+//  * grids of at most one workgroup per CU, the smallest tile of 64 x 64, 128
+//    x 64 and 128 x 128 that gives one: K shared by groups of four waves inside
+//    the workgroup (64 x 64: launch_split; the others from K = 1024 on), whose
+//    loads, barriers and MFMAs overlap as a second workgroup's would.  In us,
+//    one group / two, M x N x K: 128 x 64, 2000 x 1024 x 4096 30.9 / 28.4, 1500
+//    x 1024 x 4096 30.2 / 26.6, int8 400 x 4096 x 11008 91 / 67; 128 x 128, 4096
+//    x 1024 x 4096 51.2 / 44.0, 4000 x 1024 x 1024 17.6 / 16.4, int8 1000 x 4096
+//    x 4096 56.0 / 47.5, (against 128 x 64 / 128 x 128 of two groups) 2200 x
+//    1024 x 4096 45 / 39.3; 2000 x 1024 x 768 9.4 / 9.4, 3000 x 1024 x 512 10.2 /
+//    11.0;
+//  * other grids of 128 x 128 tiles that leave CUs idle: 128 x 64 x 64 if those
 //    fill the CUs, else 64 x 64 x 64, split along K where that pays.  A tile's
 //    time per k-tile is the CU's LDS traffic for it (its operands written,
 //    and read 1 to 2 KiB per MFMA), so on a CU with one workgroup the smaller
 //    tile is done sooner: in us, 128 x 64 / 64 x 64 tiles, M x N x K: 196 x
-//    1024 x 256 5.6 / 5.2, 3136 x 256 x 1024 10.5 / 8.5, 500 x 1024 x 1024
-//    10.6 / 8.3, 4000 x 256 x 768 9.1 / 7.4; but 2000 x 1024 x 4096 (256 tiles
-//    of 128 x 64) 30.6 / 33.6;
+//    1024 x 256 5.6 / 5.2, 4000 x 256 x 768 9.1 / 7.4; but 1000 x 4096 x 512
+//    10.8 / 11.8, 900 x 4096 x 768 13.7 / 15.0;
 //  * short K (<= 256, the 1x1 convs): 128 x 128 x 32 with a two-tile
 //    prefetch, so the few k-tiles still overlap loads with MFMAs;
 //  * otherwise 128 x 128 x 64 (two workgroups per CU; the int8 3x3 conv 32 x
 //    256 x 28 x 28 -> 256, 392 tiles: 48.7 us, against 54.4 us for 128 x 128 x
 //    32 with the two-tile prefetch and 70 us for 128 x 64 x 64).
-enum GemmTiles { kTilesPersist, kTilesStream, kTilesBig, kTiles128x64, kTiles64x64, kTiles128x128Short, kTiles128x64Deep, kTiles128x128 };
+enum GemmTiles {
+  kTilesPersist, kTilesStream, kTilesBig, kTiles128x64, kTiles64x64, kTiles128x128Short, kTiles128x64Deep,
+  kTiles128x64Groups, kTiles128x128Groups, kTiles128x128
+};
 
 template <bool INT8B, int AMODE>
 inline GemmTiles gemm_tiles(const GemmParams &p) {
@@ -819,6 +878,12 @@ inline GemmTiles gemm_tiles(const GemmParams &p) {
   }
   if (p.N <= 64) return p.K >= 512 ? kTiles64x64 : kTiles128x64;
   const int64_t cus = device_cu_count();
+  if constexpr (AMODE != kAConvScalar) {
+    if (p.K >= 1024 && tiles_of(p, 64, 64) > cus && splitk_factor(p) == 1) {
+      if (tiles_of(p, 128, 64) <= cus) return kTiles128x64Groups;
+      if (tiles_of(p, 128, 128) <= cus) return kTiles128x128Groups;
+    }
+  }
   if (tiles_of(p, 128, 128) < cus)
     return tiles_of(p, 128, 64) < cus || splitk_factor(p) > 1 ? kTiles64x64 : kTiles128x64Deep;
   return p.K <= 256 ? kTiles128x128Short : kTiles128x128;
@@ -919,6 +984,12 @@ inline bool launch_gemm_mfma(GemmParams p, int act, hipStream_t s, Scratch scr) 
     case kTiles128x64: launch_tile<128, 64, 32, 2, 2, INT8B, AMODE>(p, s); break;
     case kTiles64x64: launch_split<INT8B, AMODE>(p, s, scr); break;
     case kTiles128x128Short: launch_tile<128, 128, 32, 2, 2, INT8B, AMODE>(p, s); break;
+    case kTiles128x64Groups:
+      if constexpr (AMODE != kAConvScalar) launch_tile<128, 64, 64, 2, 2, INT8B, AMODE, 2>(p, s);
+      break;
+    case kTiles128x128Groups:
+      if constexpr (AMODE != kAConvScalar) launch_tile<128, 128, 64, 2, 2, INT8B, AMODE, 2>(p, s);
+      break;
     case kTiles128x64Deep: launch_tile<128, 64, 64, 2, 2, INT8B, AMODE>(p, s); break;
     default: launch_tile<128, 128, 64, 2, 1, INT8B, AMODE>(p, s); break;
   }

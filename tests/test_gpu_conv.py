@@ -584,3 +584,40 @@ def test_small_batch_slices(dev, B, H, Cin, Cout, s, weights):
             got = fn(xb, *args, stride=s, padding=1, act="relu").to_host()
         err = np.abs(from_bf16(got).astype(np.float64).reshape(ref.shape) - np.maximum(ref, 0))
         assert np.all(err <= bound), f"{np.max(err - bound)} beyond the bound"
+
+
+GROUPED_K = [  # B, H, C_IN, C_OUT, kernel, stride: K shared by groups of waves, 64- and 128-row tiles, ragged edges
+    (3, 20, 24, 72, 7, 1), (5, 13, 104, 200, 5, 2), (2, 15, 256, 130, 3, 2), (12, 28, 48, 120, 5, 1), (22, 28, 48, 120, 5, 1)]
+
+
+@pytest.mark.parametrize("B,H,Cin,Cout,k,s", GROUPED_K)
+@pytest.mark.parametrize("weights", ["bf16", "int8"])
+def test_grouped_k(dev, B, H, Cin, Cout, k, s, weights):
+    rng = np.random.default_rng(B + H + Cin + Cout)
+    x = rb(rng.standard_normal((B, H, H, Cin), dtype=np.float32)).reshape(B, H, H, Cin)
+    shape, pad, oh = (Cout, k, k, Cin), k // 2, (H - 1) // s + 1
+    bias = rb(rng.normal(0, 0.1, Cout).astype(np.float32))
+    xb = dev.upload(to_bf16(x), tg.bf16)
+    if weights == "int8":
+        q = rng.integers(-128, 128, shape).astype(np.int8)
+        scale = rng.uniform(1e-4, 5e-4, Cout).astype(np.float32)
+        w = q * scale[:, None, None, None].astype(np.float64)
+        args, fn = (dev.upload(q), dev.upload(scale), dev.upload(bias)), K.w8a16_conv2d
+    else:
+        w = rb(rng.standard_normal(shape, dtype=np.float32) * np.float32(0.02)).reshape(shape).astype(np.float64)
+        args = (dev.upload(to_bf16(w.astype(np.float32)), tg.bf16), dev.upload(to_bf16(bias), tg.bf16))
+        fn = lambda *a, **kw: K.conv2d(*a, layout="nhwc", **kw)  # noqa: E731
+    xp = np.zeros((B, H + 2 * pad, H + 2 * pad, Cin))
+    xp[:, pad:H + pad, pad:H + pad] = x
+    taps = [(xp[:, a:a + s * (oh - 1) + 1:s, c:c + s * (oh - 1) + 1:s], w[:, a, c]) for a in range(k) for c in range(k)]
+    ref = sum(t @ v.T for t, v in taps) + bias
+    # k k C_IN fp32 sums, each within 2^-24 of at most sum |x| |w|, and the bf16 result
+    bound = (k * k * Cin + 8) * 2.0 ** -24 * (sum(np.abs(t) @ np.abs(v).T for t, v in taps) + np.abs(bias)) \
+        + 2.0 ** -8 * np.abs(ref)
+    need = K.conv2d_workspace_size((B, H, H, Cin), shape, s, pad, 1, tg.i8 if weights == "int8" else tg.bf16)
+    for ws in {need, Cout * k * k * Cin * 2 if weights == "int8" else 0}:
+        print(f"[conv grouped k] B={B} H={H} {Cin}->{Cout} k={k} s={s} {weights} workspace={ws}", flush=True)
+        with stream_workspace(dev, ws):
+            got = fn(xb, *args, stride=s, padding=pad, act="relu").to_host()
+        err = np.abs(from_bf16(got).astype(np.float64).reshape(ref.shape) - np.maximum(ref, 0))
+        assert np.all(err <= bound), f"{np.max(err - bound)} beyond the bound"

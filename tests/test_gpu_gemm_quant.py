@@ -29,7 +29,9 @@ def test_linear_f32_fixture(dev, orc, with_bias):
 
 SMALL_GRID = [  # (M, N, K, K slices): 64 x 64 tiles with ragged edges, unsplit and in four slices of ragged K
     (65, 65, 64, 1), (130, 72, 272, 1), (1000, 520, 1040, 1), (100, 200, 2048, 4), (257, 130, 2064, 4),
-    (70, 1000, 4112, 4), (1023, 1024, 4096, 1), (1100, 1000, 4624, 4)]
+    (70, 1000, 4112, 4), (1023, 1024, 4096, 1), (1100, 1000, 4624, 4),
+    # K shared by two and four groups of waves (runs of k-tiles past K), on 64 x 64, 128 x 64 and 128 x 128 tiles
+    (300, 520, 976, 1), (500, 600, 2064, 1), (450, 500, 2032, 1), (1100, 1000, 1104, 1), (2100, 1000, 1040, 1)]
 
 
 @pytest.mark.parametrize("m,n,k,slices", SMALL_GRID)
