@@ -1215,15 +1215,22 @@ static void launch_dw_direct(const void *dy, const void *x, void *dw, const Conv
 // pixels x 128 columns of each are moved to LDS by LDS-DMA (padding taps,
 // rows past the last pixel and columns past the edge read as zeros through
 // the buffer extent) and both MFMA operands come out of LDS through
-// transposing reads.  Workgroup tile 128 x 128, four waves of 64 x 64.  The
-// pixel range is split over workgroups; with more than one split each
-// writes fp32 partials to the stream workspace and a second kernel adds them
-// in split order (deterministic).
+// transposing reads.  Workgroup tile 128 x 128, four waves of 64 x 64; with
+// at most one workgroup per CU two such groups, each with its own stages and
+// half of the pixels, whose sums meet in LDS.  The pixel range is split over
+// workgroups; with more than one split each writes fp32 partials to the
+// stream workspace and a second kernel adds them in split order
+// (deterministic).  Against two workgroups of one group per CU, which write
+// (and read back) twice the partials, in us: 2000 rows 1024 -> 4096 31.9 ->
+// 23.9 (no partials left, the bf16 tile stored in whole rows through LDS: 25.9
+// without that), 28x28 3x3 128 -> 128 at batch 32 26.0 -> 22.1, 28x28 1x1 256
+// -> 512 at batch 32 24.1 -> 19.8, 56x56 1x1 64 -> 256 at batch 8 14.2 -> 12.6.
 constexpr int kDwTile = 128, kDwStage = 64;
 
 struct DwPlan {
   bool ok = false;
   int tiles_m = 0, tiles_n = 0, splits = 1, stages_per_split = 0;
+  bool groups = false;
   size_t part_bytes = 0;  // workspace for splits > 1
 };
 
@@ -1238,15 +1245,18 @@ static DwPlan dw_plan(const ConvGeo &q, size_t workspace) {
   d.tiles_m = static_cast<int>(cdiv(M, kDwTile));
   d.tiles_n = static_cast<int>(cdiv(N, kDwTile));
   const int64_t tiles = static_cast<int64_t>(d.tiles_m) * d.tiles_n, stages = cdiv(P, kDwStage);
-  // as many as two workgroups per CU hold at once (one split more of the 144
-  // tiles of 7x7 512 -> 512 at batch 64 starts a second round: 57 us of dw
-  // against 34), and at least 7 stages each, next to which the fp32 partials
-  // are cheap (14x14 256 -> 256 at batch 16 with 4 / 7 stages 23.5 / 20.1 us)
-  int64_t splits = std::max<int64_t>(1, 2 * static_cast<int64_t>(device_cu_count()) / tiles);
+  // as many as the CUs hold at once (one split more starts a second round,
+  // 7x7 512 -> 512 at batch 64 57 us of dw against 34), and at least 7 stages
+  // each, next to which the fp32 partials are cheap (14x14 256 -> 256 at batch
+  // 16 with 4 / 7 stages 23.5 / 20.1 us).  Two groups from 4 stages on: 36 rows
+  // 512 -> 1536, one stage, 6.9 us with one, 7.2 with two.
+  const int64_t cus = device_cu_count();
+  int64_t splits = std::max<int64_t>(1, cus / tiles);
   splits = std::min<int64_t>(splits, std::max<int64_t>(1, stages / 7));
   while (splits > 1 && static_cast<size_t>(splits) * M * N * 4 > workspace) --splits;
   d.stages_per_split = static_cast<int>(cdiv(stages, splits));
   d.splits = static_cast<int>(cdiv(stages, d.stages_per_split));  // no empty split
+  d.groups = tiles <= cus && d.stages_per_split >= 4;
   d.part_bytes = d.splits > 1 ? static_cast<size_t>(d.splits) * M * N * 4 : 0;
   d.ok = tiles * d.splits <= 0x7fffffff;
   return d;
@@ -1256,23 +1266,31 @@ static DwPlan dw_plan(const ConvGeo &q, size_t workspace) {
 static size_t dw_scratch_bytes(const ConvGeo &q) { return dw_plan(q, static_cast<size_t>(1) << 26).part_bytes; }
 
 // ROWS: a 1x1 stride-1 conv without padding (and linear_backward's dw): the
-// rows of x are the pixels themselves.
-template <bool PART, bool ROWS>
-__global__ __launch_bounds__(256, 2) void conv_dw_mfma(const bf16 *__restrict__ dy, const bf16 *__restrict__ x,
+// rows of x are the pixels themselves.  KG: groups of four waves.
+template <bool PART, bool ROWS, int KG>
+__global__ __launch_bounds__(256 * KG, 2) void conv_dw_mfma(const bf16 *__restrict__ dy, const bf16 *__restrict__ x,
                                                        bf16 *__restrict__ dw, float *__restrict__ part, ConvGeo q,
                                                        int tiles_m, int tiles_n, int stages_per_split, int P) {
   constexpr int NT = 256, TILE = kDwStage * kDwTile;
-  __shared__ __attribute__((aligned(16))) bf16 abuf[2][TILE], bbuf[2][TILE];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 5, c = lane & 31;
+  __shared__ __attribute__((aligned(16))) bf16 lds[KG][2][2][TILE];
+  const int tid = threadIdx.x & 255, lane = tid & 63, w = tid >> 6, g = lane >> 5, c = lane & 31;
+  const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  bf16(*abuf)[TILE] = lds[kg][0], (*bbuf)[TILE] = lds[kg][1];
   const int ntiles = tiles_m * tiles_n;
-  // the tiles of one split (same pixels of dy and x) are consecutive ids: one XCD's L2
+  // the tiles of one split (same pixels of dy and x) are consecutive ids: one
+  // XCD's L2, which the side with fewer tiles keeps whole (runs along the
+  // longer side read all of it on every XCD: 2000 x 4096 -> 1024 27.3 us)
   const int id = xcd_remap(blockIdx.x, gridDim.x);
   const int split = id / ntiles, t = id % ntiles;
-  const int co0 = (t / tiles_n) * kDwTile, n0 = (t % tiles_n) * kDwTile;
+  const bool m_fast = tiles_m < tiles_n;
+  const int co0 = (m_fast ? t % tiles_m : t / tiles_n) * kDwTile, n0 = (m_fast ? t / tiles_m : t % tiles_n) * kDwTile;
   const int M = q.Cout, N = q.KH * q.KW * q.Cin;
   const int wm = w >> 1, wn = w & 1;
-  const int st0 = split * stages_per_split;
-  const int nst = min(stages_per_split, (P + kDwStage - 1) / kDwStage - st0);
+  // the split's stages in equal runs, one to a group (the last one's may be shorter)
+  const int split0 = split * stages_per_split;
+  const int nst_all = min(stages_per_split, (P + kDwStage - 1) / kDwStage - split0);
+  const int rounds = (nst_all + KG - 1) / KG;
+  const int st0 = split0 + kg * rounds, nst = min(rounds, nst_all - kg * rounds);
   const __amdgpu_buffer_rsrc_t dys = buffer_rsrc(dy, P * M * 2);
   const __amdgpu_buffer_rsrc_t xs = buffer_rsrc(x, q.B * q.H * q.W * q.Cin * 2);
   // LDS-DMA slot u = 256 i + tid: stage row 16 i + tid / 16, chunk position
@@ -1344,16 +1362,15 @@ __global__ __launch_bounds__(256, 2) void conv_dw_mfma(const bf16 *__restrict__ 
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = zero16();
-  if (nst > 0) {
-    issue(0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-  }
-  for (int s = 0; s < nst; ++s) {
+  if (nst > 0) issue(0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  for (int s = 0; s < rounds; ++s) {
     const int b = s & 1;
     if (s + 1 < nst) issue(b ^ 1);
 #pragma unroll
     for (int kk = 0; kk < kDwStage / 16; ++kk) {
+      if (KG > 1 && s >= nst) break;
       bf16x8 af[2], bfr[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) af[i] = frag_tr<128>(abuf[b], 16 * kk, 2 * wm + i, lane);
@@ -1367,23 +1384,57 @@ __global__ __launch_bounds__(256, 2) void conv_dw_mfma(const bf16 *__restrict__ 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   }
-  // lane (g, c) holds column n0 + 64 wn + 32 j + c, rows co0 + 64 wm + 32 i + mfma32_row(v, g)
+  if constexpr (KG == 2) {
+    // each group takes over the other's sums of one half of the rows
+    f32x4 *red = reinterpret_cast<f32x4 *>(lds);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int t = 0; t < 8; ++t)
+        if (i != kg)
+          red[(kg * 8 + t) * 256 + tid] = f32x4{acc[i][t >> 2][4 * (t & 3)], acc[i][t >> 2][4 * (t & 3) + 1],
+                                                acc[i][t >> 2][4 * (t & 3) + 2], acc[i][t >> 2][4 * (t & 3) + 3]};
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int t = 0; t < 8; ++t)
+        if (i == kg) {
+          const f32x4 o = red[((1 - kg) * 8 + t) * 256 + tid];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][t >> 2][4 * (t & 3) + e] += o[e];
+        }
+  }
+  // lane (g, c) holds column 64 wn + 32 j + c, rows 64 wm + 32 i + mfma32_row(v, g) of the tile
+  bf16 *cs = reinterpret_cast<bf16 *>(lds) + (KG - 1) * 4 * TILE;  // behind the groups' sums
+  constexpr int CP = kDwTile + 8;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const int n = n0 + 64 * wn + 32 * j + c;
-      if (n >= N) continue;
+      if (KG == 2 && i != kg) continue;
+      const int nl = 64 * wn + 32 * j + c, n = n0 + nl;
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        const int m = co0 + 64 * wm + 32 * i + mfma32_row(v, g);
-        if (m >= M) continue;
+        const int ml = 64 * wm + 32 * i + mfma32_row(v, g), m = co0 + ml;
         // partials by non-temporal stores (1x1 512 -> 2048 dw 27.2 -> 24.7 us,
         // 3x3 128 -> 128 40.1 -> 39.3 us)
-        if constexpr (PART) __builtin_nontemporal_store(acc[i][j][v], part + (static_cast<int64_t>(split) * M + m) * N + n);
-        else dw[static_cast<int64_t>(m) * N + n] = static_cast<bf16>(acc[i][j][v]);
+        if constexpr (!PART) cs[ml * CP + nl] = static_cast<bf16>(acc[i][j][v]);
+        else if (m < M && n < N)
+          __builtin_nontemporal_store(acc[i][j][v], part + (static_cast<int64_t>(split) * M + m) * N + n);
       }
     }
+  if constexpr (!PART) {
+    // whole rows of the tile, eight bytes a lane
+    __syncthreads();
+#pragma unroll
+    for (int r0 = 0; r0 < kDwTile; r0 += 8 * KG) {
+      const int ml = r0 + static_cast<int>(threadIdx.x) / 32, nl = (tid & 31) * 4;
+      if (co0 + ml < M && n0 + nl < N)
+        *reinterpret_cast<bf16x4 *>(dw + static_cast<int64_t>(co0 + ml) * N + n0 + nl) =
+            *reinterpret_cast<const bf16x4 *>(cs + ml * CP + nl);
+    }
+  }
 }
 
 // dw = sum of the splits' fp32 partials, in split order, rounded to bf16.
@@ -1461,9 +1512,10 @@ static bool conv_dw_mfma_launch(const void *dy, const void *x, void *dw, const C
   const dim3 grid(static_cast<unsigned>(d.tiles_m * d.tiles_n * d.splits));
   const bool rows = q.KH == 1 && q.KW == 1 && q.SH == 1 && q.SW == 1 && q.PH == 0 && q.PW == 0;
   float *part = d.splits > 1 ? static_cast<float *>(scr.ptr) : nullptr;
-  auto kern = d.splits > 1 ? (rows ? conv_dw_mfma<true, true> : conv_dw_mfma<true, false>)
-                           : (rows ? conv_dw_mfma<false, true> : conv_dw_mfma<false, false>);
-  hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, static_cast<const bf16 *>(dy), static_cast<const bf16 *>(x),
+  auto kern = d.splits > 1 ? (rows ? conv_dw_mfma<true, true, 2> : conv_dw_mfma<true, false, 2>)
+              : d.groups   ? (rows ? conv_dw_mfma<false, true, 2> : conv_dw_mfma<false, false, 2>)
+                           : (rows ? conv_dw_mfma<false, true, 1> : conv_dw_mfma<false, false, 1>);
+  hipLaunchKernelGGL(kern, grid, dim3(d.groups ? 512 : 256), 0, s, static_cast<const bf16 *>(dy), static_cast<const bf16 *>(x),
                      static_cast<bf16 *>(dw), part, q, d.tiles_m, d.tiles_n, d.stages_per_split, P);
   if (d.splits > 1) {
     const int64_t mn = static_cast<int64_t>(q.Cout) * q.KH * q.KW * q.Cin;

@@ -283,6 +283,9 @@ MFMA_DW_CASES = [  # bf16 NHWC, groups 1: B, H, Cin, Cout, K, stride, pad
     # and 10 ways (the split sum loads eight partials at a time, then a tail)
     (8, 28, 64, 64, 3, 1, 1),
     (16, 14, 32, 32, 3, 1, 1),
+    # stages shared by two groups of waves (4: 2 + 2, 5: 3 + 2, 6: 3 + 3), too few for it (2, 3), more tiles than CUs
+    (1, 16, 128, 136, 1, 1, 0), (1, 17, 24, 136, 1, 1, 0), (2, 13, 200, 96, 3, 1, 1), (1, 9, 2056, 264, 1, 1, 0),
+    (1, 13, 40, 72, 1, 1, 0), (1, 5, 1040, 4136, 1, 1, 0),
 ]
 
 
