@@ -72,8 +72,8 @@ __device__ __forceinline__ constexpr int mfma32_row(int v, int g) {
 // A later group fills the slots as they come free: longest first, as with
 // more than 64 blocks per head.  (In head order a CU's two workgroups are the
 // same block of two heads, and the longest pair sets the time.)  In us, heads
-// x rows x head_dim: the forward, whose workgroups ran the blocks i and
-// nb - 1 - i in turn before, 64 x 1024 x 64 25.6 -> 22.7, 256 x 256 x 64 15.5
+// x rows x head_dim: the forward, against workgroups that run the blocks i
+// and nb - 1 - i in turn, 64 x 1024 x 64 25.6 -> 22.7, 256 x 256 x 64 15.5
 // -> 13.1, 128 x 400 x 128 26.2 -> 21.2, 10 x 2500 x 128 56.2 -> 48.6, 256 x
 // 2048 x 128 334 -> 329; dq + dk/dv, in head order before and with their masks
 // now compared on edge tiles only (dq, and dk/dv at head_dim 64), 64 x 1024 x

@@ -111,7 +111,7 @@ def test_bf16_config(dev, orc, s, causal):
     # enough query blocks for one query block per workgroup: ragged rows and
     # keys, orders of several heads per group, of odd blocks and of more than 64
     (300, 40, 17, 64, True), (140, 130, 190, 64, True), (75, 257, 129, 128, True), (27, 800, 900, 128, True),
-    (1, 8300, 8260, 128, True), (300, 40, 77, 128, False), (70, 200, 130, 64, False)])
+    (1, 8300, 8260, 128, True), (32, 4070, 4090, 64, True), (300, 40, 77, 128, False), (70, 200, 130, 64, False)])
 def test_bf16_full_grids(dev, orc, bh, nq, nk, d, causal):
     print(f"[attn bf16 full grid] bh={bh} nq={nq} nk={nk} d={d} causal={causal}", flush=True)
     q, k, v = bf16_inputs(np.random.default_rng(nq * 31 + nk), bh, nq, nk, d)
