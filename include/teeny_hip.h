@@ -565,7 +565,8 @@ teeny_status teeny_linear_forward(const void *x, const void *w, const void *b, v
  * dtype F32 or BF16 (every tensor shares it), fp32 accumulation.  Contiguous
  * bf16 operands with N and K multiples of 8 run on the matrix cores (as the
  * gradients of a 1x1 convolution; faster with a stream workspace of
- * teeny_linear_backward_workspace_size bytes); any strides take a tiled
+ * teeny_linear_backward_workspace_size bytes), fp32 ones at any strides on
+ * the fp32 matrix instructions; other bf16 operands take a tiled
  * fp32-accumulating kernel. */
 teeny_status teeny_linear_backward(const void *x, const void *w, const void *dy, void *dx, void *dw, void *db,
                                    int64_t M, int64_t N, int64_t K, int64_t stride_xm, int64_t stride_xk,
