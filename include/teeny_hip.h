@@ -431,7 +431,10 @@ teeny_status teeny_conv2d_backward_workspace_size(int64_t B, int64_t C_IN, int64
  * softmax_scale, neg_inf) with const HEAD_DIM and grid (n_ctx_q, BH, 1),
  * kernels/teeny-kernels/src/nn/attention/flash_attn2.rs:52-158.  Here BH and
  * head_dim are arguments, neg_inf is internal, and `causal` != 0 masks key j
- * from query i when j > i (top-left aligned, as torch's is_causal).
+ * from query i when j > i (top-left aligned, as torch's is_causal).  An
+ * infinity or NaN in a masked row of v does not reach the queries that do not
+ * see it; in the bf16 matrix-core kernels, which multiply whole tiles of keys
+ * by zero probabilities, it may within the row's own block of 64 positions.
  * l is fp32 for every dtype and may be NULL.  head_dim 16, 32, 64, 128 or
  * 256 for both dtypes.  dtype BF16 at head_dim 64 and 128 runs the MFMA flash
  * kernel, which needs 16-byte aligned q/k/v/o and one head's K (and V) below

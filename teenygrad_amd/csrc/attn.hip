@@ -568,12 +568,11 @@ static teeny_status attention_entry(const void *q, const void *k, const void *v,
       a.O = static_cast<bf16 *>(o);
       a.L = l;
       a.part = static_cast<float *>(scr.ptr);
-      a.rows = group * nq;
       a.nq = nq;
       a.nk = nk;
       a.scale_log2 = softmax_scale * kLog2e;
-      if (head_dim == 64) (causal ? attn_split_launch<64, true> : attn_split_launch<64, false>)(plan, a, BH, group, s);
-      else (causal ? attn_split_launch<128, true> : attn_split_launch<128, false>)(plan, a, BH, group, s);
+      if (head_dim == 64) (causal ? attn_split_launch<64, true> : attn_split_launch<64, false>)(plan, a, s);
+      else (causal ? attn_split_launch<128, true> : attn_split_launch<128, false>)(plan, a, s);
       return after_launch(name, s);
     }
     if (head_dim == 64) launch_bf16<64>(q, k, v, o, l, nq, nk, softmax_scale, bh, causal, group, s);

@@ -7,7 +7,10 @@
 // K/V head once per query head that shares it, and runs as many workgroups
 // as there are heads.  Here the query rows that share a K/V head (its query
 // heads times their queries, consecutive in memory) are packed into column
-// blocks of 32; a workgroup of four waves takes one block and a range of the
+// blocks of 32 (causal and more than 32 queries: a head's rows start a new
+// block, whose keys then end with its own last query's, so that a row meets
+// no masked key past the 32-key tile of its block's last row, whose V may
+// hold an infinity or NaN); a workgroup of four waves takes one block and a range of the
 // keys, each wave every fourth 32-key tile of it, and the workgroups of a
 // block meet through the stream's workspace (fp32 partial outputs with their
 // max and sum, combined by a second small kernel in range order).
@@ -30,9 +33,10 @@ struct AttnSplitArgs {
   float *L;
   float *part;        // [unit][range][row][D] fp32, then [unit][range][row][2]; null: one range
   int64_t ml_off;     // offset of the second array in floats
-  int rows;           // query rows per K/V head
+  int rows;           // query rows of a run that blocks are cut from: a K/V head's, or one query head's
+  int kv_runs;        // runs per K/V head
   int nq;             // queries per query head
-  int blocks;         // column blocks per K/V head
+  int blocks;         // column blocks per run
   int nk, range;      // keys, keys per range (a multiple of 32)
   float scale_log2;
 };
@@ -46,12 +50,13 @@ __global__ __launch_bounds__(256, 2) void fa_split_bf16(AttnSplitArgs p) {
   static_assert(RED * 4 >= 32 * D * 2, "the V tile shares the reduction's space");
   auto fv = [](int row) { return (4 * (row / RPB)) & (CPR - 1) & ~3; };
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 31, g = lane >> 5;
-  const int64_t unit = blockIdx.y;  // (K/V head, column block)
-  const int64_t hk = unit / p.blocks;
-  const int c0 = static_cast<int>(unit - hk * p.blocks) * 32, ncol = min(32, p.rows - c0);
-  const int64_t row0 = hk * p.rows + c0;
+  const int64_t unit = blockIdx.y;  // (run, column block)
+  const int64_t run = unit / p.blocks, hk = run / p.kv_runs;
+  const int c0 = static_cast<int>(unit - run * p.blocks) * 32, ncol = min(32, p.rows - c0);
+  const int64_t row0 = run * p.rows + c0;
   const bf16 *Kb = p.K + hk * p.nk * D, *Vb = p.V + hk * p.nk * D;
   // causal: the row's query sees the keys up to its own index, the block's rows those up to their last one's
+  // (of several heads in a block, which have at most 32 queries, up to the heads' last)
   const int qi = CAUSAL ? (c0 + min(c, ncol - 1)) % p.nq : 0;
   int k_end = p.nk;
   if constexpr (CAUSAL) k_end = min(p.nk, c0 % p.nq + ncol > p.nq ? p.nq : c0 % p.nq + ncol);
@@ -212,9 +217,9 @@ __global__ __launch_bounds__(256) void fa_split_combine(AttnSplitArgs p, int ran
   const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= total) return;
-  const int64_t hk = row / p.rows;
-  const int r = static_cast<int>(row - hk * p.rows);
-  const int64_t slot = (hk * p.blocks + r / 32) * ranges * 32 + r % 32;
+  const int64_t run = row / p.rows;
+  const int r = static_cast<int>(row - run * p.rows);
+  const int64_t slot = (run * p.blocks + r / 32) * ranges * 32 + r % 32;
   const float *ml = p.part + p.ml_off;
   float m = -INFINITY;
   for (int i = 0; i < ranges; ++i) m = fmaxf(m, ml[(slot + 32 * i) * 2]);
@@ -251,7 +256,8 @@ __global__ __launch_bounds__(256) void fa_split_combine(AttnSplitArgs p, int ran
 // 19.0, but 8 x 128 x 512 11.0 -> 12.3 with two.
 struct AttnSplitPlan {
   bool use = false;
-  int blocks = 0, ranges = 1, range = 0;
+  int64_t units = 0;
+  int rows = 0, kv_runs = 1, blocks = 0, ranges = 1, range = 0;
   size_t bytes = 0;  // workspace of the ranges
 };
 
@@ -259,9 +265,13 @@ struct AttnSplitPlan {
 inline AttnSplitPlan attn_split_plan(int64_t BH, int64_t group, int64_t nq, int64_t nk, int64_t D, bool causal,
                                      size_t scratch) {
   AttnSplitPlan pl;
-  const int64_t cus = device_cu_count(), blocks = cdiv(group * nq, 32), units = BH / group * blocks;
+  const int64_t kv_runs = causal && nq > 32 ? group : 1, rows = group / kv_runs * nq;
+  const int64_t cus = device_cu_count(), blocks = cdiv(rows, 32), units = BH / group * kv_runs * blocks;
   if (units > (causal && nq > 128 && D == 64 ? 2 : 1) * cus && nq > 32) return pl;
   pl.use = true;
+  pl.units = units;
+  pl.rows = static_cast<int>(rows);
+  pl.kv_runs = static_cast<int>(kv_runs);
   pl.blocks = static_cast<int>(blocks);
   int64_t ranges = units > cus / 2 ? 1 : std::max<int64_t>(1, std::min(2 * cus / units, nk / 512));
   auto size = [&](int64_t n) { return n > 1 ? static_cast<size_t>(units) * n * 32 * (D + 2) * 4 : 0; };
@@ -273,15 +283,16 @@ inline AttnSplitPlan attn_split_plan(int64_t BH, int64_t group, int64_t nq, int6
 }
 
 template <int D, bool CAUSAL>
-inline void attn_split_launch(const AttnSplitPlan &pl, AttnSplitArgs p, int64_t BH, int64_t group, hipStream_t s) {
-  const int64_t units = BH / group * pl.blocks;
+inline void attn_split_launch(const AttnSplitPlan &pl, AttnSplitArgs p, hipStream_t s) {
+  p.rows = pl.rows;
+  p.kv_runs = pl.kv_runs;
   p.blocks = pl.blocks;
   p.range = pl.range;
-  p.ml_off = units * pl.ranges * 32 * D;
+  p.ml_off = pl.units * pl.ranges * 32 * D;
   if (pl.ranges == 1) p.part = nullptr;
-  hipLaunchKernelGGL((fa_split_bf16<D, CAUSAL>), dim3(pl.ranges, static_cast<unsigned>(units)), dim3(256), 0, s, p);
+  hipLaunchKernelGGL((fa_split_bf16<D, CAUSAL>), dim3(pl.ranges, static_cast<unsigned>(pl.units)), dim3(256), 0, s, p);
   if (pl.ranges > 1) {
-    const int64_t total = BH / group * p.rows;
+    const int64_t total = pl.units / pl.blocks * p.rows;
     hipLaunchKernelGGL(fa_split_combine<D>, dim3(static_cast<unsigned>(cdiv(total, 4))), dim3(256), 0, s, p, pl.ranges,
                        total);
   }

@@ -63,3 +63,24 @@ def test_rows_past_the_keys(dev, orc):
         o = K.flash_attention(*(dev.upload(to_bf16(a), tg.bf16) for a in (q, k, v))).to_host()
     check_bf16(o[:1], oo, "o")
     assert np.isnan(from_bf16(o[1])).all()
+
+
+@pytest.mark.parametrize("b,hq,hkv,n,cut,d", [
+    # `cut`: the first row that holds no numbers, at a 64-key tile's edge; the rows before it see no key from there on
+    (1, 2, 1, 200, 128, 128), (1, 8, 2, 100, 64, 64), (2, 6, 2, 77, 64, 64), (1, 4, 1, 333, 256, 128)])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_causal_rows_without_numbers(dev, orc, b, hq, hkv, n, cut, d, bad):
+    # a padded batch: early queries of every head of a group, the ones that
+    # follow another head's last query in a column block among them
+    rng = np.random.default_rng(n + d)
+    q, k, v = (from_bf16(to_bf16(rng.standard_normal((m, n, d), dtype=np.float32))) for m in (b * hq, b * hkv, b * hkv))
+    oo, ol = orc.flash_attention(q, *(np.repeat(a, hq // hkv, axis=0) for a in (k, v)), 1 / np.sqrt(d), True)
+    k[:, cut:], v[:, cut:] = bad, bad
+    bufs = [dev.upload(to_bf16(a), tg.bf16) for a in (q, k, v)]
+    for ws in (K.attention_workspace_size(b, hq, hkv, n, n, d, True), 0):
+        print(f"[attn split] masked b={b} hq={hq} hkv={hkv} n={n} cut={cut} d={d} bad={bad} workspace={ws}", flush=True)
+        lse = tg.Buffer(tg.f32, (b * hq, n))
+        with stream_workspace(dev, ws):
+            o = K.attention(*bufs, hq, hkv, causal=True, lse=lse).to_host()
+        check_bf16(o[:, :cut], oo[:, :cut], "o")
+        assert np.max(np.abs(lse.to_host()[:, :cut] - ol[:, :cut])) < 1e-3
