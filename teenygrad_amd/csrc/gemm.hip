@@ -44,15 +44,17 @@ __global__ __launch_bounds__(256) void gemm_generic(const TA *__restrict__ A, in
   const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
   const int m0 = blockIdx.y * T, n0 = blockIdx.x * T;
   float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += KC) {
+  const uint32_t Ku = static_cast<uint32_t>(K);  // the last k0 + KC may pass 2^31
+  for (uint32_t k0 = 0; k0 < Ku; k0 += KC) {
     for (int i = threadIdx.x; i < KC * T; i += 256) {
       const int kk = i % KC, r = i / KC;
-      const int m = m0 + r, n = n0 + r, k = k0 + kk;
-      as[kk][r] = (m < M && k < K) ? ld_f32(A, m * sam + k * sak) : 0.0f;
-      bs[kk][r] = (n < N && k < K) ? ld_f32(B, n * sbn + k * sbk) : 0.0f;
+      const int m = m0 + r, n = n0 + r;
+      const uint32_t k = k0 + kk;
+      as[kk][r] = (m < M && k < Ku) ? ld_f32(A, m * sam + k * sak) : 0.0f;
+      bs[kk][r] = (n < N && k < Ku) ? ld_f32(B, n * sbn + k * sbk) : 0.0f;
     }
     __syncthreads();
-    const int kn = min(KC, K - k0);
+    const int kn = static_cast<int>(min<uint32_t>(KC, Ku - k0));
     for (int kk = 0; kk < kn; ++kk) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)

@@ -38,7 +38,7 @@ struct GemmF32Params {
   int64_t scm, scn;    // strides of C
   int64_t slice;       // elements between partial slices
   int M, N, K;
-  int k_len;           // k's per split (a multiple of the chunk but for the last)
+  uint32_t k_len;      // k's per split (a multiple of the chunk: K rounded up, 2^31 at most)
   int tiles_n;
 };
 
@@ -125,7 +125,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_mfma(GemmF32Params
   const int wk = w % WK, wn = w / WK % WN, wm = w / WK / WN;
   const int tile = xcd_remap(blockIdx.x, gridDim.x);
   const int m0 = tile / p.tiles_n * BM, n0 = tile % p.tiles_n * BN;
-  const int kb = blockIdx.y * p.k_len, ke = min(p.K, kb + p.k_len);
+  // K may be 2^31 - 1: no end past K is formed, and rounded-up counts are unsigned
+  const int kb = static_cast<int>(blockIdx.y * p.k_len);
+  const uint32_t k_count = min(static_cast<uint32_t>(p.K - kb), p.k_len);
   OA a;
   OB b;
   a.init(p.A, p.sa, p.M, p.K, m0);
@@ -137,12 +139,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_mfma(GemmF32Params
 #pragma unroll
     for (int j = 0; j < NI; ++j) acc[i][j] = zero16();
 
-  const int n_chunks = (ke - kb + kF32KC - 1) / kF32KC;
+  const int n_chunks = static_cast<int>((k_count + kF32KC - 1) / kF32KC);
   f32x4 ra[2][OA::NV], rb[2][OB::NV];
   auto fetch = [&](int set, int chunk) {
     if (chunk >= n_chunks) return;
     const int k0 = kb + chunk * kF32KC;
-    if (k0 + kF32KC <= p.K) {
+    if (static_cast<uint32_t>(k0) + kF32KC <= static_cast<uint32_t>(p.K)) {
       a.template fetch<false>(ra[set], tid, k0);
       b.template fetch<false>(rb[set], tid, k0);
     } else {
@@ -192,7 +194,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_mfma(GemmF32Params
   };
   constexpr std::integral_constant<int, 0> s0{};
   constexpr std::integral_constant<int, 1> s1{};
-  const int n_full = (ke - kb) / kF32KC;
+  const int n_full = static_cast<int>(k_count / kF32KC);
   int ch = 0;
   for (; ch + 4 < n_full; ch += 2) {
     step(s0, std::true_type{}, ch);
@@ -266,13 +268,14 @@ __global__ __launch_bounds__(256) void gemm_f32_splitk_sum(const float *__restri
 }
 
 struct GemmF32Plan {
-  int bm, bn, splits, k_len;
+  int bm, bn, splits;
+  uint32_t k_len;
 };
 
 // Tile and split for one GEMM.  scratch: bytes of workspace that may hold slices.
 inline GemmF32Plan gemm_f32_plan(int64_t M, int64_t N, int64_t K, size_t scratch) {
   const int cus = device_cu_count();
-  GemmF32Plan pl{64, 64, 1, static_cast<int>(cdiv(K, kF32KC) * kF32KC)};
+  GemmF32Plan pl{64, 64, 1, static_cast<uint32_t>(cdiv(K, kF32KC) * kF32KC)};
   if (M <= 32) pl.bm = 32;
   else if (cdiv(M, 128) * cdiv(N, 128) >= 2 * cus) pl.bm = pl.bn = 128;
   const int64_t tiles = cdiv(M, pl.bm) * cdiv(N, pl.bn);
@@ -282,7 +285,7 @@ inline GemmF32Plan gemm_f32_plan(int64_t M, int64_t N, int64_t K, size_t scratch
     s = std::min<int64_t>(s, static_cast<int64_t>(scratch / (static_cast<size_t>(M) * N * 4)));
     if (s > 1) {
       const int64_t chunks = cdiv(cdiv(K, kF32KC), s);
-      pl.k_len = static_cast<int>(chunks * kF32KC);
+      pl.k_len = static_cast<uint32_t>(chunks * kF32KC);
       pl.splits = static_cast<int>(cdiv(K, pl.k_len));
     }
   }

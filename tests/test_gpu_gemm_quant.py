@@ -128,6 +128,27 @@ def test_linear_f32_strides(dev, m, n, k, xt, wt):
             assert np.all(err <= bound), f"{np.max(err - bound)} beyond the bound"
 
 
+@pytest.mark.parametrize("k", [2 ** 31 - 1, 2 ** 31 - 31, 2 ** 31 - 32, 2 ** 31 - 33])
+def test_linear_f32_longest_k(dev, k):
+    # the last chunk and the last of 512 slices end at, or would end past, the
+    # largest 32-bit count; strides of 0 along k: every product is x[m] w[n]
+    m = n = 4
+    x, w, b = np.arange(1, 5, dtype=np.float32), np.float32([0.5, -1, 2, 4]), np.float32([1, 2, 3, 4])
+    y = tg.Buffer(tg.f32, (m, n))
+    xb, wb, bb = dev.upload(x), dev.upload(w), dev.upload(b)
+    need = K.linear_workspace_size(m, n, k, tg.f32)
+    assert need > 0
+    print(f"[linear f32] K={k} workspace={need}", flush=True)
+    with stream_workspace(dev, need):
+        tg.check(_lib.lib.teeny_linear_forward(xb.ptr, wb.ptr, bb.ptr, y.ptr, m, n, k, 1, 0, 1, 0, n, 1,
+                                               tg.f32.code, None))
+        got = y.to_host().astype(np.float64)
+    # four waves share a slice's 2^22 k's: their sums of 2^20 small multiples of 0.5 are exact, and
+    # adding the 512 slices rounds by at most 512 * 2^-24 = 2^-15; a slice left out would show as 2^-9
+    ref = float(k) * np.outer(x, w).astype(np.float64) + b
+    assert np.all(np.abs(got - ref) <= 2.0 ** -12 * np.abs(ref)), got / ref
+
+
 def with_scratch(dev, scratch, need, fn):
     """Runs fn() with no stream workspace, or with one of ``need`` bytes."""
     if scratch == "workspace":
