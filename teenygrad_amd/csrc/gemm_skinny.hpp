@@ -186,6 +186,8 @@ inline int gemm_skinny_nb(int64_t M, int64_t N) { return M <= 16 || N < 16 * 2 *
 // split.  Weights rotated through 600 MB.
 inline bool gemm_skinny_ok(bool int8, int64_t M, int64_t N, int64_t K) {
   if (K % 16 != 0 || M > 64) return false;
+  // 2^32 threads in a grid (more of them wrap): the tiles want 4 a column, not 32
+  if (cdiv(N, 16 * gemm_skinny_nb(M, N)) >= (int64_t{1} << 32) / 512) return false;
   return M <= 32 || ((N >= 16 * 64 || K < 2048) && (int8 || gemm_skinny_nb(M, N) < 4));
 }
 

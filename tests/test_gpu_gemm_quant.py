@@ -91,6 +91,22 @@ def test_few_rows(dev, m, n, k, weights):
     assert np.all(err <= bound), f"{np.max(err - bound)} beyond the bound"
 
 
+def test_few_rows_widest(dev):
+    # 2^27 columns: 2^32 threads at 512 for every 16 columns, past what a launch takes
+    n, k, at = 2 ** 27, 16, [0, 1, 2 ** 26 - 1, 2 ** 26, 2 ** 27 - 9, 2 ** 27 - 1]
+    x, q, scale = np.full((1, k), 0.5, np.float32), tg.Buffer(tg.i8, (n, k)), tg.Buffer(tg.f32, (n,))
+    xb = dev.upload(to_bf16(x), tg.bf16)
+    tg.check(_lib.lib.teeny_hip_memset(q.ptr, 1, q.nbytes, None))
+    tg.check(_lib.lib.teeny_hip_memset(scale.ptr, 0, scale.nbytes, None))
+    vals = np.arange(1, len(at) + 1, dtype=np.float32)
+    for i, v in zip(at, vals):
+        tg.check(_lib.lib.teeny_hip_memcpy_h2d(scale.ptr + 4 * i, np.float32([v]).ctypes.data, 4, None))
+    print(f"[few rows] M=1 N={n} K={k} int8", flush=True)
+    got = K.w8a16_linear(xb, q, scale).to_host().reshape(-1)
+    np.testing.assert_array_equal(from_bf16(got[at]), 8 * vals)  # 16 times 0.5, times the scale
+    assert np.count_nonzero(got) == len(at)
+
+
 F32_GEMM = [  # (M, N, K): tile edges, ragged vectors, k tails, splits, fewer than a 16-byte load spans
     (1, 5, 4), (3, 3, 3), (31, 65, 29), (33, 64, 31), (64, 64, 32), (65, 63, 33), (129, 127, 97), (4, 4, 161),
     (5, 1000, 700), (200, 72, 3001), (2300, 2200, 40)]
