@@ -187,13 +187,14 @@ static void launch_linear_db(const T *dy, int64_t sm, int64_t sn, T *db, int64_t
   if (scratch.ptr == nullptr || scratch.bytes < static_cast<size_t>(shares) * N * 4) shares = 1;
   float *part = shares > 1 ? static_cast<float *>(scratch.ptr) : nullptr;
   const int rows = static_cast<int>(cdiv(M, shares));
-  const dim3 grid(static_cast<unsigned>(cdiv(N, vec ? 4 * V : 32)), static_cast<unsigned>(shares));
-  if (vec)
-    hipLaunchKernelGGL((linear_bwd_db<T, V, 4>), grid, dim3(1024), 0, s, dy, sm, sn, db, sdb, part,
-                       static_cast<int>(M), static_cast<int>(N), rows);
-  else
-    hipLaunchKernelGGL((linear_bwd_db<T, 1, 32>), grid, dim3(1024), 0, s, dy, sm, sn, db, sdb, part,
-                       static_cast<int>(M), static_cast<int>(N), rows);
+  auto kern = vec ? linear_bwd_db<T, V, 4> : linear_bwd_db<T, 1, 32>;
+  const int64_t cols = vec ? 4 * V : 32;
+  // 2^31 threads a launch at most: a grid of 2^32 wraps (shares > 1 only far below)
+  for (int64_t n0 = 0, step = cols << 21; n0 < N; n0 += step) {
+    const int64_t n = std::min(step, N - n0);
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(cdiv(n, cols)), static_cast<unsigned>(shares)), dim3(1024), 0, s,
+                       dy + n0 * sn, sm, sn, db + n0 * sdb, sdb, part, static_cast<int>(M), static_cast<int>(n), rows);
+  }
   if (part != nullptr)
     hipLaunchKernelGGL(linear_bwd_db_sum<T>, dim3(static_cast<unsigned>(cdiv(N, 256))), dim3(256), 0, s, part,
                        static_cast<int>(shares), db, sdb, static_cast<int>(N));

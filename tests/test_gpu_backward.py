@@ -434,6 +434,28 @@ def test_linear_backward_bias_gradient(dev, dtype, m, n, pad):
         assert np.all(err <= limit), f"db: {np.max(err - limit)} beyond its bound"
 
 
+@pytest.mark.parametrize("dtype,n", [("bf16", 2 ** 27 + 5), ("bf16", 2 ** 27 + 32), ("f32", 2 ** 26 + 16)])
+def test_linear_backward_bias_gradient_widest(dev, dtype, n):
+    # more columns than 2^32 threads have at 1024 for every 32 (16 of fp32 by
+    # vectors); K = 0, so that db alone is computed; both rows of dy the same memory
+    from teenygrad_amd._lib import check as chk, lib
+    tdt = tg.bf16 if dtype == "bf16" else tg.f32
+    dy, db = tg.Buffer(tdt, (n,)), tg.Buffer(tdt, (n,))
+    chk(lib.teeny_hip_memset(dy.ptr, 0, dy.nbytes, None))
+    chk(lib.teeny_hip_memset(db.ptr, 0xFF, db.nbytes, None))
+    at = [0, 31, 2 ** 25, 2 ** 26 - 1, 2 ** 26, n - 9, n - 1]
+    vals = np.arange(1, len(at) + 1, dtype=np.float32)
+    for j, v in zip(at, vals):
+        v = to_bf16(vals[:1] * v) if dtype == "bf16" else vals[:1] * v
+        chk(lib.teeny_hip_memcpy_h2d(dy.ptr + j * v.itemsize, v.ctypes.data, v.itemsize, None))
+    print(f"[linear db] {dtype} M=2 N={n}", flush=True)
+    chk(lib.teeny_linear_backward(None, None, dy.ptr, None, None, db.ptr, 2, n, 0, 0, 1, 1, 0, 0, 1, 0, 1, 1, 0, 1,
+                                  tdt.code, None))
+    got = db.to_host()
+    np.testing.assert_array_equal(from_bf16(got[at]) if dtype == "bf16" else got[at], 2 * vals)
+    assert np.count_nonzero(got) == len(at)
+
+
 def test_linear_backward_strided_and_empty(dev, orc):
     # x given transposed in memory (stride_xm 1, stride_xk M) and dy rows
     # padded to 16 bytes (the RuntimeOp's backward_grad_output_row_stride):
