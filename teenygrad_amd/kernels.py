@@ -95,7 +95,7 @@ class DispatchPacker(ArgVisitor):
 
 
 def _prod(s: Sequence[int]) -> int:
-    return int(math.prod(s))
+    return math.prod(map(int, s))  # a caller's shape may hold numpy integers, whose products wrap
 
 
 def _need(cond: bool, msg: str) -> None:
@@ -861,8 +861,9 @@ def _out(like: Buffer, out: Optional[Buffer], shape=None, dtype=None) -> Buffer:
     shape = like.shape if shape is None else tuple(shape)
     dtype = from_any(dtype) if dtype else like.dtype
     if out is not None:
-        if out.numel != _prod(shape):
-            raise ValueError(f"output holds {out.numel} elements, op writes {_prod(shape)}")
+        n = like.numel if shape is like.shape else _prod(shape)
+        if out.numel != n:
+            raise ValueError(f"output holds {out.numel} elements, op writes {n}")
         if out.dtype != dtype:
             raise ValueError(f"output dtype {out.dtype.name}, op writes {dtype.name}")
         return out

@@ -167,6 +167,16 @@ def test_attention_and_norm_shape_rules():
         kernels.norm_dims((16, 128), (127,))
 
 
+@pytest.mark.parametrize("dtype", [np.int8, np.int16, np.int32, np.int64])
+def test_shapes_of_numpy_integers(dtype):
+    # element counts past what one of the shape's own integers holds
+    d = {np.int8: 16, np.int16: 256}.get(dtype, 65536)
+    for shape in (np.array([d, d, 3], dtype), tuple(np.array([d, d, 3], dtype)), (dtype(d), d, 3), [d, dtype(d), 3]):
+        assert kernels._prod(shape) == 3 * d * d and type(kernels._prod(shape)) is int
+    op = kernels.LayerNormForwardInferenceRuntimeOp(1024, 1e-5)
+    assert op.grid(np.array([d, 4, 8], dtype)) == (4 * d, 1, 1)
+
+
 def test_runtime_op_buffer_check_uses_param_shapes():
     class FakeBuf(kernels.Buffer):
         def __init__(self, n):  # no device allocation
