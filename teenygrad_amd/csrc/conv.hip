@@ -1306,8 +1306,10 @@ __global__ __launch_bounds__(256 * KG, 2) void conv_dw_mfma(const bf16 *__restri
   // pixels per stage with adds: dividing the pixel index of every row of every
   // stage took longer than the stage's products (dw of 2000 x 1024 -> 4096
   // 46 -> 34 us, of 28x28 3x3 128 -> 128 at batch 64 38.5 -> 30.7 us).  Rows
-  // past the last pixel lie past the extents, a column past the edge starts at
-  // kOffNone and stays above them, and both read as zeros.
+  // past the last pixel lie past the extents and read as zeros; where 32 bits
+  // could not hold them there is only one stage (fewer than 64 pixels, of 2^24
+  // channels), so those that the first stage has are told by their index.  A
+  // column past the edge starts at kOffNone; it reaches no output.
   const int rpx = ROWS ? 0 : q.OW * q.OH;
   const int d_bb = ROWS ? 0 : kDwStage / rpx, d_oh = ROWS ? 0 : kDwStage % rpx / q.OW, d_ow = ROWS ? 0 : kDwStage % q.OW;
   const int px = q.Cin * 2;  // bytes per pixel of x
@@ -1319,14 +1321,14 @@ __global__ __launch_bounds__(256 * KG, 2) void conv_dw_mfma(const bf16 *__restri
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int p = st0 * kDwStage + 16 * i + lrow;
-    aoff[i] = a_col < M ? (p * M + a_col) * 2 : kOffNone;
+    aoff[i] = a_col < M && p < P ? (p * M + a_col) * 2 : kOffNone;
     if constexpr (ROWS) {
       ih[i] = iw[i] = 0;
-      boff[i] = nb < N ? p * px + ci * 2 : kOffNone;
+      boff[i] = nb < N && p < P ? p * px + ci * 2 : kOffNone;
     } else {
       const int r = p / q.OW, bb = r / q.OH;
       iw[i] = (p - r * q.OW) * q.SW - q.PW + kw;
-      ih[i] = (r - bb * q.OH) * q.SH - q.PH + kh;
+      ih[i] = p < P ? (r - bb * q.OH) * q.SH - q.PH + kh : -1;
       boff[i] = ((bb * q.H + ih[i]) * q.W + iw[i]) * px + ci * 2;
     }
   }

@@ -334,6 +334,27 @@ def test_conv_backward_combined_and_dispatch_hooks(dev, orc):
     assert op.has_backward()
 
 
+@pytest.mark.parametrize("stride", [1, 2])  # the rows of x as they lie, and through the gather
+def test_conv_backward_dw_widest(dev, stride):
+    # two pixels of 2^26 channels: the 62 other rows of a 64-pixel stage lie past 2^32
+    # bytes and must read as zeros, or an infinity in dy meets a zero of x
+    from teenygrad_amd._lib import check as chk, lib
+    n, k = 2 ** 26, 8
+    x = np.arange(1, 2 * k + 1, dtype=np.float32).reshape(2, 1, 1, k)
+    at = [0, 129, 2 ** 25 + 7, n - 1]
+    vals = np.float32([[np.inf, 2], [3, -np.inf], [np.inf, 5], [-7, 11]])
+    dy = tg.Buffer(tg.bf16, (2, 1, 1, n))
+    chk(lib.teeny_hip_memset(dy.ptr, 0, dy.nbytes, None))
+    for j, pair in zip(at, vals):
+        for r in range(2):
+            v = to_bf16(pair[r:r + 1])
+            chk(lib.teeny_hip_memcpy_h2d(dy.ptr + 2 * (r * n + j), v.ctypes.data, 2, None))
+    print(f"[conv dw] 2 pixels C_OUT={n} stride={stride}", flush=True)
+    dw = K.conv2d_backward_dw(dy, dev.upload(to_bf16(x), tg.bf16), (n, 1, 1, k), stride, 0, 1, "nhwc").to_host()
+    np.testing.assert_array_equal(from_bf16(dw[at]).reshape(len(at), k), vals @ x.reshape(2, k))
+    assert np.count_nonzero(dw) == len(at) * k
+
+
 def test_conv_backward_empty_batch_zeroes_dw(dev):
     # no images: dw is the sum over no pixels, written as zeros
     w_shape = (8, 4, 3, 3)
