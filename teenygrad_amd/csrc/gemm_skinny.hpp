@@ -33,17 +33,17 @@ __global__ __launch_bounds__(64 * KW) void gemm_skinny(GemmParams p) {
   __shared__ __attribute__((aligned(16))) float lds[KW * (XT > RED ? XT : RED)];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * 16 * NB;
-  const int chunks = (p.K + 63) / 64, per = (chunks + KW - 1) / KW;
+  const int chunks = p.K / 64 + (p.K % 64 != 0), per = (chunks + KW - 1) / KW;
   const int cb = min(chunks, w * per), ce = min(chunks, cb + per);
   bf16 *xt = reinterpret_cast<bf16 *>(lds + w * XT);
   // k's of lane group g in a chunk: 16 g .. 16 g + 15 (one 16-byte vector of
   // int8), or 8 g and 32 + 8 g (two of bf16)
   constexpr int KG = INT8B ? 16 : 8;
-  const char *wrow[NB];
+  using W = std::conditional_t<INT8B, int8_t, bf16>;
+  const W *wrow[NB];
 #pragma unroll
   for (int i = 0; i < NB; ++i)
-    wrow[i] = static_cast<const char *>(p.B) +
-              (static_cast<int64_t>(min(n0 + 16 * i + r, p.N - 1)) * p.ldb + KG * g) * (INT8B ? 1 : 2);
+    wrow[i] = static_cast<const W *>(p.B) + static_cast<int64_t>(min(n0 + 16 * i + r, p.N - 1)) * p.ldb + KG * g;
 
   f32x4 acc[NB][MB];
 #pragma unroll
@@ -57,27 +57,27 @@ __global__ __launch_bounds__(64 * KW) void gemm_skinny(GemmParams p) {
   const u32x4 none = {0u, 0u, 0u, 0u};
   // chunks c .. c + U - 1; WHOLE: all of them exist and end by K.  Otherwise
   // what lies past K or the wave's slice reads as zero (K % 16 == 0: a vector
-  // is inside or outside as a whole); its load goes to the row's start.
+  // is inside or outside as a whole); its load goes to the row's start.  K may
+  // be 2^31 - 16 and the last chunks then end past 2^31: compared unsigned.
   auto load = [&](auto whole_, Group &q, int c) __attribute__((always_inline)) {
     constexpr bool WHOLE = decltype(whole_)::value;
-    const int k_end = min(64 * ce, p.K);
+    const uint32_t k_end = min(64u * ce, static_cast<uint32_t>(p.K));
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int i = 0; i < NB; ++i)
 #pragma unroll
         for (int v = 0; v < WV; ++v) {
-          const int k = 64 * (c + u) + 32 * v;
-          const bool in = WHOLE || k + KG * g < k_end;
-          q.w[u][i][v] = *reinterpret_cast<const u32x4 *>(wrow[i] + (in ? k : -KG * g) * (INT8B ? 1 : 2));
+          const bool in = WHOLE || 64u * (c + u) + 32 * v + KG * g < k_end;
+          q.w[u][i][v] = *reinterpret_cast<const u32x4 *>(wrow[i] + (in ? 64 * (c + u) + 32 * v : -KG * g));
           if (!in) q.w[u][i][v] = none;
         }
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
-      const int t = 64 * i + lane, k = 64 * c + 8 * (t % (8 * U));
-      const bool in = WHOLE || k < k_end;
+      const int t = 64 * i + lane, col = 8 * (t % (8 * U));
+      const bool in = WHOLE || 64u * c + col < k_end;
       const int64_t row = min(t / (8 * U), p.M - 1);
-      q.x[i] = *reinterpret_cast<const u32x4 *>(p.A + row * p.lda + (in ? k : 0));
+      q.x[i] = *reinterpret_cast<const u32x4 *>(p.A + row * p.lda + (in ? 64 * c + col : 0));
       if (!in) q.x[i] = none;
     }
   };

@@ -107,6 +107,28 @@ def test_few_rows_widest(dev):
     assert np.count_nonzero(got) == len(at)
 
 
+@pytest.mark.parametrize("k", [2 ** 30 + 48, 2 ** 31 - 64, 2 ** 31 - 16])
+@pytest.mark.parametrize("weights", ["int8", "bf16"])
+def test_few_rows_longest_k(dev, k, weights):
+    # offsets past 2^31 bytes in bf16; ends of chunks and of groups of them past 2^31 products
+    at = [0, 63, 2 ** 28 - 1, 2 ** 29, 2 ** 30 - 1, 2 ** 30, k - 33, k - 32, k - 16, k - 1]
+    vals = np.arange(1, len(at) + 1, dtype=np.float32)
+    x, y = tg.Buffer(tg.bf16, (1, k)), tg.Buffer(tg.bf16, (1, 1))
+    w = tg.Buffer(tg.i8 if weights == "int8" else tg.bf16, (1, k))
+    for buf in (x, w):
+        tg.check(_lib.lib.teeny_hip_memset(buf.ptr, 0, buf.nbytes, None))
+        for j, v in zip(at, vals):
+            v = np.int8([v]) if buf.dtype == tg.i8 else to_bf16(np.float32([v]))
+            tg.check(_lib.lib.teeny_hip_memcpy_h2d(buf.ptr + j * v.itemsize, v.ctypes.data, v.itemsize, None))
+    print(f"[few rows] M=1 N=1 K={k} {weights}", flush=True)
+    if weights == "int8":
+        K.w8a16_linear(x, w, dev.upload(np.float32([0.5])), y=y)
+    else:
+        K.linear(x, w, y=y)
+    ref = float(np.sum(vals * vals)) * (0.5 if weights == "int8" else 1.0)
+    assert from_bf16(y.to_host()).reshape(-1)[0] == from_bf16(to_bf16(np.float32([ref])))[0]
+
+
 F32_GEMM = [  # (M, N, K): tile edges, ragged vectors, k tails, splits, fewer than a 16-byte load spans
     (1, 5, 4), (3, 3, 3), (31, 65, 29), (33, 64, 31), (64, 64, 32), (65, 63, 33), (129, 127, 97), (4, 4, 161),
     (5, 1000, 700), (200, 72, 3001), (2300, 2200, 40)]
