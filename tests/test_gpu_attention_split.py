@@ -84,3 +84,24 @@ def test_causal_rows_without_numbers(dev, orc, b, hq, hkv, n, cut, d, bad):
             o = K.attention(*bufs, hq, hkv, causal=True, lse=lse).to_host()
         check_bf16(o[:, :cut], oo[:, :cut], "o")
         assert np.max(np.abs(lse.to_host()[:, :cut] - ol[:, :cut])) < 1e-3
+
+
+@pytest.mark.parametrize("b,hq,hkv,nq,nk,d", [
+    (1, 8, 2, 64, 4096, 128), (1, 1, 1, 5, 16384, 64), (2, 8, 8, 100, 2048, 64), (1, 2, 1, 128, 1100, 128), (1, 4, 2, 700, 3000, 64)])
+def test_causal_keys_past_the_queries(dev, orc, b, hq, hkv, nq, nk, d):
+    # keys that no query sees take no part: no numbers there, and no share of the plan
+    assert K.attention_workspace_size(b, hq, hkv, nq, nk, d, True) == K.attention_workspace_size(b, hq, hkv, nq, nq, d, True)
+    rng = np.random.default_rng(nq + nk)
+    q, k, v = (from_bf16(to_bf16(rng.standard_normal((m, n, d), dtype=np.float32)))
+               for m, n in ((b * hq, nq), (b * hkv, nk), (b * hkv, nk)))
+    oo, ol = orc.flash_attention(q, *(np.repeat(a[:, :nq], hq // hkv, axis=0) for a in (k, v)), 1 / np.sqrt(d), True)
+    cut = -(-nq // 64) * 64  # the edge of the last queries' own tile
+    k[:, cut:], v[:, cut:] = np.nan, np.nan
+    bufs = [dev.upload(to_bf16(a), tg.bf16) for a in (q, k, v)]
+    for ws in {K.attention_workspace_size(b, hq, hkv, nq, nk, d, True), 0}:
+        print(f"[attn split] causal b={b} hq={hq} hkv={hkv} nq={nq} nk={nk} d={d} workspace={ws}", flush=True)
+        lse = tg.Buffer(tg.f32, (b * hq, nq))
+        with stream_workspace(dev, ws):
+            o = K.attention(*bufs, hq, hkv, causal=True, lse=lse).to_host()
+        check_bf16(o, oo, "o")
+        assert np.max(np.abs(lse.to_host() - ol)) < 1e-3
