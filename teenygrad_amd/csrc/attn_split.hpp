@@ -249,11 +249,21 @@ __global__ __launch_bounds__(256) void fa_split_combine(AttnSplitArgs p, int ran
 // 12.0 / 10.2, 8 x 2048 x 2048 30.8 / 24.6, while 128 does not, 16 x 1024 x 1024
 // 25.2 / 27.4, 32 x 512 x 512 16.5 / 17.7, 8 x 2048 x 2048 41.1 / 44.5;
 // 1024 blocks, 64 x 512 x 512 x 128 16.6 / 32.0.  At up to 32 queries most of
-// fa_fwd_bf16's rows are padding and this path is taken at any size: 32 heads
-// sharing 8 K/V heads, one query, batch x keys 1 x 16384 262 / 31, 32 x 1000
-// 57 / 23, 16 x 4000 106 / 52 (5 TB/s).  Ranges cost a second launch and pay
-// from about 512 keys each: 8 x 64 x 2048 25.3 -> 15.1, 8 x 128 x 4096 44.3 ->
-// 19.0, but 8 x 128 x 512 11.0 -> 12.3 with two.
+// fa_fwd_bf16's rows are padding: 32 heads sharing 8 K/V heads, one query, batch
+// x keys 1 x 16384 262 / 31, 32 x 1000 57 / 23, 16 x 4000 106 / 52 (5 TB/s).  On
+// a full chip that counts where packing leaves fewer blocks than heads (heads in
+// groups of 4 or 8; queries x keys x head_dim): 32 x 2048 x 128, as many blocks
+// as heads, 512 of them 55 / 79, 4096 1.19 times as long; 20 x 2048 x 128, 5
+// blocks to 8 heads, 320 54 / 61, 640 0.93; half as many blocks or fewer 0.16 to
+// 0.77 at any size.  head_dim 64, 32 x 2048, as many blocks as heads: 512 35 /
+// 40, 2048 1.09, 4096 0.9; fewer blocks than heads, or causal and so one tile of
+// keys, 0.1 to 1.07.  Heads that share no K/V gain (0.94 and 0.89 on average)
+// but for one tile of keys per wave at 128, 512 x 32 x 64 6.9 / 8.5.  With so
+// few keys at head_dim 128 also a chip that is not full waits for this path's
+// longer way to its first product and its merge: 16 x 32 x 64 5.0 / 5.9, 33 x
+// 128 5.6 / 6.2, but 100 x 128 0.94 and with 4 rows 0.96.  Ranges cost a second
+// launch and pay from about 512 keys each: 8 x 64 x 2048 25.3 -> 15.1, 8 x 128 x
+// 4096 44.3 -> 19.0, but 8 x 128 x 512 11.0 -> 12.3 with two.
 struct AttnSplitPlan {
   bool use = false;
   int64_t units = 0;
@@ -271,6 +281,12 @@ inline AttnSplitPlan attn_split_plan(int64_t BH, int64_t group, int64_t nq, int6
   const int64_t kv_runs = causal && nq > 32 ? group : 1, rows = group / kv_runs * nq;
   const int64_t cus = device_cu_count(), blocks = cdiv(rows, 32), units = BH / group * kv_runs * blocks;
   if (units > (causal && nq > 128 && D == 64 ? 2 : 1) * cus && nq > 32) return pl;
+  if (units > cus && nq <= 32) {
+    const bool packed = D == 64 ? units < BH || units > 8 * cus || nk <= 32
+                                : 2 * units <= BH || (4 * units <= 3 * BH && units > 3 * cus);
+    if (group > 1 ? !packed : D == 128 && nq > 16 && nk <= 64) return pl;
+  }
+  if (D == 128 && !causal && nk <= 128 && nq <= 64 && group * nq > 8 && BH <= cus) return pl;
   pl.use = true;
   pl.units = units;
   pl.rows = static_cast<int>(rows);

@@ -13,7 +13,12 @@ pytestmark = pytest.mark.gpu
 CASES = [  # batch, q_heads, kv_heads, nq, nk, d: rows of a column block, tile and range edges
     (1, 1, 1, 1, 1, 128), (2, 2, 1, 1, 31, 64), (1, 8, 2, 1, 129, 128), (3, 4, 4, 2, 512, 64),
     (1, 32, 4, 5, 1000, 128), (2, 8, 1, 4, 257, 64), (1, 3, 1, 32, 700, 128), (1, 2, 2, 31, 2049, 64),
-    (2, 16, 2, 1, 3001, 128), (1, 1, 1, 32, 33, 128)]
+    (2, 16, 2, 1, 3001, 128), (1, 1, 1, 32, 33, 128),
+    # both sides of the plan's lines on a full chip (256 CUs): blocks as many as heads, 5 to 8 heads (400, 800 of
+    # them), 7 to 8; one tile of keys per wave
+    (36, 16, 2, 32, 70, 128), (20, 32, 4, 20, 70, 128), (40, 32, 4, 20, 70, 128), (10, 64, 8, 28, 70, 64),
+    (80, 8, 2, 32, 40, 64), (65, 4, 4, 17, 64, 128), (65, 4, 4, 17, 65, 128), (1, 4, 2, 33, 128, 128),
+    (1, 4, 2, 33, 129, 128), (1, 8, 1, 1, 128, 128)]
 
 
 @pytest.mark.parametrize("b,hq,hkv,nq,nk,d", CASES)
