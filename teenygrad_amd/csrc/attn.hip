@@ -485,14 +485,24 @@ static void launch_f32(const void *q, const void *k, const void *v, void *o, flo
 }
 
 // Whether a causal workgroup runs two query blocks, i and nqb - 1 - i, in turn.
-// Measured in us, two / one (heads x rows x head_dim): from 32 blocks on and
+// Measured in us, two / one (heads x rows x head_dim).  From 32 blocks on and
 // two workgroups per CU it is the better one, 128 x 4096 x 64 345 / 353, 32 x
 // 8192 x 64 315 / 320, 32 x 8192 x 128 522 / 526, and past 64 blocks on any grid,
-// 4 x 16384 x 128 296 / 350 (one head's longer blocks fall to one XCD); below,
-// its second prologue and fewer workgroups cost more, 256 x 2048 x 128 334 / 329,
-// 96 x 3000 x 128 270 / 249, 10 x 2500 x 128 57 / 49, 64 x 1024 x 64 25.6 / 22.7.
+// 4 x 16384 x 128 296 / 350 (one head's longer blocks fall to one XCD).  Below,
+// its second prologue and fewer workgroups cost more in general, 256 x 2048 x
+// 128 334 / 329, 96 x 3000 x 128 270 / 249, 10 x 2500 x 128 57 / 49, 64 x 1024 x
+// 64 25.6 / 22.7, but not where the pairs, all of one length but an odd count's
+// middle block, fill the chip evenly: all of them resident at once and most
+// slots taken (one / two 320 x 256 x 64 1.13, 384 x 129 x 64 1.14, 256 x 257 x 64 1.13, 128 x 896 x 64
+// 1.22, 160 x 640 x 128 1.0), or an even count on two heads per CU and more (512
+// x 1024 x 64 1.08, 512 x 1200 x 64 1.11, 1024 x 256 x 128 1.10; odd 512 x 300 x
+// 64 0.92, 1024 x 384 x 128 0.85), or in whole rounds where causal_order's groups
+// of heads leave slots open (256 x 1536 x 64 1.17, 128 x 1536 x 128 1.09).
 static bool causal_pairs(int BH, int nqb) {
-  return nqb > 64 || (nqb >= 32 && static_cast<int64_t>(BH) * nqb >= 4 * device_cu_count());
+  const int64_t cus = device_cu_count(), pairs = static_cast<int64_t>(BH) * ((nqb + 1) / 2);
+  if (nqb >= 32) return nqb > 64 || static_cast<int64_t>(BH) * nqb >= 4 * cus;
+  if (nqb <= 12 && pairs <= 2 * cus && (nqb == 2 ? pairs > cus : 2 * pairs >= 3 * cus)) return true;
+  return nqb == 1 || (nqb % 2 == 0 && (BH >= 2 * cus || (64 % nqb != 0 && pairs % cus == 0)));
 }
 
 template <int D>

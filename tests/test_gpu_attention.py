@@ -119,3 +119,15 @@ def test_bf16_full_grids(dev, orc, bh, nq, nk, d, causal):
     oo, ol = orc.flash_attention(q, k, v, causal=causal)
     check_bf16(o, oo, "o")
     assert np.max(np.abs(lse - ol)) < 1e-3
+
+
+@pytest.mark.parametrize("bh,n,d", [
+    # few query blocks, two per workgroup in turn and one: a round of pairs, an odd count, many heads, whole rounds
+    (300, 200, 64), (192, 300, 128), (520, 150, 64), (520, 300, 64), (256, 650, 64), (90, 520, 128)])
+def test_bf16_causal_short(dev, orc, bh, n, d):
+    print(f"[attn bf16 causal] bh={bh} n={n} d={d}", flush=True)
+    q, k, v = bf16_inputs(np.random.default_rng(n * 31 + bh), bh, n, n, d)
+    o, lse = run_bf16(dev, q, k, v, True)
+    oo, ol = orc.flash_attention(q, k, v, causal=True)
+    check_bf16(o, oo, "o")
+    assert np.max(np.abs(lse - ol)) < 1e-3
