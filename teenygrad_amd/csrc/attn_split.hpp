@@ -50,11 +50,11 @@ __global__ __launch_bounds__(256, 2) void fa_split_bf16(AttnSplitArgs p) {
   static_assert(RED * 4 >= 32 * D * 2, "the V tile shares the reduction's space");
   auto fv = [](int row) { return (4 * (row / RPB)) & (CPR - 1) & ~3; };
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, c = lane & 31, g = lane >> 5;
-  const int64_t unit = blockIdx.y;  // (run, column block)
-  const int64_t run = unit / p.blocks, hk = run / p.kv_runs;
+  const uint32_t unit = blockIdx.y;  // (run, column block)
+  const uint32_t run = unit / static_cast<uint32_t>(p.blocks), hk = run / static_cast<uint32_t>(p.kv_runs);
   const int c0 = static_cast<int>(unit - run * p.blocks) * 32, ncol = min(32, p.rows - c0);
-  const int64_t row0 = run * p.rows + c0;
-  const bf16 *Kb = p.K + hk * p.nk * D, *Vb = p.V + hk * p.nk * D;
+  const int64_t row0 = static_cast<int64_t>(run) * p.rows + c0, key0 = static_cast<int64_t>(hk) * p.nk;
+  const bf16 *Kb = p.K + key0 * D, *Vb = p.V + key0 * D;
   // causal: the row's query sees the keys up to its own index, the block's rows those up to their last one's
   // (of several heads in a block, which have at most 32 queries, up to the heads' last)
   const int qi = CAUSAL ? (c0 + min(c, ncol - 1)) % p.nq : 0;
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256, 2) void fa_split_bf16(AttnSplitArgs p) {
       for (int v = 0; v < 16; ++v) red[w][(32 * d + mfma32_row(v, g)) * 33 + c] = acc[d][v] * mul;
   }
   __syncthreads();
-  const int64_t slot = (unit * gridDim.x + blockIdx.x) * 32;  // part rows of this (unit, range)
+  const int64_t slot = (static_cast<int64_t>(unit) * gridDim.x + blockIdx.x) * 32;  // part rows of this (unit, range)
   for (int i = threadIdx.x; i < ncol * (D / 4); i += 256) {
     const int r = i / (D / 4), d = 4 * (i % (D / 4));
     f32x4 o;
