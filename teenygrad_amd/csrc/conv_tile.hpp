@@ -530,7 +530,10 @@ inline bool tile_conv_fits(const GemmParams &p) {
 // idle: two or four, as fit the CUs, of at least four 32-channel chunks, each
 // a workgroup that writes fp32 partial sums to the scratch.  512 -> 512 in us,
 // whole / sliced: batch 1 22.3 / 14.3, 4 22.4 / 15.0, 16 23.1 / 17.6, stride 2
-// batch 2 22.8 / 15.6.  The wider images' units have half the chunks or fewer,
+// batch 2 22.8 / 15.6.  With fewer than 16 chunks half of them saves less than
+// the partial sums of many units cost: 256 -> 256 batch 4 13.9 / 13.6, 16 14.6 /
+// 14.4, but 32 14.5 / 15.1, 64 14.9 / 17.5; 320 -> 256 batch 16 16.6 / 15.4, 48
+// 16.9 / 17.4.  The wider images' units have half the chunks or fewer,
 // and the second launch costs what slices of two save (14x14 256 -> 256, batch
 // 1 18.1 / 14.1 but 16 18.7 / 20.9).
 struct TileSlices {
@@ -542,8 +545,9 @@ inline TileSlices tile_conv_slices(const GemmParams &p) {
   const int B = p.M / (p.OH * p.OW), nch = p.Cin / 32, units = (B + 1) / 2 * (p.N / 64);
   TileSlices t;
   int n = 1;
-  while (p.OW == 7 && n < 4 && 2 * n * units <= device_cu_count() && 2 * n <= nch / 4) n *= 2;
-  if (n == 1) return t;
+  const int cus = device_cu_count();
+  while (p.OW == 7 && n < 4 && 2 * n * units <= cus && 2 * n <= nch / 4) n *= 2;
+  if (n == 1 || (nch < 16 && 16 * units > (nch - 7) * cus)) return t;
   t.ch_slice = (nch + n - 1) / n;
   t.slices = (nch + t.ch_slice - 1) / t.ch_slice;
   t.bytes = static_cast<size_t>(t.slices) * p.M * p.N * sizeof(float);

@@ -586,6 +586,16 @@ def test_small_batch_slices(dev, B, H, Cin, Cout, s, weights):
         assert np.all(err <= bound), f"{np.max(err - bound)} beyond the bound"
 
 
+@pytest.mark.parametrize("B,H,Cin,Cout,s,sliced", [
+    (8, 7, 256, 256, 1, True), (24, 7, 256, 256, 1, False), (64, 14, 256, 256, 2, False), (24, 7, 320, 256, 1, True),
+    (48, 7, 320, 256, 1, False), (64, 7, 512, 256, 1, True), (66, 7, 512, 256, 1, False)])
+def test_slices_where_they_pay(dev, B, H, Cin, Cout, s, sliced):
+    # fewer than 16 chunks of C_IN: sliced only for few units of work
+    if dev.info()["compute_units"] != 256:
+        pytest.skip("the plan's lines are those of 256 CUs")
+    assert (K.conv2d_workspace_size((B, H, H, Cin), (Cout, 3, 3, Cin), s, 1, 1, tg.bf16) > 0) == sliced
+
+
 GROUPED_K = [  # B, H, C_IN, C_OUT, kernel, stride: K shared by groups of waves, 64- and 128-row tiles, ragged edges
     (3, 20, 24, 72, 7, 1), (5, 13, 104, 200, 5, 2), (2, 15, 256, 130, 3, 2), (12, 28, 48, 120, 5, 1), (22, 28, 48, 120, 5, 1)]
 
