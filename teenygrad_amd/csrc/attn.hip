@@ -34,10 +34,10 @@
 // fa_split_bf16 (attn_split.hpp: few queries per K/V head, bf16 at head_dim 64
 // and 128): the keys shared out over waves and workgroups.
 //
-// fa_fwd_f32 (attn_f32.hpp: fp32 at head_dim 16 .. 128, bf16 at 16 and 32):
-// fp32 products on the fp32 matrix cores.
+// fa_fwd_f32 (attn_f32.hpp: fp32 at head_dim 16 .. 128, bf16 at 16 and 32, but
+// for the least work): fp32 products on the fp32 matrix cores.
 //
-// fa_fwd_rows (head_dim 256).  The reference's per-query-row structure — grid
+// fa_fwd_rows (head_dim 256, and where fa_rows_q says so).  The reference's per-query-row structure — grid
 // (N_q, BH), one wave per query row — with the key loop vectorised across
 // lanes: each lane scores one key of a 64-key chunk, and the chunk is folded
 // into the running (m, l, acc) state.  bf16 operands are widened to fp32 on
@@ -406,7 +406,7 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void fa_fwd_bf16(const bf16 
   }  // pass
 }
 
-// Per-row path (head_dim 256): grid (nq, BH), one wave per query row (flash_attn2.rs:48-51).
+// Per-row path: grid (nq, BH), one wave per query row (flash_attn2.rs:48-51).
 template <typename T, int D>
 __global__ __launch_bounds__(64) void fa_fwd_rows(const T *__restrict__ Q, const T *__restrict__ K,
                                                   const T *__restrict__ V, T *__restrict__ O,
@@ -440,8 +440,9 @@ __global__ __launch_bounds__(64) void fa_fwd_rows(const T *__restrict__ Q, const
       s = dot * scale;
     }
     const float m_new = fmaxf(m_i, wave_max(s));
-    const float ed = expf(m_i - m_new);
-    const float p = key < kend ? expf(s - m_new) : 0.0f;
+    const float ref = m_new == -INFINITY ? 0.0f : m_new;  // a chunk of scores that are all -inf
+    const float ed = expf(m_i - ref);
+    const float p = key < kend ? expf(s - ref) : 0.0f;
     l_i = ed * l_i + wave_sum(p);
     ps[lane] = p;
     __syncthreads();
@@ -464,7 +465,8 @@ __global__ __launch_bounds__(64) void fa_fwd_rows(const T *__restrict__ Q, const
     const int d = lane + 64 * i;
     if (d < D) orow[d] = from_f32<T>(acc[i] / l_i);
   }
-  if (L != nullptr && lane == 0) L[bh * nq + qi] = m_i + logf(l_i);
+  // a row whose every score is -inf has no softmax: NaN, as its outputs
+  if (L != nullptr && lane == 0) L[bh * nq + qi] = m_i == -INFINITY ? __builtin_nanf("") : m_i + logf(l_i);
 }
 
 template <typename T, int D>
@@ -478,6 +480,10 @@ static void launch_rows(const void *q, const void *k, const void *v, void *o, fl
 template <typename T, int D>
 static void launch_f32(const void *q, const void *k, const void *v, void *o, float *l, int nq, int nk, float scale,
                        int BH, int causal, int kv_group, hipStream_t s) {
+  if (fa_rows_q(false, sizeof(T) == 4, BH, nq, causal ? std::min(nk, nq) : nk, D)) {
+    launch_rows<T, D>(q, k, v, o, l, nq, nk, scale, BH, causal, kv_group, s);
+    return;
+  }
   const int split = fa_f32_split(cdiv(nq, 32) * BH, cdiv(nk, 32), D);
   fa_f32_launch(TEENY_FA_F32(fa_fwd_f32, T, D, split), nq, BH, split, s, static_cast<const T *>(q),
                 static_cast<const T *>(k), static_cast<const T *>(v), static_cast<T *>(o), l,

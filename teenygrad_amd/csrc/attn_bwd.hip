@@ -37,8 +37,9 @@
 // Any other case (fp32, other head sizes, unaligned bf16, dk/dv alone without
 // a workspace): fp32 products on the fp32 matrix cores (attn_f32.hpp);
 // head_dim 256, whose operands and accumulators do not fit a wave's registers
-// there, runs the reference's per-row structure, one wave per query row (dq)
-// or key row (dkv), with the inner loop vectorised across lanes.
+// there, and the least work (fa_rows_q, fa_rows_k) run the reference's per-row
+// structure, one wave per query row (dq) or key row (dkv), with the inner loop
+// vectorised across lanes.
 #include "attn_f32.hpp"
 #include "mfma.hpp"
 
@@ -46,7 +47,7 @@ namespace teeny {
 
 constexpr float kBwdLog2e = 1.4426950408889634f;
 
-// ── per-row kernels (head_dim 256) ───────────────────────────────────────────────────────
+// ── per-row kernels ───────────────────────────────────────────────────────
 
 template <typename T, int D>
 __global__ __launch_bounds__(64) void fa_bwd_dq_rows(const T *__restrict__ Q, const T *__restrict__ K,
@@ -624,8 +625,17 @@ static void rows_dkv(const BwdArgs &a, const float *delta) {
                      static_cast<T *>(a.dk), static_cast<T *>(a.dv), a.nq, a.nk, a.scale, a.causal, a.group);
 }
 
+// Whether dq runs on the per-row kernel, which leaves no D_m.
+static bool dq_by_rows(const BwdArgs &a, bool f32) {
+  return a.D == 256 || fa_rows_q(true, f32, a.BH, a.nq, a.causal ? std::min(a.nk, a.nq) : a.nk, a.D);
+}
+
 template <typename T, int D>
 static void f32_dq(const BwdArgs &a, float *delta_out) {
+  if (dq_by_rows(a, sizeof(T) == 4)) {
+    rows_dq<T, D>(a);
+    return;
+  }
   const int split = fa_f32_split(cdiv(a.nq, 32) * a.BH, cdiv(a.nk, 32), D);
   fa_f32_launch(TEENY_FA_F32(fa_bwd_dq_f32, T, D, split), a.nq, a.BH, split, a.s, static_cast<const T *>(a.q),
                 static_cast<const T *>(a.k), static_cast<const T *>(a.v), static_cast<const T *>(a.o),
@@ -636,11 +646,15 @@ static void f32_dq(const BwdArgs &a, float *delta_out) {
 template <typename T, int D>
 static void f32_dkv(const BwdArgs &a, const float *delta) {
   const int64_t heads = a.BH / a.group;
+  if (fa_rows_k(sizeof(T) == 4, heads, static_cast<int64_t>(a.nq) * a.group, a.nk, D)) {
+    rows_dkv<T, D>(a, delta);
+    return;
+  }
   const int split = fa_f32_split(cdiv(a.nk, 32) * heads, cdiv(a.nq, 32) * a.group, D);
-  fa_f32_launch(TEENY_FA_F32(fa_bwd_dkv_f32, T, D, split), a.nk, heads, split, a.s, static_cast<const T *>(a.q), static_cast<const T *>(a.k), static_cast<const T *>(a.v),
-                static_cast<const T *>(a.o), static_cast<const T *>(a.dout), a.l, delta, static_cast<T *>(a.dk),
-                static_cast<T *>(a.dv), static_cast<uint32_t>(a.nq), static_cast<uint32_t>(a.nk), a.scale, a.causal,
-                a.group);
+  fa_f32_launch(TEENY_FA_F32(fa_bwd_dkv_f32, T, D, split), a.nk, heads, split, a.s, static_cast<const T *>(a.q),
+                static_cast<const T *>(a.k), static_cast<const T *>(a.v), static_cast<const T *>(a.o),
+                static_cast<const T *>(a.dout), a.l, delta, static_cast<T *>(a.dk), static_cast<T *>(a.dv),
+                static_cast<uint32_t>(a.nq), static_cast<uint32_t>(a.nk), a.scale, a.causal, a.group);
 }
 
 // dq (writing D_m to `delta` when not NULL) or dk/dv (reading it when not NULL).
@@ -790,7 +804,7 @@ static teeny_status bwd_entry(BwdArgs a, int64_t batch, int64_t q_heads, int64_t
   }
   // dq first: given a workspace it leaves D_m there for dk/dv
   const Scratch scr = stream_scratch(a.s);
-  const bool ws = which == 3 && a.D != 256 && scr.ptr != nullptr && scr.bytes >= delta_bytes(a);
+  const bool ws = which == 3 && !dq_by_rows(a, dtype == TEENY_F32) && scr.ptr != nullptr && scr.bytes >= delta_bytes(a);
   float *delta = ws ? static_cast<float *>(scr.ptr) : nullptr;
   if (which & 1) (dtype == TEENY_F32 ? f32_launch<float> : f32_launch<bf16>)(a, true, delta);
   if (which & 2) (dtype == TEENY_F32 ? f32_launch<float> : f32_launch<bf16>)(a, false, delta);

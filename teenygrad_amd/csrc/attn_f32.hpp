@@ -33,6 +33,8 @@
 // (masked_outer), so that it reaches only the queries that see it.
 #pragma once
 
+#include <algorithm>
+
 #include "mfma.hpp"
 
 namespace teeny {
@@ -578,6 +580,40 @@ inline void fa_f32_launch(K kernel, int64_t cols, int64_t heads, int split, hipS
   const unsigned blocks = static_cast<unsigned>(cdiv(cols, 32));
   const dim3 grid(split > 1 ? blocks : (blocks + 3) / 4, static_cast<unsigned>(heads));
   hipLaunchKernelGGL(kernel, grid, dim3(64 * (split == 1 ? 4 : split)), 0, s, args..., static_cast<int>(blocks));
+}
+
+// Where the per-row kernels (a wave per query or key row, its lanes the rows of
+// the other side) are the faster ones, though a wave here does the same for 32
+// columns: with most of the 32 missing, on a chip that the blocks fill, and with
+// so little of everything that the way to the first product counts.  Measured in
+// us, rows / here, forward, fp32 (heads x queries x keys x head_dim): 2048 x 1 x
+// 1024 x 16 83 / 129, x 128 427 / 1573, 4096 x 2 x 512 x 64 367 / 441, 1024 x 1 x
+// 64 x 64 7.2 / 16, but 1024 x 1 x 512 x 64 60 / 55 (the tiles shared by four
+// waves), 2048 x 4 x 256 x 64 175 / 112; 8 x 16 x 64 x 128 7.1 / 10.2, 32 x 16 x
+// 64 x 32 4.2 / 4.5, 32 x 33 x 32 x 128 8.5 / 10.7 (the call's host time in it),
+// but 128 x 8 x 64 x 128 14.9 / 10.1.  dq gains up to twice the keys, 1536 x 1 x
+// 512 x 16 25 / 38, but not for two queries at head_dim 32 and 64, 2048 x 2 x 512
+// x 64 314 / 278.  dk/dv 8 x 8 x 64 x 64 8.6 / 10.7, 1024 x 1 x 1 x 64 8.7 / 18.5,
+// but 128 x 16 x 16 x 64 27.8 / 9.7.
+//
+// Forward and dq: BH heads of nq queries, which see at most nk keys.
+inline bool fa_rows_q(bool dq, bool f32, int64_t BH, int64_t nq, int64_t nk, int D) {
+  const int64_t cus = device_cu_count();
+  if (nk <= 64 && BH * nq * std::max<int64_t>(nk, 16) <= (!dq && D == 128 && nk <= 32 ? 65536 : 32768)) return true;
+  if (BH < 2 * cus) return false;
+  if (BH >= 8 * cus) {
+    const bool four = f32 ? !dq && D == 128 : D == 16, one = f32 && dq && (D == 32 || D == 64);
+    if (nq <= (four ? 4 : one ? 1 : 2)) return true;
+  }
+  if (nq > 4) return nq * std::max<int64_t>(nk, 8) <= D;
+  if (nq > 1) return nk <= (nq > 2 ? std::max<int64_t>(16, D / nq) : 64);
+  return nk <= (dq && D <= 32 && BH >= 3 * cus ? 512 : dq || BH >= 4 * cus ? 256 : 128);
+}
+
+// dk/dv: K/V heads of nk keys, nq queries of all heads that share them.
+inline bool fa_rows_k(bool f32, int64_t heads, int64_t nq, int64_t nk, int D) {
+  if ((f32 || D != 32) && (nq <= 8 ? heads * nk <= 1024 : nq <= 16 && heads * nk <= 256)) return true;
+  return heads >= 2 * device_cu_count() && nk * std::max<int64_t>(nq, 8) <= 16;
 }
 
 // The kernel template NAME<T, D, SPLIT> for a split (8: D <= 64 only).

@@ -75,6 +75,35 @@ def test_forward_backward(dev, dtype, bh, nq, nk, d, causal, group):
                 check_f32(g, r, name)
 
 
+LEAST = [  # bh, nq, nk, d, causal, group: both sides of the lines between these kernels and the per-row ones (256 CUs)
+    (32, 16, 64, 128, False, 1), (33, 16, 64, 128, True, 1), (2, 16, 65, 64, False, 1), (128, 16, 16, 32, True, 1),
+    (512, 1, 128, 64, False, 1), (512, 1, 129, 64, False, 1), (1024, 1, 256, 16, False, 2), (520, 2, 64, 32, False, 4),
+    (520, 2, 65, 32, False, 4), (512, 4, 32, 128, False, 1), (512, 16, 9, 128, False, 2), (2048, 2, 70, 16, False, 1),
+    (2048, 2, 70, 64, False, 8), (2048, 4, 70, 128, True, 8), (2047, 3, 17, 64, False, 1), (4, 8, 256, 64, False, 1),
+    (4, 8, 257, 64, False, 1), (16, 16, 16, 32, True, 1), (512, 16, 2, 16, False, 1)]
+
+
+@pytest.mark.parametrize("bh,nq,nk,d,causal,group", LEAST)
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_least_work(dev, dtype, bh, nq, nk, d, causal, group):
+    test_forward_backward(dev, dtype, bh, nq, nk, d, causal, group)
+
+
+@pytest.mark.parametrize("bh,nk", [(2048, 130), (8, 140)])  # the per-row kernel, and this file's
+def test_first_keys_without_weight(dev, bh, nk):
+    # the first keys' scores are all -inf: they weigh nothing, the others as if alone
+    rng = np.random.default_rng(nk)
+    q, k, v = (rng.standard_normal((bh, n, 16), dtype=np.float32) for n in (1, nk, nk))
+    q[..., 0] = 1.0
+    o, lse, *_ = reference(q, k[:, 70:], v[:, 70:], q, False, 1)
+    k[:, :70, 0] = -np.inf
+    print(f"[attn f32] scores of -inf bh={bh} nk={nk}", flush=True)
+    lb = tg.Buffer(tg.f32, (bh, 1))
+    ob = K.flash_attention(*(dev.upload(x) for x in (q, k, v)), lse=lb)
+    check_f32(ob.to_host(), o, "o")
+    check_f32(lb.to_host(), lse, "lse")
+
+
 @pytest.mark.parametrize("d", [16, 64, 128])
 @pytest.mark.parametrize("bad", [np.nan, np.inf])
 def test_masked_rows_without_numbers(dev, d, bad):
