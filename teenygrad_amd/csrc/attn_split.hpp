@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256) void fa_split_combine(AttnSplitArgs p, int ran
 // x keys 1 x 16384 262 / 31, 32 x 1000 57 / 23, 16 x 4000 106 / 52 (5 TB/s).  On
 // a full chip that counts where packing leaves fewer blocks than heads (heads in
 // groups of 4 or 8; queries x keys x head_dim): 32 x 2048 x 128, as many blocks
-// as heads, 512 of them 55 / 79, 4096 1.19 times as long; 20 x 2048 x 128, 5
+// as heads, 256 of them 38 / 41, 512 55 / 79, 4096 1.19 times as long; 20 x 2048 x 128, 5
 // blocks to 8 heads, 320 54 / 61, 640 0.93; half as many blocks or fewer 0.16 to
 // 0.77 at any size.  head_dim 64, 32 x 2048, as many blocks as heads: 512 35 /
 // 40, 2048 1.09, 4096 0.9; fewer blocks than heads, or causal and so one tile of
@@ -280,11 +280,11 @@ inline AttnSplitPlan attn_split_plan(int64_t BH, int64_t group, int64_t nq, int6
   if (causal) nk = std::min(nk, nq);
   const int64_t kv_runs = causal && nq > 32 ? group : 1, rows = group / kv_runs * nq;
   const int64_t cus = device_cu_count(), blocks = cdiv(rows, 32), units = BH / group * kv_runs * blocks;
-  if (units > (causal && nq > 128 && D == 64 ? 2 : 1) * cus && nq > 32) return pl;
-  if (units > cus && nq <= 32) {
+  const int64_t room = causal && nq > 128 && D == 64 ? 2 * cus : D == 128 && !causal && nq <= 64 ? cus - 1 : cus;
+  if (units > room) {
     const bool packed = D == 64 ? units < BH || units > 8 * cus || nk <= 32
                                 : 2 * units <= BH || (4 * units <= 3 * BH && units > 3 * cus);
-    if (group > 1 ? !packed : D == 128 && nq > 16 && nk <= 64) return pl;
+    if (nq > 32 || (group > 1 ? !packed : D == 128 && nq > 16 && nk <= 64)) return pl;
   }
   if (D == 128 && !causal && nk <= 128 && nq <= 64 && group * nq > 8 && BH <= cus) return pl;
   pl.use = true;

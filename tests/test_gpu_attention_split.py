@@ -18,7 +18,8 @@ CASES = [  # batch, q_heads, kv_heads, nq, nk, d: rows of a column block, tile a
     # them), 7 to 8; one tile of keys per wave
     (36, 16, 2, 32, 70, 128), (20, 32, 4, 20, 70, 128), (40, 32, 4, 20, 70, 128), (10, 64, 8, 28, 70, 64),
     (80, 8, 2, 32, 40, 64), (65, 4, 4, 17, 64, 128), (65, 4, 4, 17, 65, 128), (1, 4, 2, 33, 128, 128),
-    (1, 4, 2, 33, 129, 128), (1, 8, 1, 1, 128, 128)]
+    (1, 4, 2, 33, 129, 128), (1, 8, 1, 1, 128, 128),
+    (32, 8, 1, 32, 200, 128), (31, 8, 1, 32, 200, 128), (32, 4, 2, 64, 140, 128)]
 
 
 @pytest.mark.parametrize("b,hq,hkv,nq,nk,d", CASES)
