@@ -205,7 +205,7 @@ template <bool INT8B> inline void launch_gemm_skinny(GemmParams p, int act, hipS
   else if (p.M <= 32) TEENY_SKINNY(32, 4, 1);
   else if (nb == 1) TEENY_SKINNY(64, 1, 1);
   else if (nb == 2) TEENY_SKINNY(64, 2, 1);
-  else TEENY_SKINNY(64, 4, 1);
+  else if constexpr (INT8B) TEENY_SKINNY(64, 4, 1);  // bf16: gemm_skinny_ok
 #undef TEENY_SKINNY
 }
 

@@ -31,7 +31,9 @@ SMALL_GRID = [  # (M, N, K, K slices): 64 x 64 tiles with ragged edges, unsplit 
     (65, 65, 64, 1), (130, 72, 272, 1), (1000, 520, 1040, 1), (100, 200, 2048, 4), (257, 130, 2064, 4),
     (70, 1000, 4112, 4), (1023, 1024, 4096, 1), (1100, 1000, 4624, 4),
     # K shared by two and four groups of waves (runs of k-tiles past K), on 64 x 64, 128 x 64 and 128 x 128 tiles
-    (300, 520, 976, 1), (500, 600, 2064, 1), (450, 500, 2032, 1), (1100, 1000, 1104, 1), (2100, 1000, 1040, 1)]
+    (300, 520, 976, 1), (500, 600, 2064, 1), (450, 500, 2032, 1), (1100, 1000, 1104, 1), (2100, 1000, 1040, 1),
+    # few rows whose narrow output and deep K stay on the tiles
+    (64, 130, 4656, 4)]
 
 
 @pytest.mark.parametrize("m,n,k,slices", SMALL_GRID)
@@ -65,7 +67,9 @@ def test_small_grids(dev, m, n, k, slices, weights):
 
 SKINNY = [  # (M, N, K): row blocks of 16, column tails, K tails of 16 .. 64, fewer chunks than waves
     (1, 16, 16), (1, 1, 64), (7, 100, 528), (15, 33, 4096), (16, 48, 80), (17, 65, 1008), (32, 31, 2080), (33, 47, 1040),
-    (64, 130, 4656), (2, 11008, 64)]
+    (64, 130, 2032), (2, 11008, 64),
+    # two and four blocks of 16 columns per workgroup, the last one ragged (bf16 past 32 rows has no four)
+    (19, 5130, 528), (31, 10250, 208), (40, 5130, 1040), (64, 10250, 144)]
 
 
 @pytest.mark.parametrize("m,n,k", SKINNY)
@@ -88,6 +92,26 @@ def test_few_rows(dev, m, n, k, weights):
     # k fp32 sums, each within 2^-24 of at most sum |x| |w|, and the bf16 result
     bound = (k + 3) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T + np.abs(bias)) + 2.0 ** -8 * np.abs(ref)
     err = np.abs(from_bf16(got).astype(np.float64).reshape(m, n) - ref)
+    assert np.all(err <= bound), f"{np.max(err - bound)} beyond the bound"
+
+
+@pytest.mark.parametrize("m,n,k", [
+    # ragged K in rows padded to 16 bytes: K shared by two and four groups of waves on 64 x 64 tiles (with runs of
+    # k-tiles past K), by two on 128 x 64 and 128 x 128 tiles
+    (300, 130, 1001), (70, 200, 2051), (70, 72, 1985), (1100, 1000, 1101), (2100, 1000, 1039)])
+def test_small_grids_padded_rows(dev, m, n, k):
+    rng = np.random.default_rng(m + 3 * n + 5 * k)
+    x, w = (rb(rng.standard_normal((r, k), dtype=np.float32)).reshape(r, k) for r in (m, n))
+    ld = -(-k // 8) * 8
+    pad = lambda a: np.pad(a, ((0, 0), (0, ld - k)), constant_values=np.nan)  # noqa: E731 (not to be read)
+    xb, wb = (dev.upload(to_bf16(pad(a)), tg.bf16) for a in (x, w))
+    y = tg.Buffer(tg.bf16, (m, n))
+    print(f"[small grid] M={m} N={n} K={k} rows of {ld}", flush=True)
+    tg.check(_lib.lib.teeny_linear_forward(xb.ptr, wb.ptr, None, y.ptr, m, n, k, ld, 1, ld, 1, n, 1, tg.bf16.code, None))
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    # k fp32 sums, each within 2^-24 of at most sum |x| |w|, and the bf16 result
+    bound = (k + 8) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T) + 2.0 ** -8 * np.abs(ref)
+    err = np.abs(from_bf16(y.to_host()).astype(np.float64).reshape(m, n) - ref)
     assert np.all(err <= bound), f"{np.max(err - bound)} beyond the bound"
 
 
