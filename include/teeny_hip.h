@@ -441,7 +441,7 @@ teeny_status teeny_conv2d_backward_workspace_size(int64_t B, int64_t C_IN, int64
  * 2 GiB (n_ctx_k * head_dim * 2 bytes; TEENY_ERR_SHAPE_MISMATCH otherwise);
  * the other bf16 head sizes and fp32 run fp32 products (on bf16 operands
  * widened to fp32), on the fp32 matrix cores up to head_dim 128 and in the
- * reference's per-query-row structure at 256. */
+ * reference's per-query-row structure at 256 and for the least work. */
 teeny_status teeny_flash_attention2_forward(const void *q, const void *k, const void *v, void *o,
                                             float *l, int64_t n_ctx_q, int64_t n_ctx_k,
                                             float softmax_scale, int64_t BH, int64_t head_dim,
@@ -487,7 +487,7 @@ teeny_status teeny_attention_workspace_size(int64_t batch, int64_t q_heads, int6
  * bytes for its D_m pre-pass, else it takes the fp32 kernel); fp32 and any
  * other head_dim in {16, 32, 64, 128, 256} run fp32 products, on the fp32
  * matrix cores up to head_dim 128 and in the reference's per-row structure at
- * 256. */
+ * 256 and for the least work. */
 teeny_status teeny_flash_attention2_backward_dq(const void *q, const void *k, const void *v, const void *o,
                                                 const void *dout, const float *l, void *dq, int64_t n_ctx_q,
                                                 int64_t n_ctx_k, float softmax_scale, int64_t BH, int64_t head_dim,

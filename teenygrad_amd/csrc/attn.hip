@@ -94,6 +94,8 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void fa_fwd_bf16(const bf16 
 
   // All query blocks of one (b, h) are consecutive logical ids on one XCD,
   // so they run together and read K/V once from HBM into that XCD's L2.
+  // Without the mask the blocks are alike (in index order, not the reverse as
+  // once: 999 full grids took 0.997 of the time on average, none beyond noise).
   // Causal: a query block's work grows with its index.  Either causal_order
   // balances the CUs, or (pairs) workgroup p of a head runs blocks nqb-1-p and
   // then p, and every workgroup does the same nqb + 1 key tiles.

@@ -25,8 +25,12 @@
 // depend on timing (no atomics).
 //
 // Measured, 16 heads of 500 x 500 x 64 fp32, forward + dq + dk/dv: 2987 us
-// with one wave per row (152 + 288 + 2504) -> 70 us, 65 TFLOP/s of the seven
-// products executed (1024 waves, one per SIMD, on 16 tiles of 32 x 32 each).
+// with one wave per row (152 + 288 + 2504) -> 69 us (18 + 24 + 32 traced), 67
+// TFLOP/s of the nine products executed (256 blocks of 32 columns, one
+// workgroup per CU: 2048 waves, two per SIMD, with two 32 x 32 tiles each).
+// dk/dv holds two operands and two accumulators: at head_dim 64 all of its 256
+// registers with 39 to 54 spilled (84 to 104 bytes a lane), at 128 28 to 37
+// beside the accumulation registers, reloaded in the tile loop.
 //
 // A product with a masked pair is p = 0 times a row that the query may not
 // see; if such a row holds an infinity or NaN the tile is redone pair by pair
@@ -223,10 +227,9 @@ __device__ __forceinline__ bool fa_unit(int w, int blocks, int &blk, int64_t &he
 }
 
 template <typename T, int D, int SPLIT>
-__global__ __launch_bounds__(64 * kFaWaves<SPLIT>, D <= 64 ? 2 : 1) void fa_fwd_f32(const T *__restrict__ Q, const T *__restrict__ K,
-                                                                   const T *__restrict__ V, T *__restrict__ O,
-                                                                   float *__restrict__ L, uint32_t nq, uint32_t nk,
-                                                                   float scale, int causal, int kv_group, int nqb) {
+__global__ __launch_bounds__(64 * kFaWaves<SPLIT>, D <= 64 ? 2 : 1) void fa_fwd_f32(
+    const T *__restrict__ Q, const T *__restrict__ K, const T *__restrict__ V, T *__restrict__ O,
+    float *__restrict__ L, uint32_t nq, uint32_t nk, float scale, int causal, int kv_group, int nqb) {
   using Tile = FaTile<T, D>;
   __shared__ __attribute__((aligned(16))) float lds[kFaWaves<SPLIT>][2 * Tile::FLOATS];
   __shared__ float ml[2][kFaWaves<SPLIT>][32];

@@ -1311,7 +1311,8 @@ __global__ __launch_bounds__(256 * KG, 2) void conv_dw_mfma(const bf16 *__restri
   // channels), so those that the first stage has are told by their index.  A
   // column past the edge starts at kOffNone; it reaches no output.
   const int rpx = ROWS ? 0 : q.OW * q.OH;
-  const int d_bb = ROWS ? 0 : kDwStage / rpx, d_oh = ROWS ? 0 : kDwStage % rpx / q.OW, d_ow = ROWS ? 0 : kDwStage % q.OW;
+  const int d_bb = ROWS ? 0 : kDwStage / rpx;
+  const int d_oh = ROWS ? 0 : kDwStage % rpx / q.OW, d_ow = ROWS ? 0 : kDwStage % q.OW;
   const int px = q.Cin * 2;  // bytes per pixel of x
   const int step = ROWS ? kDwStage * px : ((d_bb * q.H + d_oh * q.SH) * q.W + d_ow * q.SW) * px;
   const int wrap_w = (q.SH * q.W - q.OW * q.SW) * px, wrap_h = (q.H - q.OH * q.SH) * q.W * px;
@@ -1517,8 +1518,9 @@ static bool conv_dw_mfma_launch(const void *dy, const void *x, void *dw, const C
   auto kern = d.splits > 1 ? (rows ? conv_dw_mfma<true, true, 2> : conv_dw_mfma<true, false, 2>)
               : d.groups   ? (rows ? conv_dw_mfma<false, true, 2> : conv_dw_mfma<false, false, 2>)
                            : (rows ? conv_dw_mfma<false, true, 1> : conv_dw_mfma<false, false, 1>);
-  hipLaunchKernelGGL(kern, grid, dim3(d.groups ? 512 : 256), 0, s, static_cast<const bf16 *>(dy), static_cast<const bf16 *>(x),
-                     static_cast<bf16 *>(dw), part, q, d.tiles_m, d.tiles_n, d.stages_per_split, P);
+  hipLaunchKernelGGL(kern, grid, dim3(d.groups ? 512 : 256), 0, s, static_cast<const bf16 *>(dy),
+                     static_cast<const bf16 *>(x), static_cast<bf16 *>(dw), part, q, d.tiles_m, d.tiles_n,
+                     d.stages_per_split, P);
   if (d.splits > 1) {
     const int64_t mn = static_cast<int64_t>(q.Cout) * q.KH * q.KW * q.Cin;
     int sub = 1;

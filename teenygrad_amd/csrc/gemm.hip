@@ -173,7 +173,8 @@ __global__ __launch_bounds__(256) void linear_bwd_db_sum(const float *__restrict
 
 // Row shares of linear_bwd_db: one while a workgroup's rows are few enough to
 // be read in about the time that a second launch would cost (2048 rows of 64
-// bytes), and never more workgroups than CUs.
+// bytes), and no more of them than give each CU a workgroup of 32 columns (the
+// fp32 vector form owns 16, so up to two; wider outputs give more by themselves).
 static int64_t linear_db_shares(int64_t M, int64_t N) {
   return std::max<int64_t>(1, std::min(M / 2048, device_cu_count() / cdiv(N, 32)));
 }
@@ -192,8 +193,9 @@ static void launch_linear_db(const T *dy, int64_t sm, int64_t sn, T *db, int64_t
   // 2^31 threads a launch at most: a grid of 2^32 wraps (shares > 1 only far below)
   for (int64_t n0 = 0, step = cols << 21; n0 < N; n0 += step) {
     const int64_t n = std::min(step, N - n0);
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(cdiv(n, cols)), static_cast<unsigned>(shares)), dim3(1024), 0, s,
-                       dy + n0 * sn, sm, sn, db + n0 * sdb, sdb, part, static_cast<int>(M), static_cast<int>(n), rows);
+    const dim3 grid(static_cast<unsigned>(cdiv(n, cols)), static_cast<unsigned>(shares));
+    hipLaunchKernelGGL(kern, grid, dim3(1024), 0, s, dy + n0 * sn, sm, sn, db + n0 * sdb, sdb, part,
+                       static_cast<int>(M), static_cast<int>(n), rows);
   }
   if (part != nullptr)
     hipLaunchKernelGGL(linear_bwd_db_sum<T>, dim3(static_cast<unsigned>(cdiv(N, 256))), dim3(256), 0, s, part,

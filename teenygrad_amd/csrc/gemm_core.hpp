@@ -613,48 +613,48 @@ __global__ __launch_bounds__(256 * KG, (gemm_min_waves<BM, BN>())) void gemm_mfm
   static_assert(WN % 16 == 0 && WM % 16 == 0, "fragment rows keep the swizzle of lane c");
   bf16 *cs = smem0;
   if (kg == 0) {
-  // scale / bias per group of four columns (shared by the MB row blocks)
-#pragma clang loop unroll(full)
-  for (int i = 0; i < NB; ++i)
-#pragma clang loop unroll(full)
-    for (int v4 = 0; v4 < 4; ++v4) {
-      float mul[4], add[4];
-      epi_coeffs(p, n0 + wn * WN + i * 32 + 8 * v4 + 4 * g, mul, add);
-#pragma clang loop unroll(full)
-      for (int j = 0; j < MB; ++j)
-#pragma clang loop unroll(full)
-        for (int e = 0; e < 4; ++e) acc[i][j][4 * v4 + e] = __builtin_fmaf(acc[i][j][4 * v4 + e], mul[e], add[e]);
-    }
-  const EpiAct ea = epi_act(p.act);
-  if (ea.sig) {
+    // scale / bias per group of four columns (shared by the MB row blocks)
 #pragma clang loop unroll(full)
     for (int i = 0; i < NB; ++i)
 #pragma clang loop unroll(full)
-      for (int j = 0; j < MB; ++j)
-#pragma clang loop unroll(full)
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = epi_sig(acc[i][j][v], ea);
-  }
-  const float lo = ea.relu ? 0.0f : -INFINITY;
-#pragma clang loop unroll(full)
-  for (int j = 0; j < MB; ++j) {
-    const int ml = wm * WM + j * 32 + c;
-#pragma clang loop unroll(full)
-    for (int i = 0; i < NB; ++i) {
-#pragma clang loop unroll(full)
       for (int v4 = 0; v4 < 4; ++v4) {
-        const int nl = wn * WN + i * 32 + 8 * v4 + 4 * g;
-        bf16x4 o4;
+        float mul[4], add[4];
+        epi_coeffs(p, n0 + wn * WN + i * 32 + 8 * v4 + 4 * g, mul, add);
 #pragma clang loop unroll(full)
-        for (int e = 0; e < 4; ++e) {
-          const float r = acc[i][j][4 * v4 + e];
-          o4[e] = static_cast<bf16>(r < lo ? lo : r);
+        for (int j = 0; j < MB; ++j)
+#pragma clang loop unroll(full)
+          for (int e = 0; e < 4; ++e) acc[i][j][4 * v4 + e] = __builtin_fmaf(acc[i][j][4 * v4 + e], mul[e], add[e]);
+      }
+    const EpiAct ea = epi_act(p.act);
+    if (ea.sig) {
+#pragma clang loop unroll(full)
+      for (int i = 0; i < NB; ++i)
+#pragma clang loop unroll(full)
+        for (int j = 0; j < MB; ++j)
+#pragma clang loop unroll(full)
+          for (int v = 0; v < 16; ++v) acc[i][j][v] = epi_sig(acc[i][j][v], ea);
+    }
+    const float lo = ea.relu ? 0.0f : -INFINITY;
+#pragma clang loop unroll(full)
+    for (int j = 0; j < MB; ++j) {
+      const int ml = wm * WM + j * 32 + c;
+#pragma clang loop unroll(full)
+      for (int i = 0; i < NB; ++i) {
+#pragma clang loop unroll(full)
+        for (int v4 = 0; v4 < 4; ++v4) {
+          const int nl = wn * WN + i * 32 + 8 * v4 + 4 * g;
+          bf16x4 o4;
+#pragma clang loop unroll(full)
+          for (int e = 0; e < 4; ++e) {
+            const float r = acc[i][j][4 * v4 + e];
+            o4[e] = static_cast<bf16>(r < lo ? lo : r);
+          }
+          // 16-byte chunk nl / 8 of row ml sits at chunk (nl / 8) ^ ((ml >> 4) & 1):
+          // rows c and c + 16 of one write instruction then use different banks
+          *reinterpret_cast<bf16x4 *>(cs + ml * CP + (((nl >> 3) ^ ((ml >> 4) & 1)) << 3) + (nl & 7)) = o4;
         }
-        // 16-byte chunk nl / 8 of row ml sits at chunk (nl / 8) ^ ((ml >> 4) & 1):
-        // rows c and c + 16 of one write instruction then use different banks
-        *reinterpret_cast<bf16x4 *>(cs + ml * CP + (((nl >> 3) ^ ((ml >> 4) & 1)) << 3) + (nl & 7)) = o4;
       }
     }
-  }
   }
   __syncthreads();
   constexpr int CPR_C = BN / 8;             // 16-byte chunks per C row
